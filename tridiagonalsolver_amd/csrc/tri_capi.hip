@@ -216,7 +216,7 @@ static const TileEntry<T> *choose_tile(int algo, int layout, int64_t n, bool vec
         for (int fi = 0; fi < (fam == 0 ? 1 : 2); ++fi)
         for (const TuneRow &r : g_tune) {
             if (r.prec != prec || r.layout != tl || r.family != fams[fi] || n > r.nmax) continue;
-            if (r.vec && !vec_ok) continue;
+            if (r.vec && !r.xp && !vec_ok) continue;
             const int nws = il ? r.NW : r.NW / r.S;
             const int64_t cap = (int64_t)(il ? 64 / r.S : 64) * nws * r.M;
             if (cap < n || cap > 2 * n) continue;   // bucket too coarse for this n
@@ -234,7 +234,7 @@ static const TileEntry<T> *choose_tile(int algo, int layout, int64_t n, bool vec
         const TileEntry<T> &e = tab.entries[i];
         if (e.IL != il || e.cap < n || e.BIG != big) continue;
         if (!e.BIG && e.PAD != (e.cap != n)) continue;   // exact tiles take the unpredicated kernel
-        if (e.VEC && !vec_ok) continue;
+        if (e.VEC && !e.XP && !vec_ok) continue;   // whole-chunk tiles take any row start
         if (fM && e.M != fM) continue;
         if (lds_need(e, algo) > max_lds_per_block()) continue;
         const int nws = il ? e.NW : e.NW / e.S;
