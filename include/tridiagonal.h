@@ -294,7 +294,8 @@ int tridiag_div_mode(void);
  *                      64/S*NW*M rows (interleaved) or 64*NW*M rows (contiguous),
  *                      on chip, 4 three passes over chunks through global
  *                      memory, 5 interleaved systems solved through a contiguous
- *                      copy; -1 on a bad argument.
+ *                      copy, 6 a bulk-row form, 7 several short contiguous
+ *                      systems per wave, on chip; -1 on a bad argument.
  *   tridiag_plan       for kinds 2 and 3, rows-per-lane M, waves per workgroup
  *                      NW, systems per workgroup S; TRIDIAG_EUNSUPPORTED for the
  *                      other kinds. */

@@ -132,7 +132,8 @@ def algo_names(precision):
             for i in range(L.tridiag_algo_count(precision))]
 
 
-PLAN_KINDS = ["lane", "thomas", "tile", "cooperative", "chunked", "via_contiguous", "bulk_row"]
+PLAN_KINDS = ["lane", "thomas", "tile", "cooperative", "chunked", "via_contiguous", "bulk_row",
+              "short"]
 
 
 def plan(precision, algo, layout, n, batch):

@@ -551,6 +551,7 @@ enum PlanKind {
     kPlanChunked = 4,        // three passes over chunks through global memory
     kPlanViaContiguous = 5,  // interleaved systems solved through a contiguous copy
     kPlanBulk = 6,           // the reference's own form of ids 2-13 (bulk rows, CR levels)
+    kPlanShort = 7,          // several short contiguous systems per wave
 };
 template <typename T> struct SolvePlan {
     int kind = kPlanTile;
@@ -683,6 +684,17 @@ static SolvePlan<T> make_plan(int algo, int layout, int64_t n, int64_t batch, in
     const bool il = layout == kInterleaved;
     const int prec = sizeof(T) == 4 ? TRIDIAG_SINGLE : TRIDIAG_DOUBLE;
     const int32_t bb = buffer_extent<T>(n, batch, sstride, layout);
+    // short contiguous systems: several per wave, for the automatic choice above the 8
+    // rows that fill the lane kernel (2^22 unknowns, lane / this: 9 rows FP32 21.1 / 14.7
+    // us, 16 rows 15.8 / 15.8, FP64 32.4 / 28.7) and up to where a tile's wave per system
+    // holds few padding rows (192 rows, tile / this: FP32 14.8 / 15.4 us, FP64 31.2 /
+    // 28.9; 200 rows FP32 16.5 either way, FP64 29.5 / 30.2).  Up to 64 systems of 16
+    // rows are one wave of the lane kernel and keep it.
+    if (algo == TRIDIAG_ALGO_AUTO && layout == kContiguous && n > 8 && n <= kShortMaxRows &&
+        (n > 16 || batch > 64)) {
+        pl.kind = kPlanShort;
+        return pl;
+    }
     // short systems: one system per lane in registers (Thomas), for the Thomas id and
     // for the automatic choice up to lane_auto_rows()
     if (bb != 0 && n <= lane_thomas_max_rows(prec) && (il || layout == kContiguous) &&
@@ -771,6 +783,14 @@ static int solve_impl(int algo, int layout, int64_t n, int64_t batch, T *a, T *b
             : launch_lane_thomas_f64((const double *)a, (const double *)b, (const double *)c,
                                      (double *)d, n, batch, sstride, rstride, il, bb, st);
         return e == hipSuccess ? TRIDIAG_OK : hip_fail(e, "lane Thomas launch");
+    }
+    case kPlanShort: {
+        const hipError_t e = (sizeof(T) == 4)
+            ? launch_short_f32((const float *)a, (const float *)b, (const float *)c, (float *)d, n,
+                               batch, st)
+            : launch_short_f64((const double *)a, (const double *)b, (const double *)c, (double *)d,
+                               n, batch, st);
+        return e == hipSuccess ? TRIDIAG_OK : hip_fail(e, "short-system launch");
     }
     case kPlanThomas: {
         if (!il && bb != 0) {
