@@ -93,8 +93,7 @@ __global__ void __launch_bounds__(256) short_kernel(const T *a, const T *b, cons
 #pragma unroll
     for (int q = 0; q < NQ; ++q)
         if ((q + 1) * 64 <= TOT || q * 64 + lane < TOT)
-            __builtin_amdgcn_raw_buffer_store_b128(xb[q * 64 + lane], rr[3], lane * 16, q * 1024,
-                                                   cpol<true>());
+            store16<true>(xb[q * 64 + lane], rr[3], lane * 16 + q * 1024);
 }
 
 template <typename T, int M, int P>

@@ -120,6 +120,17 @@ __device__ __forceinline__ void bstore(T x, __amdgpu_buffer_rsrc_t r, int vo, in
 }
 using u32x4 = __attribute__((ext_vector_type(4))) unsigned;
 
+// Stores a 16-byte chunk at byte offset vo.  The whole offset goes through the address
+// register and the instruction's immediate, never through the scalar offset: the store
+// still reads its data registers while the next instruction issues, and the compiler
+// keeps that instruction off them only where the scalar offset is a constant.  With an
+// SGPR there, an FP32 kernel whose next instruction overwrote the data stored wrong
+// first elements in a few chunks of a launch.
+template <bool NT>
+__device__ __forceinline__ void store16(u32x4 t, __amdgpu_buffer_rsrc_t r, int vo) {
+    __builtin_amdgcn_raw_buffer_store_b128(t, r, vo, 0, cpol<NT>());
+}
+
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void *p, int32_t bytes) {
     // raw buffer (stride 0); word 3 = 0x00020000 selects 32-bit data format on gfx9
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), (short)0, bytes, 0x00020000);
@@ -151,8 +162,7 @@ __device__ __forceinline__ void sys_chunk_store(u32x4 t, __amdgpu_buffer_rsrc_t 
                                                 int64_t e, int64_t n) {
     constexpr int VV = 16 / (int)sizeof(T);
     if (e + VV <= n) {
-        __builtin_amdgcn_raw_buffer_store_b128(t, r, (int)((base + e) * (int64_t)sizeof(T)), 0,
-                                               cpol<NT>());
+        store16<NT>(t, r, (int)((base + e) * (int64_t)sizeof(T)));
     } else if (e < n) {
 #pragma unroll
         for (int v = 0; v < VV; ++v)
@@ -386,7 +396,7 @@ __device__ __forceinline__ void il_block_store(__amdgpu_buffer_rsrc_t rd, int64_
         const int64_t s0 = col0 + h * VV;                  // first system of the chunk
         const u32x4 t = xb[cidx];
         if (s0 + VV <= batch) {
-            __builtin_amdgcn_raw_buffer_store_b128(t, rd, off, 0, cpol<NT>());
+            store16<NT>(t, rd, off);
         } else {
 #pragma unroll
             for (int v = 0; v < VV; ++v)
@@ -801,8 +811,7 @@ __global__ void __launch_bounds__(64 * NW)
         const int wvo = (int)(((PAD ? 0 : base) + (int64_t)ws * 64 * M) * (int64_t)sizeof(T)) + lane * 16;
 #pragma unroll
         for (int q = 0; q < NQ; ++q)
-            __builtin_amdgcn_raw_buffer_store_b128(xbuf[wave][q * 64 + lane], rx, wvo, q * 1024,
-                                                   cpol<NT>());
+            store16<NT>(xbuf[wave][q * 64 + lane], rx, wvo + q * 1024);
         return;
     }
     T *__restrict__ D = prm.d;
@@ -821,7 +830,7 @@ __global__ void __launch_bounds__(64 * NW)
                 u32x4 xs;
 #pragma unroll
                 for (int vv = 0; vv < V; ++vv) reinterpret_cast<T *>(&xs)[vv] = xv[vv];
-                __builtin_amdgcn_raw_buffer_store_b128(xs, rd_rsrc, vo, j0 * rowb, cpol<NT>());
+                store16<NT>(xs, rd_rsrc, vo + j0 * (int)sizeof(T));   // VEC: rows are adjacent
             } else {
                 bstore<T, NT>(xv[0], rd_rsrc, vo, j0 * rowb);
             }
@@ -842,7 +851,7 @@ __global__ void __launch_bounds__(64 * NW)
                 u32x4 xs;
 #pragma unroll
                 for (int vv = 0; vv < V; ++vv) reinterpret_cast<T *>(&xs)[vv] = xv[vv];
-                __builtin_amdgcn_raw_buffer_store_b128(xs, rd_rsrc, vo, j0 * rowb, cpol<NT>());
+                store16<NT>(xs, rd_rsrc, vo + j0 * (int)sizeof(T));   // VEC: rows are adjacent
             } else {
 #pragma unroll
                 for (int vv = 0; vv < V; ++vv)
