@@ -35,22 +35,28 @@ __device__ __forceinline__ T rowload(__amdgpu_buffer_rsrc_t r, int vo, int64_t r
     return (row >= 0 && row < n) ? bload<T>(r, vo, 0) : T(0);
 }
 
-// Contiguous layout: a wave's rows [wrow, wrow + 64*M) of one system are read as
-// whole 16-byte chunks (consecutive lanes, consecutive chunks; nontemporal) and
-// handed to the lanes through the wave's LDS block `xb`.  Returns the lane's M
-// rows and the values one row before (prev) and one row after (next) its
-// segment, which come from the neighbouring lanes' rows or, at the block edges,
-// from one extra load.  Rows at or past n read as zero.
+// Contiguous layout: a wave's rows [wrow, wrow + 64*M) of one system are read as whole
+// 16-byte chunks (consecutive lanes, consecutive chunks; nontemporal).  The descriptor
+// spans the system's own rows, so chunks that straddle or pass its end need no predicate
+// (the buffer checks each dword: loads past it give zero, stores past it are dropped)
+// and rows may start at any element.
 template <typename T, int M>
-__device__ __forceinline__ void adj_wave_rows(__amdgpu_buffer_rsrc_t r, int64_t wrow, int64_t n,
-                                              int lane, u32x4 *xb, T (&rows)[M], T &prev,
-                                              T &next, bool want_prev, bool want_next) {
+__device__ __forceinline__ void adj_issue(__amdgpu_buffer_rsrc_t r, int64_t wrow, int lane,
+                                          u32x4 (&g)[M * (int)sizeof(T) / 16]) {
+#pragma unroll
+    for (int q = 0; q < M * (int)sizeof(T) / 16; ++q)
+        g[q] = __builtin_amdgcn_raw_buffer_load_b128(r, (int)(wrow * (int64_t)sizeof(T)) + lane * 16,
+                                                     q * 1024, cpol<true>());
+}
+
+// Hands every lane its M rows of the chunks in g through the wave's LDS block `xb`, with
+// the row before (prev) and after (next) its segment: the neighbouring lanes' rows or,
+// at the ends of the block, the given values.
+template <typename T, int M>
+__device__ __forceinline__ void adj_take(const u32x4 (&g)[M * (int)sizeof(T) / 16], int lane,
+                                         u32x4 *xb, T (&rows)[M], T &prev, T &next) {
     constexpr int VV = 16 / (int)sizeof(T);
     constexpr int NQ = M / VV;
-    u32x4 g[NQ];
-#pragma unroll
-    for (int q = 0; q < NQ; ++q)
-        g[q] = tail_chunk_load<T, true>(r, wrow + (int64_t)(q * 64 + lane) * VV, n);
     wave_lds_sync();                                  // the block is free
 #pragma unroll
     for (int q = 0; q < NQ; ++q) xb[q * 64 + lane] = g[q];
@@ -62,24 +68,14 @@ __device__ __forceinline__ void adj_wave_rows(__amdgpu_buffer_rsrc_t r, int64_t 
         for (int v = 0; v < VV; ++v) rows[i * VV + v] = reinterpret_cast<const T *>(&t)[v];
     }
     const T *tb = reinterpret_cast<const T *>(xb);
-    prev = 0;
-    next = 0;
-    if (want_prev) {
-        prev = (lane > 0) ? tb[lane * M - 1] : T(0);
-        const int64_t rp = wrow - 1;
-        if (lane == 0 && rp >= 0 && rp < n) prev = bload<T, true>(r, (int)(rp * (int64_t)sizeof(T)), 0);
-    }
-    if (want_next) {
-        next = (lane < 63) ? tb[lane * M + M] : T(0);
-        const int64_t rn = wrow + 64 * M;
-        if (lane == 63 && rn < n) next = bload<T, true>(r, (int)(rn * (int64_t)sizeof(T)), 0);
-    }
+    if (lane > 0) prev = tb[lane * M - 1];
+    if (lane < 63) next = tb[lane * M + M];
 }
 
 // Writes the lane's M values back as whole 16-byte chunks of the wave block.
 template <typename T, int M>
-__device__ __forceinline__ void adj_wave_store(__amdgpu_buffer_rsrc_t r, int64_t wrow, int64_t n,
-                                               int lane, u32x4 *xb, const T (&vals)[M]) {
+__device__ __forceinline__ void adj_wave_store(__amdgpu_buffer_rsrc_t r, int64_t wrow, int lane,
+                                               u32x4 *xb, const T (&vals)[M]) {
     constexpr int VV = 16 / (int)sizeof(T);
     constexpr int NQ = M / VV;
     wave_lds_sync();
@@ -93,7 +89,8 @@ __device__ __forceinline__ void adj_wave_store(__amdgpu_buffer_rsrc_t r, int64_t
     wave_lds_sync();
 #pragma unroll
     for (int q = 0; q < NQ; ++q)
-        tail_chunk_store<T, true>(xb[q * 64 + lane], r, wrow + (int64_t)(q * 64 + lane) * VV, n);
+        store16<true>(xb[q * 64 + lane], r,
+                      (int)(wrow * (int64_t)sizeof(T)) + lane * 16 + q * 1024);
 }
 
 template <typename T, int M, int NW, int S, bool IL, int MODE>
@@ -123,11 +120,11 @@ __global__ void __launch_bounds__(64 * NW) tile_adj_kernel(AdjParams<T> prm) {
     T c_before, a_after, x_before = 0, x_after = 0;
     __shared__ u32x4 xbuf[IL ? 1 : NW][IL ? 1 : 64 * M * (int)sizeof(T) / 16];
     (void)xbuf;
-    // contiguous: per-wave descriptors on the system's own rows
+    // contiguous: per-wave descriptors on the system's own rows (none of an idle wave)
     const int64_t sbase = IL ? 0 : wave_uniform(sysc * n);
-    const int64_t nn = valid ? n : 0;
+    const int32_t sbytes = valid ? (int32_t)(n * (int64_t)sizeof(T)) : 0;
     const int64_t wrow = (int64_t)ws * 64 * M;
-    auto RW = [&](const T *p) { return make_rsrc(p + sbase, (int32_t)(n * (int64_t)sizeof(T))); };
+    auto RW = [&](const T *p) { return make_rsrc(p + sbase, sbytes); };
     if constexpr (IL) {
         const int64_t rs = prm.rstride;
         const int nb = prm.buf_bytes;
@@ -153,16 +150,44 @@ __global__ void __launch_bounds__(64 * NW) tile_adj_kernel(AdjParams<T> prm) {
             x_after = rowload<T>(RS(prm.x), vo0 + M * rowb, row0 + M, n);
         }
     } else {
+        // Two arrays in flight: the next one is issued while the first goes through LDS.
+        // The kernel streams, so what counts is that loads never drain: one array at a
+        // time and all five at once both lose.  Measured on MI355X, one / two / three /
+        // all arrays in flight (us): FP32 fused 512 x 8192 31.8 / 31.9 / 34.0 / 33.0,
+        // 100 x 40,000 61.7 / 56.5 / 54.8 / 52.4; adjoint 2047 x 2048 29.8 / 28.4 / 29.6
+        // / 30.5, 4096 x 1024 28.5 / 29.5 / 29.7 / 30.8; FP64 adjoint 2048 x 1024 26.5 /
+        // 24.3 / 25.2 / 25.3 (6.2 TB/s).  With a predicate per chunk instead of the
+        // descriptor's bounds (FP64 adjoint 777 x 4000) 62.0, now 43.0; FP32 2047 x 2048
+        // 35.2, now 28.4.
+        constexpr int NQ = M * (int)sizeof(T) / 16;
+        u32x4 g[5][NQ];
+        const T *in[5] = {prm.b, prm.c, prm.a, prm.g, MODE == kFused ? prm.d : prm.x};
         u32x4 *xb = xbuf[wave];
-        T dummy0, dummy1;
-        adj_wave_rows<T, M>(RW(prm.b), wrow, nn, lane, xb, rb, dummy0, dummy1, false, false);
-        adj_wave_rows<T, M>(RW(prm.c), wrow, nn, lane, xb, rc, c_before, dummy1, true, false);
-        adj_wave_rows<T, M>(RW(prm.a), wrow, nn, lane, xb, ra, dummy0, a_after, false, true);
-        adj_wave_rows<T, M>(RW(prm.g), wrow, nn, lane, xb, rg, dummy0, dummy1, false, false);
-        if constexpr (MODE == kFused)
-            adj_wave_rows<T, M>(RW(prm.d), wrow, nn, lane, xb, rx, dummy0, dummy1, false, false);
-        else
-            adj_wave_rows<T, M>(RW(prm.x), wrow, nn, lane, xb, rx, x_before, x_after, true, true);
+        T unused = 0;
+        adj_issue<T, M>(RW(in[0]), wrow, lane, g[0]);
+        adj_issue<T, M>(RW(in[1]), wrow, lane, g[1]);
+        c_before = 0;
+        a_after = 0;
+        if constexpr (NWS > 1) {
+            // the rows just outside the block (past an end of the system: zero); through
+            // LDS and a barrier they were slower (FP64 1024 x 3000 38.2 / 40.5 us)
+            const int before = wrow > 0 ? (int)((wrow - 1) * (int64_t)sizeof(T)) : sbytes;
+            const int after = (int)((wrow + 64 * M) * (int64_t)sizeof(T));
+            c_before = bload<T>(RW(prm.c), before, 0);
+            a_after = bload<T>(RW(prm.a), after, 0);
+            if constexpr (MODE == kAdjoint) {
+                x_before = bload<T>(RW(prm.x), before, 0);
+                x_after = bload<T>(RW(prm.x), after, 0);
+            }
+        }
+        adj_take<T, M>(g[0], lane, xb, rb, unused, unused);
+        adj_issue<T, M>(RW(in[2]), wrow, lane, g[2]);
+        adj_take<T, M>(g[1], lane, xb, rc, c_before, unused);
+        adj_issue<T, M>(RW(in[3]), wrow, lane, g[3]);
+        adj_take<T, M>(g[2], lane, xb, ra, unused, a_after);
+        adj_issue<T, M>(RW(in[4]), wrow, lane, g[4]);
+        adj_take<T, M>(g[3], lane, xb, rg, unused, unused);
+        adj_take<T, M>(g[4], lane, xb, rx, x_before, x_after);
     }
 #pragma unroll
     for (int j = 0; j < M; ++j)
@@ -270,7 +295,7 @@ __global__ void __launch_bounds__(64 * NW) tile_adj_kernel(AdjParams<T> prm) {
             T v[M];
 #pragma unroll
             for (int j = 0; j < M; ++j) v[j] = grad(k, j);
-            adj_wave_store<T, M>(RW(outs[k]), wrow, n, lane, xbuf[wave], v);
+            adj_wave_store<T, M>(RW(outs[k]), wrow, lane, xbuf[wave], v);
         }
     }
 }
