@@ -16,7 +16,8 @@ TOL = {np.float32: 1e-5, np.float64: 1e-12}
 
 # around the tiles' capacities, the wave blocks (64 lanes of 4 or 8 rows) and the chunks
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
-@pytest.mark.parametrize("n", [1, 5, 255, 257, 511, 513, 777, 1023, 1025, 2047, 3001, 4093])
+@pytest.mark.parametrize("n", [1, 5, 255, 257, 383, 385, 511, 513, 767, 777, 1023, 1025, 1535, 1537, 2047,
+                               3001, 3073, 4093, 4097, 6143, 6145])
 @pytest.mark.parametrize("fused", [False, True])
 def test_odd_rows(dtype, n, fused):
     import torch

@@ -162,10 +162,23 @@ def _table_sources(T, suffix):
     return files
 
 
-# Adjoint / fused forward+adjoint kernels: (M, NW, S) per layout.
-# Contiguous shapes keep 512-lane workgroups (8 waves: S systems of 8/S waves),
-# plus 1024 lanes for one system of up to 8192 rows.
-ADJ_C = [(M, 8, S) for M in (4, 8) for S in (8, 4, 2, 1)] + [(M, 16, 1) for M in (4, 8)]
+# Adjoint / fused forward+adjoint kernels: (M, NW, S) per layout; the smallest capacity
+# that holds n runs.  Contiguous shapes: capacities at the powers of two from 256 and,
+# with M = 12, halfway between, so that at most a third of the lanes hold padding.  The
+# fused kernel keeps three coefficient arrays and two solves in registers, so from 12
+# rows per lane (FP64: from 8) it runs smaller workgroups, of which more share a CU.
+# Measured on MI355X at 2^22 (FP64 2^21) unknowns, next power of two -> M = 12: FP32
+# adjoint 1536 rows 32.2 -> 26.8 us, fused 41.3 -> 34.2 (NW = 8: 42.1), 6144 rows 54.3 ->
+# 45.6; FP64 adjoint 768 rows 30.3 -> 27.0, fused 50.2 -> 35.0; M = 8, NW = 8 -> 4: FP64
+# fused 512 rows 36.5 -> 33.5, 1024 rows 40.8 -> 36.3, 2048 rows 41.5 -> 37.1, adjoint
+# 1024 rows 23.7 / 27.6 (stays at 8).
+ADJ_C = {("float", 0): [(4, 8, 8)] + [(M, 8, S) for M in (8, 12) for S in (8, 4, 2, 1)] + [(8, 16, 1)],
+         ("float", 1): [(4, 8, 8)] + [(8, 8, S) for S in (8, 4, 2, 1)] +
+                       [(12, 4, S) for S in (4, 2, 1)] + [(12, 8, 1), (8, 16, 1)],
+         ("double", 0): [(4, 8, 8), (6, 8, 8)] + [(8, 8, S) for S in (8, 4, 2, 1)] +
+                        [(12, 4, S) for S in (4, 2, 1)] + [(12, 8, 1)],
+         ("double", 1): [(4, 8, 8), (6, 8, 8)] + [(M, 4, S) for M in (8, 12) for S in (4, 2, 1)] +
+                        [(8, 8, 1), (12, 8, 1)]}
 ADJ_IL = {"float": [(M, NW, 8) for M in (4, 8) for NW in (1, 2, 4, 8, 16)],
           "double": [(M, NW, 4) for M in (4, 8) for NW in (1, 2, 4, 8, 16)]}
 
@@ -175,22 +188,18 @@ def _adjoint_source():
              '#include "tri_adjoint.hpp"', "", "namespace tri {", ""]
     for T, suffix in (("float", "f32"), ("double", "f64")):
         ents = []
-        for (M, NW, S) in ADJ_C:
-            if T == "double" and NW == 16:
-                continue                         # over the 128-VGPR budget of 1024 lanes
-            ents.append((M, NW, S, False))
+        for mode in (0, 1):
+            ents += [(M, NW, S, False, mode) for (M, NW, S) in ADJ_C[T, mode]]
         for (M, NW, S) in ADJ_IL[T]:
-            if T == "double" and NW == 16:
+            if T == "double" and NW == 16:       # over the 128-VGPR budget of 1024 lanes
                 continue
-            ents.append((M, NW, S, True))
+            ents += [(M, NW, S, True, mode) for mode in (0, 1)]
         lines.append("AdjTable<%s> adj_table_%s() {" % (T, suffix))
         lines.append("    static const AdjEntry<%s> t[] = {" % T)
-        for (M, NW, S, il) in ents:
-            cap = _cap(M, NW, S, il)
-            for mode in (0, 1):
-                lines.append("        {%d, %d, %d, %s, %d, %d, &launch_adj<%s, %d, %d, %d, %s, %d>},"
-                             % (M, NW, S, "true" if il else "false", mode, cap, T, M, NW, S,
-                                "true" if il else "false", mode))
+        for (M, NW, S, il, mode) in ents:
+            lines.append("        {%d, %d, %d, %s, %d, %d, &launch_adj<%s, %d, %d, %d, %s, %d>},"
+                         % (M, NW, S, "true" if il else "false", mode, _cap(M, NW, S, il), T, M,
+                            NW, S, "true" if il else "false", mode))
         lines += ["    };", "    return {t, (int)(sizeof(t) / sizeof(t[0]))};", "}", ""]
     lines += ["}  // namespace tri", ""]
     return "\n".join(lines)
