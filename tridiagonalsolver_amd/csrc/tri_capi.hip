@@ -21,7 +21,7 @@
 
 #include "../../include/tridiagonal.h"
 #include "tri_adjoint.hpp"
-#include "tri_coop.hpp"
+#include "tri_coop_tree.hpp"
 #include "tri_host.hpp"
 #include "tri_large.hpp"
 #include "tri_ragged.hpp"
@@ -450,28 +450,46 @@ static int32_t coop_spread(int groups_per_round) {
     return v != 0 ? groups_per_round : 0;
 }
 
-// The entry of the cooperative table for (layout, n): the first whose blocks
-// divide n (interleaved) and whose kmax holds K = blocks per system (K >= 2);
-// interleaved systems up to 64 blocks (16384 rows).  Contiguous systems take it up to
-// 32 blocks (FP32 131072 rows, FP64 65536): measured on MI355X at 2^24 unknowns
-// against the chunked solve, FP32 20000 rows 0.076 vs 0.113 ms and 131072 rows
-// 0.088 vs 0.107 ms, FP64 20000 rows 0.147 vs 0.209 ms and 65536 rows 0.173 vs
-// 0.206 ms.  Far beyond (2^20 rows, 512 blocks) every group would wait on hundreds
-// of workgroups: an early version ran 1.6 ms against the chunked 0.21 ms.
+// The entry of the cooperative table for a batch, K = blocks per system (K >= 2) and P =
+// workgroups of its grid: the tasks, or as many whole groups as are resident at once.
+//
+// Interleaved: the first entry whose blocks divide n and whose kmax holds K (up to 64
+// blocks, 16384 rows).
+//
+// Contiguous: small blocks up to 64 of them, or where the whole batch is one round of the
+// grid (more CUs per row); large blocks above (fewer forms to read and flags to wait
+// for).  Measured on MI355X, chunked solve / small / large blocks (us): FP32 20,000 x 800
+// 106.6 / 68.2 / 79.8, 131,072 x 128 104.7 / 72.1 / 77.4, 524,288 x 32 105.3 / 88.5 /
+// 80.8, 2^20 x 16 102.7 / 97.0 / 84.4, 500,000 x 1 17.7 / 12.7 / 13.5; FP64 65,536 x 256
+// 205 / 148 / 154, 262,144 x 64 209 / 180 / 163, 2^20 x 16 206 / - / 185, 500,000 x 1
+// 21.3 / 14.3 / 15.8.  The serial chain over the blocks that this replaced stopped at 32
+// (FP32 131,072 x 128 88, FP64 65,536 x 256 173 us).  Where the groups of several rounds
+// fill less than 2/3 (FP32) or 3/4 (FP64) of the resident workgroups the chunked solve is
+// faster (FP64 700,000 x 20, 2/3: 176 / 190 us; 1,500,000 x 8, 0.72: 156 / 171 us; FP32
+// 1,500,000 x 8, 0.72: 79 / 76 us, 2,000,000 x 8, 0.96: 100 / 89 us).
 template <typename T>
-static const CoopEntry<T> *choose_coop(bool il, int64_t n, int &K) {
+static const CoopEntry<T> *choose_coop(bool il, int64_t n, int64_t batch, int &K, int64_t &P) {
     CoopTable<T> tab = coop_table<T>();
     static const int64_t forced = env_int("TRIDIAG_COOP_ENTRY", -1);   // experiments
+    const CoopEntry<T> *best = nullptr;
     for (int i = 0; i < tab.count; ++i) {
         if (forced >= 0 && i != forced) continue;
         const CoopEntry<T> &e = tab.entries[i];
         if (e.IL != il) continue;
         const int64_t k = il ? (n % e.R == 0 ? n / e.R : 0) : (n + e.R - 1) / e.R;
         if (k < 2 || k > e.kmax) continue;
+        const int64_t cap = e.max_grid(il && coop_pipelined(e.pipe) != 0);
+        const int64_t tasks = (batch + e.S - 1) / e.S * k;
+        if (cap < k) continue;
+        const int64_t grid = std::min<int64_t>(tasks, cap / k * k);
+        if (!il && tasks > grid && (sizeof(T) == 4 ? 3 * grid < 2 * cap : 4 * grid < 3 * cap))
+            continue;
+        best = &e;
         K = (int)k;
-        return &e;
+        P = grid;
+        if (il || k <= 64 || tasks <= cap) break;
     }
-    return nullptr;
+    return best;
 }
 
 // Bulk-row form of a reference id (tri_bulk.hip): form 0 PCR-pThomas, 1
@@ -548,7 +566,8 @@ enum PlanKind {
     kPlanThomas = 1,         // the Thomas recurrence (algorithm 1)
     kPlanTile = 2,           // on chip, one workgroup per system or per S systems
     kPlanCoop = 3,           // on chip, K workgroups per group of systems
-    kPlanChunked = 4,        // three passes over chunks through global memory
+    kPlanChunked = 4,        // over chunks: cooperatively where a system's chunks fit on chip
+                             // at once, else three passes through global memory
     kPlanViaContiguous = 5,  // interleaved systems solved through a contiguous copy
     kPlanBulk = 6,           // the reference's own form of ids 2-13 (bulk rows, CR levels)
     kPlanShort = 7,          // several short contiguous systems per wave
@@ -574,23 +593,23 @@ static bool coop_plan(int algo, int layout, int64_t n, int64_t batch, size_t fix
     if (coop_min_rows_il(prec) < 0 || algo_spec(algo).iface != kIfaceWM) return false;
     const bool il = layout == kInterleaved;
     if (il && n < coop_min_rows_il(prec)) return false;
-    int K = 0;
-    const CoopEntry<T> *e = choose_coop<T>(il, n, K);
-    if (!e) return false;
     // interleaved: 32-bit offsets into whole arrays; contiguous: into one system
     const int64_t elems = il ? n * batch : n;
     if (elems * (int64_t)sizeof(T) >= (int64_t)0x7fffff00) return false;
+    // every task of a round must be resident: P workgroups, a multiple of K
+    int K = 0;
+    int64_t P = 0;
+    const CoopEntry<T> *e = choose_coop<T>(il, n, batch, K, P);
+    if (!e) return false;
     const int64_t ngroups = (batch + e->S - 1) / e->S;
     const int64_t ntask = ngroups * K;
     if (ntask > 0x7fffffff) return false;
-    // every task of a round must be resident: P workgroups, a multiple of K
-    const int cap = e->max_grid(coop_pipelined(e->pipe) != 0);
-    if (cap < K) return false;
-    const int64_t P = std::min<int64_t>(ntask, (cap / K) * (int64_t)K);
     const size_t forms = (((size_t)ntask * e->S * 6 * sizeof(T)) + 255) & ~(size_t)255;
-    const size_t bytes = forms + (size_t)ngroups * kCoopFlagStride * sizeof(uint64_t);
+    const size_t words = !il ? 2 * (size_t)ntask : (size_t)ngroups * kCoopFlagStride;
+    const size_t bytes = forms + words * sizeof(uint64_t);
     if (fixed_bytes && bytes > fixed_bytes) return false;
-    pl.kind = kPlanCoop;
+    // (systems of more than 32 blocks report the chunked kind)
+    pl.kind = il || K <= 32 ? kPlanCoop : kPlanChunked;
     pl.coop = e;
     pl.K = K;
     pl.grid = (int)P;
@@ -614,13 +633,22 @@ static int coop_run(const SolvePlan<T> &pl, int layout, int64_t n, int64_t batch
     }
     CoopParams<T> p{a, b, c, d, n, batch, il ? 1 : sstride, il ? batch : 1,
                     (int32_t)(il ? n * batch * (int64_t)sizeof(T) : 0), (int32_t)pl.K,
-                    (int32_t)ngroups, coop_spin_limit(), coop_pipelined(e.pipe),
+                    (int32_t)ngroups,
+                    il ? coop_spin_limit() : std::min(coop_spin_limit(), kCoopTreePolls),
+                    il ? coop_pipelined(e.pipe) : 0,
                     il ? coop_spread(pl.grid / pl.K) : 0, reinterpret_cast<T *>(scratch),
                     reinterpret_cast<uint64_t *>(reinterpret_cast<char *>(scratch) +
                                                  pl.forms_bytes),
-                    coop_next_tag()};
+                    coop_next_tag(), nullptr};
+    if (!il) p.done = p.flags + ngroups * pl.K;
     int rc = TRIDIAG_OK;
-    const hipError_t err = e.launch(p, pl.grid, st);
+    hipError_t err = hipSuccess;
+    // a captured solve is replayed with the tag of its capture, which the words hold
+    // from the second replay on: they are cleared in the graph
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (st && hipStreamIsCapturing(st, &cap) == hipSuccess && cap == hipStreamCaptureStatusActive)
+        err = launch_coop_clear(p.flags, (int64_t)((pl.scratch_bytes - pl.forms_bytes) / sizeof(uint64_t)), st);
+    if (err == hipSuccess) err = e.launch(p, pl.grid, st);
     if (err != hipSuccess) rc = hip_fail(err, "cooperative solve launch");
     if (!fx) {
         const hipError_t ef = hipFreeAsync(scratch, st);
@@ -820,6 +848,7 @@ static int solve_impl(int algo, int layout, int64_t n, int64_t batch, T *a, T *b
     case kPlanCoop:
         return coop_run<T>(pl, layout, n, batch, sstride, a, b, c, d, st, fx);
     case kPlanChunked:
+        if (pl.coop) return coop_run<T>(pl, layout, n, batch, sstride, a, b, c, d, st, fx);
         return large_impl<T>(algo, n, batch, sstride, a, b, c, d, st, fx);
     case kPlanViaContiguous:
         if (fx)

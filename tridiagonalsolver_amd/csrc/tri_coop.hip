@@ -2,83 +2,111 @@
 #include <algorithm>
 #include <mutex>
 
-#include "tri_coop.hpp"
+#include "tri_coop_tree.hpp"
 
 namespace tri {
 
-template <typename T, int M, int NW, int S, bool IL, int KMAX, bool PF, int OCC>
-static hipError_t launch_coop(const CoopParams<T> &p, int grid, hipStream_t st) {
-    if (grid < 1 || p.K < 1 || p.K > KMAX || grid % p.K != 0) return hipErrorInvalidValue;
-    if (p.pipelined)
-        hipLaunchKernelGGL((coop_pipe_kernel<T, M, NW, S, IL, KMAX>), dim3((unsigned)grid),
-                           dim3(64 * NW), 0, st, p);
-    else
-        hipLaunchKernelGGL((coop_kernel<T, M, NW, S, IL, KMAX, PF, OCC>), dim3((unsigned)grid),
-                           dim3(64 * NW), 0, st, p);
-    return hipGetLastError();
-}
-
-// Workgroups of the entry's kernel (pipelined or not) that the current device holds
-// at once (0 if unknown), cached per device.
-template <typename T, int M, int NW, int S, bool IL, int KMAX, bool PF, int OCC>
-static int coop_max_grid(bool pipelined) {
-    constexpr int kDevs = 64;
+// Workgroups of 64 * NW lanes of `fn` that the current device holds at once (0 if
+// unknown); cache[device] keeps the answer.
+static int resident_workgroups(const void *fn, int lanes, int (&cache)[64]) {
     static std::mutex mu;
-    static int cache[kDevs][2] = {};
     int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kDevs) return 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
     std::lock_guard<std::mutex> lk(mu);
-    int &c = cache[dev][pipelined ? 1 : 0];
+    int &c = cache[dev];
     if (c == 0) {
         int per_cu = 0, cus = 0;
-        const void *fn = pipelined
-            ? reinterpret_cast<const void *>(coop_pipe_kernel<T, M, NW, S, IL, KMAX>)
-            : reinterpret_cast<const void *>(coop_kernel<T, M, NW, S, IL, KMAX, PF, OCC>);
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, 64 * NW, 0) != hipSuccess)
-            return 0;
-        if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, lanes, 0) != hipSuccess ||
+            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
             return 0;
         c = per_cu * cus;
     }
     return c;
 }
 
-#define TRI_COOP_ENTRY(T, M, NW, S, IL, KMAX, PIPE, PF, OCC)                                 \
-    {M, NW, S, IL, CoopShape<T, M, NW, S, IL>::R, KMAX, PIPE,                                 \
-     &launch_coop<T, M, NW, S, IL, KMAX, PF, OCC>, &coop_max_grid<T, M, NW, S, IL, KMAX, PF, OCC>}
+// Interleaved systems.
+template <typename T, int M, int NW, int S, int KMAX, int OCC>
+static hipError_t launch_coop(const CoopParams<T> &p, int grid, hipStream_t st) {
+    if (grid < 1 || p.K < 1 || p.K > KMAX || grid % p.K != 0) return hipErrorInvalidValue;
+    if (p.pipelined)
+        hipLaunchKernelGGL((coop_pipe_kernel<T, M, NW, S, KMAX>), dim3((unsigned)grid),
+                           dim3(64 * NW), 0, st, p);
+    else
+        hipLaunchKernelGGL((coop_kernel<T, M, NW, S, KMAX, OCC>), dim3((unsigned)grid),
+                           dim3(64 * NW), 0, st, p);
+    return hipGetLastError();
+}
+template <typename T, int M, int NW, int S, int KMAX, int OCC>
+static int coop_max_grid(bool pipelined) {
+    static int cache[2][64];
+    const void *fn = pipelined
+        ? reinterpret_cast<const void *>(coop_pipe_kernel<T, M, NW, S, KMAX>)
+        : reinterpret_cast<const void *>(coop_kernel<T, M, NW, S, KMAX, OCC>);
+    return resident_workgroups(fn, 64 * NW, cache[pipelined ? 1 : 0]);
+}
+
+// Contiguous systems: the solve, and the pass over blocks whose wait gave up.
+template <typename T, int M, int NW, int OCC>
+static hipError_t launch_coop_tree(const CoopParams<T> &p, int grid, hipStream_t st) {
+    if (grid < 1 || p.K < 1 || p.K > 64 * NW || grid % p.K != 0) return hipErrorInvalidValue;
+    hipLaunchKernelGGL((coop_tree_kernel<T, M, NW, OCC>), dim3((unsigned)grid), dim3(64 * NW), 0,
+                       st, p);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL((coop_mend_kernel<T, M, NW, OCC>), dim3((unsigned)std::min(grid, 256)),
+                       dim3(64 * NW), 0, st, p);
+    return hipGetLastError();
+}
+template <typename T, int M, int NW, int OCC> static int coop_tree_max_grid(bool) {
+    static int cache[64];
+    return resident_workgroups(reinterpret_cast<const void *>(coop_tree_kernel<T, M, NW, OCC>),
+                               64 * NW, cache);
+}
+
+__global__ void __launch_bounds__(256) coop_clear_kernel(uint64_t *w, int64_t count) {
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < count; i += (int64_t)gridDim.x * 256)
+        w[i] = 0;
+}
+hipError_t launch_coop_clear(uint64_t *words, int64_t count, hipStream_t st) {
+    hipLaunchKernelGGL(coop_clear_kernel, dim3((unsigned)std::min<int64_t>((count + 255) / 256, 256)),
+                       dim3(256), 0, st, words, count);
+    return hipGetLastError();
+}
+
+#define TRI_COOP_ENTRY(T, M, NW, S, KMAX, PIPE, OCC)                                          \
+    {M, NW, S, true, CoopShape<T, M, NW, S>::R, KMAX, PIPE, &launch_coop<T, M, NW, S, KMAX, OCC>, \
+     &coop_max_grid<T, M, NW, S, KMAX, OCC>}
+#define TRI_COOP_TREE(T, M, NW, OCC)                                                          \
+    {M, NW, 1, false, 64 * NW * M, 64 * NW, false, &launch_coop_tree<T, M, NW, OCC>,           \
+     &coop_tree_max_grid<T, M, NW, OCC>}
 
 // Interleaved: S systems = one 128-byte line per row, blocks of 2*NW*M (FP32) or
 // 4*NW*M (FP64) rows, up to 32 blocks, and an entry for 33-64 blocks whose larger
 // block-form staging leaves one workgroup per CU (interleaved 12288 / 16384 rows x
 // 1024: FP32 0.129 / 0.167 ms, FP64 0.266 / 0.367 ms, against 0.164 / 0.213 and
-// 0.363 / 0.477 ms through a contiguous copy).  Contiguous: one system, blocks of
-// 64*NW*M rows, up to 32 blocks (a group of 64 measured slower than the chunked
-// solve).  PIPE: coop_pipe_kernel by default; PF: the
-// next block in flight in registers; OCC: waves per SIMD.
-// Measured on MI355X (ms; 16.7 M unknowns unless noted):
-//   interleaved  FP32 4096 x 4096: PF, 1 workgroup per CU 0.117; pipelined 0.109;
-//                no PF, 2 per CU (OCC 4) 0.108.  FP32 2048 x 8192: 0.102 / 0.091
-//                (pipelined / OCC 4); 8192 x 2048: 0.129 / 0.123.  FP64 4096 x
-//                4096: 0.233 / 0.223 / 0.214 (PF / pipelined / OCC 4).  Blocks of
-//                128 rows (M = 8 FP32, 4 FP64) with K = 32: 0.148 / 0.282; 16-wave
-//                workgroups of M = 8 / 4 (no spills, one per CU): 0.133 / 0.286.
-//   contiguous   FP32 20000 rows: PF OCC 2 0.083, OCC 4 0.082, OCC 3 0.076;
-//                131072 rows (32 blocks): OCC 4 0.093, OCC 3 0.088, chunked 0.107.
-//                FP64 20000 rows: PF OCC 2 0.180, OCC 4 0.147, OCC 3 0.151, chunked
-//                0.209; 65536 x 256 (32 blocks): OCC 4 0.173, chunked 0.206.
-// The register prefetch costs more occupancy than it hides latency; more
-// workgroups per CU keep more loads in flight, even where the kernel spills.
+// 0.363 / 0.477 ms through a contiguous copy).  PIPE: coop_pipe_kernel by default;
+// OCC: waves per SIMD.
+// Measured on MI355X (ms; 16.7 M unknowns):
+//   FP32 4096 x 4096: pipelined 0.109; no prefetch, 2 per CU (OCC 4) 0.108.  FP32
+//   2048 x 8192: 0.102 / 0.091 (pipelined / OCC 4); 8192 x 2048: 0.129 / 0.123.  FP64
+//   4096 x 4096: 0.223 / 0.214.  Blocks of 128 rows (M = 8 FP32, 4 FP64) with K = 32:
+//   0.148 / 0.282; 16-wave workgroups of M = 8 / 4 (one per CU): 0.133 / 0.286.
+// Contiguous: one system, blocks of 64*NW*M rows, up to 64*NW blocks; small blocks
+// first (choose_coop says which).  Both run 16 waves per CU, four or two workgroups.
 static const CoopEntry<float> kCoopF32[] = {
-    TRI_COOP_ENTRY(float, 16, 8, 32, true, 32, false, false, 4),
-    TRI_COOP_ENTRY(float, 16, 8, 32, true, 64, false, false, 4),
-    TRI_COOP_ENTRY(float, 16, 4, 1, false, 32, false, false, 3),
+    TRI_COOP_ENTRY(float, 16, 8, 32, 32, false, 4),
+    TRI_COOP_ENTRY(float, 16, 8, 32, 64, false, 4),
+    TRI_COOP_TREE(float, 16, 4, 4),
+    TRI_COOP_TREE(float, 16, 8, 4),
 };
 static const CoopEntry<double> kCoopF64[] = {
-    TRI_COOP_ENTRY(double, 8, 8, 16, true, 32, false, false, 4),
-    TRI_COOP_ENTRY(double, 8, 8, 16, true, 64, false, false, 4),
-    TRI_COOP_ENTRY(double, 8, 4, 1, false, 32, false, false, 4),
+    TRI_COOP_ENTRY(double, 8, 8, 16, 32, false, 4),
+    TRI_COOP_ENTRY(double, 8, 8, 16, 64, false, 4),
+    TRI_COOP_TREE(double, 8, 4, 4),
+    TRI_COOP_TREE(double, 8, 8, 4),
 };
 #undef TRI_COOP_ENTRY
+#undef TRI_COOP_TREE
 
 CoopTable<float> coop_table_f32() { return {kCoopF32, (int)(sizeof(kCoopF32) / sizeof(kCoopF32[0]))}; }
 CoopTable<double> coop_table_f64() {

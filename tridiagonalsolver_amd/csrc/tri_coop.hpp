@@ -3,9 +3,12 @@
 // together, each keeping its own block on chip from load to store (5 words of
 // HBM traffic per unknown).
 //
+// This file: interleaved systems, and what both layouts share.  Contiguous systems:
+// tri_coop_tree.hpp.
+//
 //   task (g, j) = rows [j*R, (j+1)*R) of the S systems of group g
-//     1. the block's rows (interleaved: whole row pieces of S*sizeof(T) bytes;
-//        contiguous: whole 16-byte chunks) go to the lanes through LDS; lane
+//     1. the block's rows (whole row pieces of S*sizeof(T) bytes) go to the lanes
+//        through LDS; lane
 //        sweeps, Wang-Mou merges inside each wave and a fold over the waves give
 //        the block's first row F and last row E in outer form relative to
 //        U = x of the row before the block and V = x of the row after it
@@ -21,12 +24,9 @@
 // device holds, and a multiple of K), and workgroup w takes tasks w, w + P,
 // w + 2P, ...  The K tasks of a slot are consecutive, so they fall in the same
 // round and every member publishes before it waits: with all P workgroups
-// resident, every wait ends.  Slot s solves group s of a contiguous batch; in an
-// interleaved batch the slots of a round take groups spread over the whole batch
-// (coop_group), so that a round reads whole interleaved rows rather than a strip.  Each workgroup keeps the next round's block in
-// flight (in registers) while it waits and finishes the current task, so the
-// memory system stays busy while groups wait for their slowest member.  Every
-// wait is still bounded (spin_limit polls): a workgroup whose partners do not
+// resident, every wait ends.  The slots of a round take groups spread over the whole
+// batch (coop_group), so that a round reads whole interleaved rows rather than a strip.
+// Every wait is still bounded (spin_limit polls): a workgroup whose partners do not
 // publish in time (which needs another kernel to hold CUs that this grid
 // counted on) gives up and writes NaN for x of its block, so the kernel always
 // ends and a lost wait shows in the result rather than as a wrong finite value.
@@ -70,6 +70,7 @@ template <typename T> struct CoopParams {
     T *forms;            // [ngroups][K][S][6] block outer forms
     uint64_t *flags;     // [kCoopFlagStride * g + j]: the tag once block j of group g is published
     uint64_t tag;        // this solve's tag: different from every earlier solve's
+    uint64_t *done;      // coop_tree_kernel: the tag once block t of the grid is solved
 };
 
 // Publication flags: one 8-byte word per block of a group (up to 64 blocks), the
@@ -84,16 +85,13 @@ constexpr int kCoopFlagStride = 64;
 #define TRI_COOP_POLL_SLEEP 8
 #endif
 
-// Group solved by slot s: interleaved groups are spread over the batch within a
-// round (coop_group); contiguous groups hold one system each and keep slot order.
-template <bool IL, typename T>
-__device__ __forceinline__ int coop_gi(const CoopParams<T> &p, int s) {
-    if constexpr (IL) return coop_group(s, p.ngroups, p.spread);
-    else return s;
+// Group solved by slot s: a round's groups are spread over the batch (coop_group).
+template <typename T> __device__ __forceinline__ int coop_gi(const CoopParams<T> &p, int s) {
+    return coop_group(s, p.ngroups, p.spread);
 }
 
-template <typename T, int M, int NW, int S, bool IL> struct CoopShape {
-    static constexpr int SW = IL ? 64 / S : 64;      // segments of a system per wave
+template <typename T, int M, int NW, int S> struct CoopShape {
+    static constexpr int SW = 64 / S;                // segments of a system per wave
     static constexpr int R = SW * NW * M;            // rows per block
 };
 
@@ -197,28 +195,6 @@ __device__ __forceinline__ void chain_with_ends(T (*blk)[6], T (*uv)[2], int nw,
     }
 }
 
-// Contiguous-layout stores of x: the wave's 64*M rows as whole 16-byte chunks
-// through LDS, rows past the system not written.
-template <typename T, int M, bool NT>
-__device__ __forceinline__ void contig_block_store(__amdgpu_buffer_rsrc_t rd, int64_t wrow,
-                                                   int64_t len, int lane, u32x4 *xb,
-                                                   const T (&xs)[M]) {
-    constexpr int VV = 16 / (int)sizeof(T);
-    constexpr int NQ = M / VV;
-    wave_lds_sync();
-#pragma unroll
-    for (int i = 0; i < NQ; ++i) {
-        u32x4 t;
-#pragma unroll
-        for (int v = 0; v < VV; ++v) reinterpret_cast<T *>(&t)[v] = xs[i * VV + v];
-        xb[lane * NQ + i] = t;
-    }
-    wave_lds_sync();
-#pragma unroll
-    for (int q = 0; q < NQ; ++q)
-        tail_chunk_store<T, NT>(xb[q * 64 + lane], rd, wrow + (int64_t)(q * 64 + lane) * VV, len);
-}
-
 // block_chain (below) one block at a time: the form the FP64 kernels take.
 template <typename T>
 __device__ __forceinline__ void block_chain_serial(T (*blk)[6], int K, int j, T &U, T &V) {
@@ -307,77 +283,22 @@ __device__ __forceinline__ void block_chain(T (*blk)[6], int K, int j, T &U, T &
     for (; k >= j; --k) bwd(k, blk[k][0], blk[k][1], blk[k][2], blk[k][3]);
 }
 
-// Contiguous blocks: whole 16-byte chunks of the wave's 64*M rows, issued
-// unconditionally (the buffer ends at the system's last row, so chunks past it
-// read as zero).
-template <typename T, int M, bool NT>
-__device__ __forceinline__ void contig_block_issue(const __amdgpu_buffer_rsrc_t (&rr)[4], int64_t wrow,
-                                                   int lane, u32x4 (&g)[4][M * (int)sizeof(T) / 16]) {
-    constexpr int VV = 16 / (int)sizeof(T);
-    constexpr int NQ = M / VV;
-#pragma unroll
-    for (int q = 0; q < NQ; ++q)
-#pragma unroll
-        for (int k = 0; k < 4; ++k)
-            g[k][q] = __builtin_amdgcn_raw_buffer_load_b128(
-                rr[k], (int)((wrow + (int64_t)(q * 64 + lane) * VV) * (int64_t)sizeof(T)), 0,
-                cpol<NT>());
+template <typename T>
+__device__ __forceinline__ void coop_rsrc(const CoopParams<T> &p, __amdgpu_buffer_rsrc_t (&rr)[4]) {
+    rr[0] = make_rsrc(p.a, p.buf_bytes); rr[1] = make_rsrc(p.b, p.buf_bytes);
+    rr[2] = make_rsrc(p.c, p.buf_bytes); rr[3] = make_rsrc(p.d, p.buf_bytes);
 }
 
-template <typename T, int M>
-__device__ __forceinline__ void contig_block_transpose(const u32x4 (&g)[4][M * (int)sizeof(T) / 16],
-                                                       int lane, u32x4 *xb, T (&rows)[4][M]) {
-    constexpr int VV = 16 / (int)sizeof(T);
-    constexpr int NQ = M / VV;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        if (k > 0) wave_lds_sync();
-#pragma unroll
-        for (int q = 0; q < NQ; ++q) xb[q * 64 + lane] = g[k][q];
-        wave_lds_sync();
-#pragma unroll
-        for (int i = 0; i < NQ; ++i) {
-            const u32x4 t = xb[lane * NQ + i];
-#pragma unroll
-            for (int v = 0; v < VV; ++v) rows[k][i * VV + v] = reinterpret_cast<const T *>(&t)[v];
-        }
-    }
-}
-
-// Buffers of one task: interleaved, the whole arrays; contiguous, from the
-// block's first row to the system's last row.
-template <typename T, bool IL>
-__device__ __forceinline__ void coop_rsrc(const CoopParams<T> &p, int g, int64_t brow,
-                                          __amdgpu_buffer_rsrc_t (&rr)[4]) {
-    if constexpr (IL) {
-        rr[0] = make_rsrc(p.a, p.buf_bytes); rr[1] = make_rsrc(p.b, p.buf_bytes);
-        rr[2] = make_rsrc(p.c, p.buf_bytes); rr[3] = make_rsrc(p.d, p.buf_bytes);
-    } else {
-        const int64_t base = (int64_t)g * p.sstride + brow;
-        const int32_t bytes = (int32_t)((p.n - brow) * (int64_t)sizeof(T));
-        rr[0] = make_rsrc(p.a + base, bytes); rr[1] = make_rsrc(p.b + base, bytes);
-        rr[2] = make_rsrc(p.c + base, bytes); rr[3] = make_rsrc(p.d + base, bytes);
-    }
-}
-
-// PF: the next task's block is loaded into registers while this one finishes;
 // OCC: waves per SIMD the kernel is built for (its register budget).
-template <typename T, int M, int NW, int S, bool IL, int KMAX, bool PF, int OCC>
+template <typename T, int M, int NW, int S, int KMAX, int OCC>
 __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(OCC)))
     coop_kernel(CoopParams<T> p) {
-    using Sh = TileShape<T, M, NW, S, IL, !IL, false, false, !IL, true, true>;
-    constexpr int SW = IL ? 64 / S : 64;     // segments of a system per wave
+    using Sh = TileShape<T, M, NW, S, true, false, false, false, false, true, true>;
+    constexpr int SW = 64 / S;               // segments of a system per wave
     constexpr int R = SW * NW * M;           // rows per block
     constexpr int NQ = M * (int)sizeof(T) / 16;
-    static_assert(IL || S == 1, "contiguous groups hold one system");
-    static_assert(IL ? (S * (int)sizeof(T)) % 16 == 0 : M % (16 / (int)sizeof(T)) == 0,
-                  "blocks move whole 16-byte chunks");
+    static_assert((S * (int)sizeof(T)) % 16 == 0, "blocks move whole 16-byte chunks");
     static_assert(KMAX <= kCoopFlagStride, "a group's flags fit its flag words");
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int sl = IL ? lane % S : 0;        // system of the lane inside the group
-    const int kw = IL ? lane / S : lane;     // segment inside the wave-block
-    const int ws = wave;                     // wave-block inside the block
-    const int64_t wrow = (int64_t)ws * SW * M;   // first row of the wave-block, in the block
     __shared__ u32x4 xbuf[NW][64 * M * (int)sizeof(T) / 16];
     __shared__ T sh_blk[S][NW][6];
     __shared__ T sh_uv[S][NW][2];
@@ -388,36 +309,25 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(OC
     const int P = (int)gridDim.x;
     const int ntask = p.ngroups * K;
     const int64_t n = p.n;
-    int task = (int)blockIdx.x;
-    u32x4 g[4][NQ];
-    auto issue = [&](int t) {
-        const int s0 = t / K, j0 = t - s0 * K;
-        const int g0 = coop_gi<IL>(p, s0);
-        __amdgpu_buffer_rsrc_t rr[4];
-        coop_rsrc<T, IL>(p, g0, (int64_t)j0 * R, rr);
-        if constexpr (IL) il_block_issue<T, M, SW, S, true>(rr, (int64_t)j0 * R + wrow, p.rstride,
-                                                            (int64_t)g0 * S, lane, g);
-        else contig_block_issue<T, M, true>(rr, wrow, lane, g);
-    };
-    if (PF && task < ntask) issue(task);
-    for (; task < ntask; task += P) {
-        if constexpr (!PF) issue(task);
+    for (int task = (int)blockIdx.x; task < ntask; task += P) {
+        // an opaque copy: lane-dependent addresses and masks stay inside the task loop
+        // instead of occupying registers across it
+        int tid = threadIdx.x;
+        asm volatile("" : "+v"(tid));
+        const int lane = tid & 63, wave = tid >> 6;
+        const int sl = lane % S;             // system of the lane inside the group
+        const int kw = lane / S;             // segment inside the wave-block
+        const int ws = wave;                 // wave-block inside the block
+        const int64_t wrow = (int64_t)ws * SW * M;   // first row of the wave-block, in the block
         const int si = task / K, j = task - si * K;
-        const int gi = coop_gi<IL>(p, si);
+        const int gi = coop_gi(p, si);
         const int64_t brow = (int64_t)j * R;               // first row of the block
         const int64_t row0 = brow + wrow + (int64_t)kw * M;   // first row of the lane
-        const int64_t len = IL ? R : ((n - brow < R) ? n - brow : R);
+        __amdgpu_buffer_rsrc_t rr[4];
+        coop_rsrc(p, rr);
         T rows[4][M];
-        if constexpr (IL) {
-            il_block_transpose<T, M, S>(g, lane, sl, kw, xbuf[wave], rows);
-        } else {
-            contig_block_transpose<T, M>(g, lane, xbuf[wave], rows);
-#pragma unroll
-            for (int q = 0; q < M; ++q)
-                if (wrow + kw * M + q >= len) {   // identity rows past the system
-                    rows[0][q] = 0; rows[1][q] = 1; rows[2][q] = 0; rows[3][q] = 0;
-                }
-        }
+        il_block_load<T, M, SW, S, true>(rr, brow + wrow, p.rstride, (int64_t)gi * S, lane, sl, kw,
+                                         xbuf[wave], rows);
         // lane sweep; global row numbers drop a_0 and c_{n-1}
         T al_r[Sh::NI];
         SweepOut<T, Sh::NI> o;
@@ -427,7 +337,7 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(OC
         const T ARr = -(o.aR * o.alp), DRr = o.bR - o.aR * o.g, FRr = o.dR - o.aR * o.del;
         Outer<T> oL, oR;
         segment_outer(o.aL, DLr, ELr, FLr, ARr, DRr, o.cR, FRr, oL, oR);
-        wm_wave_merges<T, SW, (IL ? S : 1)>(oL, oR, lane, sl, kw, SW, false, nullptr);
+        wm_wave_merges<T, SW, S>(oL, oR, lane, sl, kw, SW, false, nullptr);
         if (kw == 0) { sh_blk[sl][ws][0] = oL.r; sh_blk[sl][ws][1] = oL.p; sh_blk[sl][ws][2] = oL.q; }
         if (kw == SW - 1) { sh_blk[sl][ws][3] = oR.r; sh_blk[sl][ws][4] = oR.p; sh_blk[sl][ws][5] = oR.q; }
         __syncthreads();
@@ -449,8 +359,6 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(OC
         if (tid == 0)
             __hip_atomic_store(p.flags + kCoopFlagStride * gi + j, p.tag, __ATOMIC_RELAXED,
                                __HIP_MEMORY_SCOPE_AGENT);
-        // the next round's block streams in while this group completes
-        if (PF && task + P < ntask) issue(task + P);
         if (tid < 64) {
             const int okw = coop_wait(p, gi, tid);
             if (tid == 0) s_ok = okw;
@@ -481,13 +389,8 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(OC
 #pragma unroll
             for (int q = 0; q < M; ++q) xs[q] = __builtin_nan("");
         }
-        __amdgpu_buffer_rsrc_t rw[4];
-        coop_rsrc<T, IL>(p, gi, brow, rw);
-        if constexpr (IL)
-            il_block_store<T, M, SW, S, true>(rw[3], brow + wrow, p.rstride, (int64_t)gi * S,
-                                              p.batch, lane, sl, kw, xbuf[wave], xs);
-        else
-            contig_block_store<T, M, true>(rw[3], wrow, len, lane, xbuf[wave], xs);
+        il_block_store<T, M, SW, S, true>(rr[3], brow + wrow, p.rstride, (int64_t)gi * S, p.batch,
+                                          lane, sl, kw, xbuf[wave], xs);
         __syncthreads();                           // LDS of this task free before the next
     }
 }
@@ -495,19 +398,17 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(OC
 // Back-substitution of one task once its group has published: waits for the K
 // block forms of group gi, chains them to U, V of block j, chains the wave-blocks
 // (blk: this task's wave-block forms, overwritten) and stores x of the block.
-template <typename T, int M, int NW, int S, bool IL, int KMAX, int NI>
+template <typename T, int M, int NW, int S, int KMAX, int NI>
 __device__ __forceinline__ void coop_finish(const CoopParams<T> &p, int gi, int j, T (*blk)[NW][6],
                                             T (*sh_uv)[NW][2], T (*sh_k)[KMAX][6], int *s_ok,
                                             u32x4 *xb, int tid, int lane, int sl, int kw, int ws,
                                             int64_t wrow, const Outer<T> &oL, const Outer<T> &oR,
                                             const T (&de)[NI], const T (&ga)[NI],
                                             const T (&al)[NI]) {
-    constexpr int SW = IL ? 64 / S : 64;
+    constexpr int SW = 64 / S;
     constexpr int R = SW * NW * M;
     const int K = p.K;
-    const int64_t n = p.n;
     const int64_t brow = (int64_t)j * R;
-    const int64_t len = IL ? R : ((n - brow < R) ? n - brow : R);
     const T *fg = p.forms + (int64_t)gi * K * S * 6;
     if (tid < 64) {
         const int ok = coop_wait(p, gi, tid);
@@ -540,12 +441,9 @@ __device__ __forceinline__ void coop_finish(const CoopParams<T> &p, int gi, int 
         for (int q = 0; q < M; ++q) xs[q] = __builtin_nan("");
     }
     __amdgpu_buffer_rsrc_t rw[4];
-    coop_rsrc<T, IL>(p, gi, brow, rw);
-    if constexpr (IL)
-        il_block_store<T, M, SW, S, true>(rw[3], brow + wrow, p.rstride, (int64_t)gi * S, p.batch,
-                                          lane, sl, kw, xb, xs);
-    else
-        contig_block_store<T, M, true>(rw[3], wrow, len, lane, xb, xs);
+    coop_rsrc(p, rw);
+    il_block_store<T, M, SW, S, true>(rw[3], brow + wrow, p.rstride, (int64_t)gi * S, p.batch,
+                                      lane, sl, kw, xb, xs);
     __syncthreads();                           // LDS of this task free
 }
 
@@ -557,18 +455,17 @@ __device__ __forceinline__ void coop_finish(const CoopParams<T> &p, int gi, int 
 // Every wait for task t still comes after the workgroup has published task t + P,
 // and every member of a group publishes it before waiting on anything later, so
 // with all P workgroups resident every wait ends.
-template <typename T, int M, int NW, int S, bool IL, int KMAX>
+template <typename T, int M, int NW, int S, int KMAX>
 __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)))
     coop_pipe_kernel(CoopParams<T> p) {
-    using Sh = TileShape<T, M, NW, S, IL, !IL, false, false, !IL, true, true>;
-    constexpr int SW = IL ? 64 / S : 64;
+    using Sh = TileShape<T, M, NW, S, true, false, false, false, false, true, true>;
+    constexpr int SW = 64 / S;
     constexpr int R = SW * NW * M;
     constexpr int NQ = M * (int)sizeof(T) / 16;
     constexpr int NI = Sh::NI;
-    static_assert(IL || S == 1, "contiguous groups hold one system");
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int sl = IL ? lane % S : 0;
-    const int kw = IL ? lane / S : lane;
+    const int sl = lane % S;
+    const int kw = lane / S;
     const int ws = wave;
     const int64_t wrow = (int64_t)ws * SW * M;
     __shared__ u32x4 xbuf[NW][64 * M * (int)sizeof(T) / 16];
@@ -585,12 +482,11 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)
     u32x4 g[4][NQ];
     if (task < ntask) {
         const int s0 = task / K, j0 = task - s0 * K;
-        const int g0 = coop_gi<IL>(p, s0);
+        const int g0 = coop_gi(p, s0);
         __amdgpu_buffer_rsrc_t rr[4];
-        coop_rsrc<T, IL>(p, g0, (int64_t)j0 * R, rr);
-        if constexpr (IL) il_block_issue<T, M, SW, S, true>(rr, (int64_t)j0 * R + wrow, p.rstride,
-                                                            (int64_t)g0 * S, lane, g);
-        else contig_block_issue<T, M, true>(rr, wrow, lane, g);
+        coop_rsrc(p, rr);
+        il_block_issue<T, M, SW, S, true>(rr, (int64_t)j0 * R + wrow, p.rstride, (int64_t)g0 * S,
+                                          lane, g);
     }
     // the pending task: published, not yet finished
     int pend = -1, par = 0;
@@ -598,21 +494,11 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)
     T pde[NI], pga[NI], pal[NI];
     for (; task < ntask; task += P) {
         const int si = task / K, j = task - si * K;
-        const int gi = coop_gi<IL>(p, si);
+        const int gi = coop_gi(p, si);
         const int64_t brow = (int64_t)j * R;
         const int64_t row0 = brow + wrow + (int64_t)kw * M;
-        const int64_t len = IL ? R : ((n - brow < R) ? n - brow : R);
         T rows[4][M];
-        if constexpr (IL) {
-            il_block_transpose<T, M, S>(g, lane, sl, kw, xbuf[wave], rows);
-        } else {
-            contig_block_transpose<T, M>(g, lane, xbuf[wave], rows);
-#pragma unroll
-            for (int q = 0; q < M; ++q)
-                if (wrow + kw * M + q >= len) {
-                    rows[0][q] = 0; rows[1][q] = 1; rows[2][q] = 0; rows[3][q] = 0;
-                }
-        }
+        il_block_transpose<T, M, S>(g, lane, sl, kw, xbuf[wave], rows);
         T al_r[NI];
         SweepOut<T, NI> o;
         RegLoader<T, Sh::CH, M> ld{rows};
@@ -621,7 +507,7 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)
         const T ARr = -(o.aR * o.alp), DRr = o.bR - o.aR * o.g, FRr = o.dR - o.aR * o.del;
         Outer<T> oL, oR;
         segment_outer(o.aL, DLr, ELr, FLr, ARr, DRr, o.cR, FRr, oL, oR);
-        wm_wave_merges<T, SW, (IL ? S : 1)>(oL, oR, lane, sl, kw, SW, false, nullptr);
+        wm_wave_merges<T, SW, S>(oL, oR, lane, sl, kw, SW, false, nullptr);
         if (kw == 0) {
             sh_blk[par][sl][ws][0] = oL.r; sh_blk[par][sl][ws][1] = oL.p; sh_blk[par][sl][ws][2] = oL.q;
         }
@@ -647,16 +533,15 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)
         const int next = task + P;
         if (next < ntask) {
             const int s1 = next / K, j1 = next - s1 * K;
-            const int g1 = coop_gi<IL>(p, s1);
+            const int g1 = coop_gi(p, s1);
             __amdgpu_buffer_rsrc_t rr[4];
-            coop_rsrc<T, IL>(p, g1, (int64_t)j1 * R, rr);
-            if constexpr (IL) il_block_issue<T, M, SW, S, true>(rr, (int64_t)j1 * R + wrow,
-                                                                p.rstride, (int64_t)g1 * S, lane, g);
-            else contig_block_issue<T, M, true>(rr, wrow, lane, g);
+            coop_rsrc(p, rr);
+            il_block_issue<T, M, SW, S, true>(rr, (int64_t)j1 * R + wrow, p.rstride,
+                                              (int64_t)g1 * S, lane, g);
         }
         if (pend >= 0) {
             const int ps = pend / K;
-            coop_finish<T, M, NW, S, IL, KMAX, NI>(p, coop_gi<IL>(p, ps),
+            coop_finish<T, M, NW, S, KMAX, NI>(p, coop_gi(p, ps),
                                                    pend - ps * K, sh_blk[par ^ 1], sh_uv,
                                                    sh_k, &s_ok, xbuf[wave], tid, lane, sl, kw, ws,
                                                    wrow, poL, poR, pde, pga, pal);
@@ -674,7 +559,7 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)
     }
     if (pend >= 0) {
         const int ps = pend / K;
-        coop_finish<T, M, NW, S, IL, KMAX, NI>(p, coop_gi<IL>(p, ps), pend - ps * K,
+        coop_finish<T, M, NW, S, KMAX, NI>(p, coop_gi(p, ps), pend - ps * K,
                                                sh_blk[par ^ 1], sh_uv, sh_k,
                                                &s_ok, xbuf[wave], tid, lane, sl, kw, ws, wrow, poL,
                                                poR, pde, pga, pal);
@@ -684,7 +569,7 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)
 
 template <typename T> struct CoopEntry {
     int M, NW, S;
-    bool IL;
+    bool IL;     // interleaved: coop_kernel; contiguous: coop_tree_kernel
     int R;       // rows per block
     int kmax;    // most blocks per system (LDS for the block chain)
     bool pipe;   // coop_pipe_kernel by default
@@ -697,5 +582,7 @@ template <typename T> struct CoopTable {
 };
 CoopTable<float> coop_table_f32();
 CoopTable<double> coop_table_f64();
+// Sets `count` words to zero (flags of a solve recorded into a graph).
+hipError_t launch_coop_clear(uint64_t *words, int64_t count, hipStream_t st);
 
 }  // namespace tri
