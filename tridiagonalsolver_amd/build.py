@@ -59,6 +59,12 @@ IL_SHAPES = {
                if not (M == 32 and NW == 16)] + [(16, 8, 2), (8, 16, 2)] +
               [(8, 16, 16), (16, 8, 16), (8, 8, 16), (16, 16, 8), (8, 16, 8)],
 }
+# Interleaved shapes built only as tiles that read whole 128-byte row pieces: the
+# capacities between those of IL_SHAPES, so that short columns waste few lanes.
+IL_XP_SHAPES = {
+    "float": [(8, 2, 32), (12, 2, 32), (8, 4, 32), (12, 4, 32), (12, 8, 32), (12, 16, 32)],
+    "double": [(8, 1, 16), (6, 2, 16), (8, 2, 16), (6, 4, 16), (8, 4, 16), (12, 4, 16), (12, 8, 16)],
+}
 C_SHAPES = {
     "float": [(M, NW, S) for (NW, S) in ((4, 4), (4, 2), (4, 1), (8, 1), (16, 1))
               for M in (2, 4, 8, 16, 32) if not (M == 32 and NW == 16)] +
@@ -80,6 +86,12 @@ BIG_IL = {(8, 8), (16, 8)}
 N_TABLE_FILES = 6
 
 
+def _xp_padded(M, NW, S):
+    # streaming for rows that start on 128-byte lines; cached for the others, whose lines
+    # neighbouring workgroups share
+    return [(M, NW, S, True, False, False, False, True, nt, True) for nt in (True, False)]
+
+
 def _entries(T):
     """(M, NW, S, IL, VEC, ALDS, BIG, PAD, NT, XP) tuples of every compiled kernel."""
     out = []
@@ -94,8 +106,13 @@ def _entries(T):
         if (M, NW) in BIG_IL:
             out.append((M, NW, S, True, False, False, True, True, False, False))
         if S * WORD[T] in (64, 128) and not heavy:
-            # exact tiles reading whole row pieces, handed to lanes through LDS
+            # tiles reading whole row pieces, handed to lanes through LDS
             out.append((M, NW, S, True, False, False, False, False, True, True))
+            if S * WORD[T] == 128:
+                out += _xp_padded(M, NW, S)
+    for (M, NW, S) in IL_XP_SHAPES[T]:
+        out.append((M, NW, S, True, False, False, False, False, True, True))
+        out += _xp_padded(M, NW, S)
     for (M, NW, S) in C_SHAPES[T]:
         heavy = M >= ALDS_MIN_M[T]
         alds = heavy and (NW == 16 or (T == "float" and M == 64) or (T == "double" and M == 32))

@@ -326,8 +326,8 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(OC
         __amdgpu_buffer_rsrc_t rr[4];
         coop_rsrc(p, rr);
         T rows[4][M];
-        il_block_load<T, M, SW, S, true>(rr, brow + wrow, p.rstride, (int64_t)gi * S, lane, sl, kw,
-                                         xbuf[wave], rows);
+        il_block_load<T, M, SW, S, true, false>(rr, brow + wrow, p.rstride, (int64_t)gi * S, n,
+                                                lane, sl, kw, xbuf[wave], rows);
         // lane sweep; global row numbers drop a_0 and c_{n-1}
         T al_r[Sh::NI];
         SweepOut<T, Sh::NI> o;
@@ -389,8 +389,8 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(OC
 #pragma unroll
             for (int q = 0; q < M; ++q) xs[q] = __builtin_nan("");
         }
-        il_block_store<T, M, SW, S, true>(rr[3], brow + wrow, p.rstride, (int64_t)gi * S, p.batch,
-                                          lane, sl, kw, xbuf[wave], xs);
+        il_block_store<T, M, SW, S, true, false>(rr[3], brow + wrow, p.rstride, (int64_t)gi * S, n,
+                                                 p.batch, lane, sl, kw, xbuf[wave], xs);
         __syncthreads();                           // LDS of this task free before the next
     }
 }
@@ -442,8 +442,8 @@ __device__ __forceinline__ void coop_finish(const CoopParams<T> &p, int gi, int 
     }
     __amdgpu_buffer_rsrc_t rw[4];
     coop_rsrc(p, rw);
-    il_block_store<T, M, SW, S, true>(rw[3], brow + wrow, p.rstride, (int64_t)gi * S, p.batch,
-                                      lane, sl, kw, xb, xs);
+    il_block_store<T, M, SW, S, true, false>(rw[3], brow + wrow, p.rstride, (int64_t)gi * S, p.n,
+                                             p.batch, lane, sl, kw, xb, xs);
     __syncthreads();                           // LDS of this task free
 }
 
@@ -485,8 +485,8 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)
         const int g0 = coop_gi(p, s0);
         __amdgpu_buffer_rsrc_t rr[4];
         coop_rsrc(p, rr);
-        il_block_issue<T, M, SW, S, true>(rr, (int64_t)j0 * R + wrow, p.rstride, (int64_t)g0 * S,
-                                          lane, g);
+        il_block_issue<T, M, SW, S, true, false>(rr, (int64_t)j0 * R + wrow, p.rstride,
+                                                (int64_t)g0 * S, n, lane, g);
     }
     // the pending task: published, not yet finished
     int pend = -1, par = 0;
@@ -536,8 +536,8 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)
             const int g1 = coop_gi(p, s1);
             __amdgpu_buffer_rsrc_t rr[4];
             coop_rsrc(p, rr);
-            il_block_issue<T, M, SW, S, true>(rr, (int64_t)j1 * R + wrow, p.rstride,
-                                              (int64_t)g1 * S, lane, g);
+            il_block_issue<T, M, SW, S, true, false>(rr, (int64_t)j1 * R + wrow, p.rstride,
+                                                (int64_t)g1 * S, n, lane, g);
         }
         if (pend >= 0) {
             const int ps = pend / K;

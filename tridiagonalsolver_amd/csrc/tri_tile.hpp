@@ -67,6 +67,9 @@ template <typename T> struct TileParams {
     // Interleaved tiles: line groups resident at once, whose tiles are spread over the
     // batch (coop_group); 0: tiles in dispatch order.  Set by launch_tile.
     int32_t spread = 0;
+    // Interleaved tiles: neighbouring tiles that share lines of a row (xcd_group).  Set by
+    // launch_tile.
+    int32_t line_tiles = 1;
 };
 
 template <typename T, int M, int NW, int S, bool IL, bool VEC, bool ALDS, bool BIG, bool PAD,
@@ -323,15 +326,25 @@ template <typename T, int CH, int V> struct SafeLoader {
     }
 };
 
+// Byte offset of 16-byte chunk h of a row piece.  PAD: rows at or past n go past the
+// buffer (arrays end below 0x7fffff00), which reads them as zero and drops their stores;
+// their own offset could wrap around 32 bits.
+template <typename T, bool PAD>
+__device__ __forceinline__ int il_chunk_offset(int64_t row, int64_t rs, int64_t col0, int64_t n,
+                                               int h) {
+    const int off = (int)((row * rs + col0) * (int64_t)sizeof(T)) + h * 16;
+    return PAD && row >= n ? 0x7fffff00 : off;
+}
+
 // Interleaved whole-piece loads ("XP-IL"): rows [wrow, wrow + SW*M) of the S
 // consecutive systems starting at col0, where every row piece is S*sizeof(T)
 // contiguous bytes (CPR 16-byte chunks).  Consecutive lanes read consecutive
 // chunks (il_block_issue, NQ = M*sizeof(T)/16 chunks per lane and array); lane
 // (system sl, segment kw) then takes its M rows of system sl from the wave's LDS
 // block xb (il_block_transpose).  Offsets are 32-bit: the arrays are below 2 GiB.
-template <typename T, int M, int SW, int S, bool NT>
+template <typename T, int M, int SW, int S, bool NT, bool PAD>
 __device__ __forceinline__ void il_block_issue(const __amdgpu_buffer_rsrc_t (&rr)[4], int64_t wrow,
-                                               int64_t rs, int64_t col0, int lane,
+                                               int64_t rs, int64_t col0, int64_t n, int lane,
                                                u32x4 (&g)[4][M * (int)sizeof(T) / 16]) {
     constexpr int CPR = S * (int)sizeof(T) / 16;
     constexpr int RB = SW * M;
@@ -341,7 +354,7 @@ __device__ __forceinline__ void il_block_issue(const __amdgpu_buffer_rsrc_t (&rr
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
         const int cidx = q * 64 + lane, r = cidx / CPR, h = cidx % CPR;
-        const int off = (int)(((wrow + r) * rs + col0) * (int64_t)sizeof(T)) + h * 16;
+        const int off = il_chunk_offset<T, PAD>(wrow + r, rs, col0, n, h);
 #pragma unroll
         for (int k = 0; k < 4; ++k)
             g[k][q] = __builtin_amdgcn_raw_buffer_load_b128(rr[k], off, 0, cpol<NT>());
@@ -365,21 +378,31 @@ __device__ __forceinline__ void il_block_transpose(const u32x4 (&g)[4][M * (int)
     }
 }
 
-template <typename T, int M, int SW, int S, bool NT>
+// Rows of the lane (from row0) past the system: identity rows.
+template <typename T, int M>
+__device__ __forceinline__ void identity_rows(int64_t row0, int64_t n, T (&rows)[4][M]) {
+#pragma unroll
+    for (int j = 0; j < M; ++j)
+        if (row0 + j >= n) { rows[0][j] = 0; rows[1][j] = 1; rows[2][j] = 0; rows[3][j] = 0; }
+}
+
+template <typename T, int M, int SW, int S, bool NT, bool PAD>
 __device__ __forceinline__ void il_block_load(const __amdgpu_buffer_rsrc_t (&rr)[4], int64_t wrow,
-                                              int64_t rs, int64_t col0, int lane, int sl, int kw,
-                                              u32x4 *xb, T (&rows)[4][M]) {
+                                              int64_t rs, int64_t col0, int64_t n, int lane, int sl,
+                                              int kw, u32x4 *xb, T (&rows)[4][M]) {
     u32x4 g[4][M * (int)sizeof(T) / 16];
-    il_block_issue<T, M, SW, S, NT>(rr, wrow, rs, col0, lane, g);
+    il_block_issue<T, M, SW, S, NT, PAD>(rr, wrow, rs, col0, n, lane, g);
     il_block_transpose<T, M, S>(g, lane, sl, kw, xb, rows);
+    if (PAD) identity_rows<T, M>(wrow + kw * M, n, rows);
 }
 
 // Stores x of the same block (xs[j] = x of the lane's row j) the same way; chunks
-// of systems at or past `batch` are not written.  Every lane of the wave takes part.
-template <typename T, int M, int SW, int S, bool NT>
+// of systems at or past `batch` are not written, nor are rows at or past n (their offset
+// is past the buffer).  Every lane of the wave takes part.
+template <typename T, int M, int SW, int S, bool NT, bool PAD>
 __device__ __forceinline__ void il_block_store(__amdgpu_buffer_rsrc_t rd, int64_t wrow, int64_t rs,
-                                               int64_t col0, int64_t batch, int lane, int sl,
-                                               int kw, u32x4 *xb, const T (&xs)[M]) {
+                                               int64_t col0, int64_t n, int64_t batch, int lane,
+                                               int sl, int kw, u32x4 *xb, const T (&xs)[M]) {
     constexpr int VV = 16 / (int)sizeof(T);
     constexpr int CPR = S * (int)sizeof(T) / 16;
     constexpr int RB = SW * M;
@@ -392,7 +415,7 @@ __device__ __forceinline__ void il_block_store(__amdgpu_buffer_rsrc_t rd, int64_
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
         const int cidx = q * 64 + lane, r = cidx / CPR, h = cidx % CPR;
-        const int off = (int)(((wrow + r) * rs + col0) * (int64_t)sizeof(T)) + h * 16;
+        const int off = il_chunk_offset<T, PAD>(wrow + r, rs, col0, n, h);
         const int64_t s0 = col0 + h * VV;                  // first system of the chunk
         const u32x4 t = xb[cidx];
         if (s0 + VV <= batch) {
@@ -631,8 +654,8 @@ template <typename T, int M, int NW, int S, bool IL, bool VEC, bool ALDS, bool B
 __global__ void __launch_bounds__(64 * NW)
     __attribute__((amdgpu_waves_per_eu(tile_min_waves<T, M, NW, XP>()))) tile_wm_kernel(TileParams<T> prm) {
     using Sh = TileShape<T, M, NW, S, IL, VEC, ALDS, BIG, PAD, NT, XP>;
-    static_assert(!XP || (!BIG && (IL ? (!PAD && (S * (int)sizeof(T)) % 16 == 0) : VEC)),
-                  "transposed loads need 16-byte rows (and exact tiles when interleaved)");
+    static_assert(!XP || (!BIG && (IL ? (S * (int)sizeof(T)) % 16 == 0 : VEC)),
+                  "transposed loads move 16-byte chunks");
     constexpr int SW = Sh::SW, NWS = Sh::NWS, LS = Sh::LS, V = Sh::V, CH = Sh::CH;
     constexpr int LANES = 64 * NW;
     const int tid = threadIdx.x;
@@ -646,7 +669,7 @@ __global__ void __launch_bounds__(64 * NW)
     if (IL) {
         // tiles that share 128-byte lines on one XCD, then those line groups spread
         // over the batch so that the resident ones read whole rows, not a strip
-        constexpr int G = (S * (int)sizeof(T) >= 128) ? 1 : 128 / (S * (int)sizeof(T));
+        const int G = prm.line_tiles;
         tile = xcd_group(blockIdx.x, gridDim.x, G);
         if (prm.spread > 1) {
             const int lg = tile / G;
@@ -693,8 +716,8 @@ __global__ void __launch_bounds__(64 * NW)
             // whole row pieces and handed to the lanes through LDS
             const __amdgpu_buffer_rsrc_t rr[4] = {ra, rb, rc, rd_rsrc};
             T rows[4][M];
-            il_block_load<T, M, SW, S, NT>(rr, (int64_t)ws * SW * M, rs, (int64_t)tile * S, lane,
-                                           sl, kw, xbuf[wave], rows);
+            il_block_load<T, M, SW, S, NT, PAD>(rr, (int64_t)ws * SW * M, rs, (int64_t)tile * S, n,
+                                                lane, sl, kw, xbuf[wave], rows);
             RegLoader<T, CH, M> ld{rows};
             lane_sweep<T, Sh>(o, ld, row0, n, al_store);
         } else if constexpr (XP) {
@@ -737,11 +760,7 @@ __global__ void __launch_bounds__(64 * NW)
                         rows[k][i * (16 / (int)sizeof(T)) + v] = reinterpret_cast<const T *>(&t)[v];
                 }
             }
-            if constexpr (PAD) {
-#pragma unroll
-                for (int j = 0; j < M; ++j)   // rows past the system: identity rows
-                    if (row0 + j >= n) { rows[0][j] = 0; rows[1][j] = 1; rows[2][j] = 0; rows[3][j] = 0; }
-            }
+            if constexpr (PAD) identity_rows<T, M>(row0, n, rows);
             RegLoader<T, CH, M> ld{rows};
             lane_sweep<T, Sh>(o, ld, row0, n, al_store);
         } else if constexpr (fast) {
@@ -783,8 +802,8 @@ __global__ void __launch_bounds__(64 * NW)
 #pragma unroll
         for (int j = 0; j < M; ++j)
             xs[j] = (j == 0) ? xL : ((j == M - 1) ? xR : de[(j >= 1 && j <= M - 2) ? j - 1 : 0]);
-        il_block_store<T, M, SW, S, NT>(rd_rsrc, (int64_t)ws * SW * M, rs, (int64_t)tile * S,
-                                        prm.batch, lane, sl, kw, xbuf[wave], xs);
+        il_block_store<T, M, SW, S, NT, PAD>(rd_rsrc, (int64_t)ws * SW * M, rs, (int64_t)tile * S, n,
+                                             prm.batch, lane, sl, kw, xbuf[wave], xs);
         return;
     }
     if (!valid) return;
