@@ -321,11 +321,13 @@ template <typename T> static int64_t large_min_rows() {
     return v;
 }
 
-// A fixed device buffer that a solve uses in place of stream-ordered
-// allocations (null: allocate).
+// A device buffer that a solve uses in place of stream-ordered allocations.  only: nothing
+// may be allocated beside it (plans fit it or are refused); otherwise it is the caller's
+// offer to the cooperative solve, which allocates where it is too small.
 struct FixedScratch {
     void *ptr;
     size_t bytes;
+    bool only;
 };
 
 // Systems above the on-chip capacity: the three-pass chunked solve, in groups
@@ -631,7 +633,8 @@ static int coop_run(const SolvePlan<T> &pl, int layout, int64_t n, int64_t batch
     const CoopEntry<T> &e = *pl.coop;
     const int64_t ngroups = (batch + e.S - 1) / e.S;
     void *scratch = nullptr;
-    if (fx) {
+    const bool given = fx && fx->bytes >= pl.scratch_bytes;
+    if (given) {
         scratch = fx->ptr;
     } else {
         const hipError_t ea = hipMallocAsync(&scratch, pl.scratch_bytes, st);
@@ -657,7 +660,7 @@ static int coop_run(const SolvePlan<T> &pl, int layout, int64_t n, int64_t batch
         err = launch_coop_clear(p.flags, (int64_t)((pl.scratch_bytes - pl.forms_bytes) / sizeof(uint64_t)), st);
     if (err == hipSuccess) err = e.launch(p, pl.grid, st);
     if (err != hipSuccess) rc = hip_fail(err, "cooperative solve launch");
-    if (!fx) {
+    if (!given) {
         const hipError_t ef = hipFreeAsync(scratch, st);
         if (rc == TRIDIAG_OK && ef != hipSuccess) rc = hip_fail(ef, "cooperative solve scratch");
     }
@@ -807,8 +810,9 @@ static int solve_impl(int algo, int layout, int64_t n, int64_t batch, T *a, T *b
     const int V = 16 / (int)sizeof(T);
     const bool vec_ok = layout != kInterleaved && (sstride % V) == 0 && aligned16<T>(a) &&
                         aligned16<T>(b) && aligned16<T>(c) && aligned16<T>(d);
+    const FixedScratch *only = fx && fx->only ? fx : nullptr;
     const SolvePlan<T> pl = make_plan<T>(algo, layout, n, batch, sstride, vec_ok,
-                                         fx ? fx->bytes : 0);
+                                         only ? only->bytes : 0);
     const int32_t bb = buffer_extent<T>(n, batch, sstride, layout);
     const bool il = layout == kInterleaved;
     switch (pl.kind) {
@@ -847,7 +851,7 @@ static int solve_impl(int algo, int layout, int64_t n, int64_t batch, T *a, T *b
         return e == hipSuccess ? TRIDIAG_OK : hip_fail(e, "Thomas launch");
     }
     case kPlanBulk: {
-        if (fx && algo == kCR)
+        if (only && algo == kCR)
             return fail(TRIDIAG_EUNSUPPORTED, "the global-memory CR form keeps its levels in "
                                               "an allocated buffer");
         const hipError_t e = bulk_launch<T>(algo, a, b, c, d, n, batch, sstride, bb, st);
@@ -857,9 +861,9 @@ static int solve_impl(int algo, int layout, int64_t n, int64_t batch, T *a, T *b
         return coop_run<T>(pl, layout, n, batch, sstride, a, b, c, d, st, fx);
     case kPlanChunked:
         if (pl.coop) return coop_run<T>(pl, layout, n, batch, sstride, a, b, c, d, st, fx);
-        return large_impl<T>(algo, n, batch, sstride, a, b, c, d, st, fx);
+        return large_impl<T>(algo, n, batch, sstride, a, b, c, d, st, only);
     case kPlanViaContiguous:
-        if (fx)
+        if (only)
             return fail(TRIDIAG_EUNSUPPORTED,
                         "interleaved n_eqt=" + std::to_string(n) + " is solved through a "
                         "contiguous copy of all four arrays, which needs an allocation");
@@ -1312,6 +1316,13 @@ int tridiag_algo_layout(int precision, int algo) {
 
 int tridiag_solve(int precision, int algo, int layout, int64_t n_eqt, int64_t n_batch, void *a,
                   void *b, void *c, void *d, void *stream) {
+    return tridiag_solve_scratch(precision, algo, layout, n_eqt, n_batch, a, b, c, d, nullptr, 0,
+                                 stream);
+}
+
+int tridiag_solve_scratch(int precision, int algo, int layout, int64_t n_eqt, int64_t n_batch,
+                          void *a, void *b, void *c, void *d, void *scratch, int64_t scratch_bytes,
+                          void *stream) {
     g_last_error.clear();
     if (precision != TRIDIAG_SINGLE && precision != TRIDIAG_DOUBLE)
         return fail(TRIDIAG_EINVAL, "precision must be 0 (single) or 1 (double)");
@@ -1337,11 +1348,12 @@ int tridiag_solve(int precision, int algo, int layout, int64_t n_eqt, int64_t n_
                                           (int)n_eqt, (int)n_batch);
     }
     hipStream_t st = (hipStream_t)stream;
+    const FixedScratch given{scratch, (size_t)(scratch && scratch_bytes > 0 ? scratch_bytes : 0), false};
     if (precision == TRIDIAG_SINGLE)
         return solve_impl<float>(algo, layout, n_eqt, n_batch, (float *)a, (float *)b,
-                                 (float *)c, (float *)d, st);
+                                 (float *)c, (float *)d, st, &given);
     return solve_impl<double>(algo, layout, n_eqt, n_batch, (double *)a, (double *)b,
-                              (double *)c, (double *)d, st);
+                              (double *)c, (double *)d, st, &given);
 }
 
 int tridiag_solve_bulk(int precision, int algo, int layout, int64_t n_eqt, int64_t n_batch,
@@ -1371,7 +1383,7 @@ int tridiag_solve_noalloc(int precision, int algo, int layout, int64_t n_eqt, in
                                           "own buffer; tridiag_solve_noalloc does not run it");
     void *ptr = nullptr;
     if (const int rc = noalloc_scratch(&ptr)) return rc;
-    const FixedScratch fx{ptr, kNoAllocScratchBytes};
+    const FixedScratch fx{ptr, kNoAllocScratchBytes, true};
     hipStream_t st = (hipStream_t)stream;
     if (precision == TRIDIAG_SINGLE)
         return solve_impl<float>(algo, layout, n_eqt, n_batch, (float *)a, (float *)b,
@@ -1441,6 +1453,17 @@ int tridiag_plan_kind(int precision, int algo, int layout, int64_t n_eqt, int64_
     }
     fail(TRIDIAG_EINVAL, "precision must be 0 or 1");
     return -1;
+}
+
+int64_t tridiag_scratch_bytes(int precision, int algo, int layout, int64_t n_eqt, int64_t n_batch) {
+    g_last_error.clear();
+    SolvePlan<float> f;
+    SolvePlan<double> d;
+    if (precision == TRIDIAG_SINGLE)
+        return plan_impl<float>(algo, layout, n_eqt, n_batch, f) ? 0 : (int64_t)f.scratch_bytes;
+    if (precision == TRIDIAG_DOUBLE)
+        return plan_impl<double>(algo, layout, n_eqt, n_batch, d) ? 0 : (int64_t)d.scratch_bytes;
+    return 0;
 }
 
 int tridiag_tile_count(int precision) {

@@ -1,6 +1,7 @@
 """Torch-facing entry points over the C-ABI (device memory and streams come from torch;
 all arithmetic happens in the HIP kernels of libtridiag_amd.so)."""
 import ctypes
+import functools
 
 import torch
 
@@ -16,19 +17,22 @@ def _precision(t):
 
 
 def _stream_handle(device):
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    # the handle alone: building a Stream object takes 2 us of a small solve's 8
+    index = device.index if device.index is not None else torch.cuda.current_device()
+    return torch._C._cuda_getCurrentRawStream(index)
 
 
 def _ptr(t):
-    return ctypes.c_void_p(t.data_ptr())
+    return t.data_ptr()
 
 
 def _check_tensors(ts):
     t0 = ts[0]
     if not t0.is_cuda:
         raise ValueError("tensors must be on a GPU device")
+    dtype, index = t0.dtype, t0.get_device()
     for t in ts:
-        if t.dtype != t0.dtype or t.device != t0.device:
+        if t.dtype != dtype or t.get_device() != index or not t.is_cuda:
             raise ValueError("all tensors must share dtype and device")
         if not t.is_contiguous():
             raise ValueError("tensors must be contiguous")
@@ -46,6 +50,18 @@ def _shape(t, layout, n, batch):
     return t.shape[1], t.shape[0]
 
 
+@functools.lru_cache(maxsize=4096)
+def _scratch_bytes(prec, algo, layout, n, batch, device_index, current_device):
+    # (the plan depends on the GPU that is current when the solve is launched)
+    return lib().tridiag_scratch_bytes(prec, algo, layout, n, batch)
+
+
+def _scratch(prec, algo, layout, n, batch, device):
+    """Scratch of a solve on the current stream, from torch's caching allocator, or None."""
+    size = _scratch_bytes(prec, algo, layout, n, batch, device.index, torch.cuda.current_device())
+    return torch.empty(size, dtype=torch.uint8, device=device) if size else None
+
+
 def solve(a, b, c, d, algo=ALGO_AUTO, layout=CONTIGUOUS, n=None, batch=None):
     """Solves in place: x is written to d; c may be clobbered (naive Thomas writes c').
 
@@ -56,8 +72,15 @@ def solve(a, b, c, d, algo=ALGO_AUTO, layout=CONTIGUOUS, n=None, batch=None):
     _check_tensors(ts)
     n, batch = _shape(a if layout == PACKED else d, layout, n, batch)
     prec = _precision(a)
-    args = [_ptr(a)] + ([_ptr(a)] * 3 if layout == PACKED else [_ptr(b), _ptr(c), _ptr(d)])
-    check(lib().tridiag_solve(prec, algo, layout, n, batch, *args, _stream_handle(a.device)))
+    pa = _ptr(a)
+    args = (pa, pa, pa, pa) if layout == PACKED else (pa, _ptr(b), _ptr(c), _ptr(d))
+    device = a.device
+    w = _scratch(prec, algo, layout, n, batch, device) if n > 512 and batch > 0 else None
+    if w is None:
+        check(lib().tridiag_solve(prec, algo, layout, n, batch, *args, _stream_handle(device)))
+    else:
+        check(lib().tridiag_solve_scratch(prec, algo, layout, n, batch, *args, _ptr(w), w.numel(),
+                                          _stream_handle(device)))
     return a if layout == PACKED else d
 
 
