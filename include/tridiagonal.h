@@ -307,10 +307,18 @@ int tridiag_div_mode(void);
  *                      memory, 5 interleaved systems solved through a contiguous
  *                      copy, 6 a bulk-row form, 7 several short contiguous
  *                      systems per wave, on chip; -1 on a bad argument.
+ *   tridiag_plan_blocks  K, the row blocks per system, where the batch is solved
+ *                      cooperatively, with M, NW and S as above; 0 elsewhere, -1 on a
+ *                      bad argument.  Batches of kinds 2, 4 and 5 can be: long
+ *                      contiguous systems, and interleaved systems of more than 512
+ *                      rows whose rows or blocks are not whole.  The kind is then what
+ *                      runs where the cooperative solve is switched off.
  *   tridiag_plan       for kinds 2 and 3, rows-per-lane M, waves per workgroup
  *                      NW, systems per workgroup S; TRIDIAG_EUNSUPPORTED for the
  *                      other kinds. */
 int tridiag_plan_kind(int precision, int algo, int layout, int64_t n_eqt, int64_t n_batch);
+int tridiag_plan_blocks(int precision, int algo, int layout, int64_t n_eqt, int64_t n_batch, int *M,
+                        int *NW, int *S);
 int tridiag_plan(int precision, int algo, int layout, int64_t n_eqt, int64_t n_batch, int *M,
                  int *NW, int *S);
 

@@ -98,6 +98,8 @@ def lib():
     L.tridiag_plan.restype = ci
     L.tridiag_plan_kind.argtypes = [ci, ci, ci, i64, i64]
     L.tridiag_plan_kind.restype = ci
+    L.tridiag_plan_blocks.argtypes = L.tridiag_plan.argtypes
+    L.tridiag_plan_blocks.restype = ci
     L.tridiag_tile_count.argtypes = [ci]
     L.tridiag_tile_count.restype = ci
     pi = ctypes.POINTER(ci)
@@ -142,21 +144,24 @@ PLAN_KINDS = ["lane", "thomas", "tile", "cooperative", "chunked", "via_contiguou
 
 def plan(precision, algo, layout, n, batch):
     """How tridiag_solve solves the batch: kind (PLAN_KINDS) and, for on-chip
-    workgroup plans, rows per lane M, waves per workgroup NW, systems per workgroup S
-    (cooperative plans: also the rows per block and blocks per system K)."""
+    workgroup plans, rows per lane M, waves per workgroup NW, systems per workgroup S.
+    Batches solved cooperatively also have `K` blocks of `block_rows` rows per system;
+    those of another kind than "cooperative" are what `kind` says without them."""
     L = lib()
     k = L.tridiag_plan_kind(precision, algo, layout, n, batch)
     if k < 0:
         raise TridiagError(EINVAL, L.tridiag_last_error().decode())
     out = dict(kind=PLAN_KINDS[k])
+    M, NW, S = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
     if PLAN_KINDS[k] in ("tile", "cooperative"):
-        M, NW, S = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
         check(L.tridiag_plan(precision, algo, layout, n, batch, ctypes.byref(M),
                              ctypes.byref(NW), ctypes.byref(S)))
         out.update(M=M.value, NW=NW.value, S=S.value)
-        if PLAN_KINDS[k] == "cooperative":
-            rows = (64 // S.value if layout == INTERLEAVED else 64) * NW.value * M.value
-            out.update(block_rows=rows, K=-(-n // rows))
+    K = L.tridiag_plan_blocks(precision, algo, layout, n, batch, ctypes.byref(M),
+                              ctypes.byref(NW), ctypes.byref(S))
+    if K > 0:
+        rows = (64 // S.value if layout == INTERLEAVED else 64) * NW.value * M.value
+        out.update(block_rows=rows, K=K)
     return out
 
 

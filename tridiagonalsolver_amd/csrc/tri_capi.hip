@@ -395,35 +395,34 @@ static int64_t env_int(const char *name, int64_t dflt) {
 }
 
 // Interleaved systems of at least this many rows take the cooperative solve
-// ($TRIDIAG_COOP_MIN_ROWS overrides for both precisions; a negative value turns
-// the cooperative solve off for both layouts).  Measured on MI355X (groups of a
-// round spread over the batch) against the one-workgroup tiles, at about 2^24
-// unknowns: FP32 768 rows 0.082 vs 0.093 ms, 1024 rows 0.082 vs 0.090 ms, 1280
-// rows 0.082 vs 0.143 ms, 1536 rows 0.083 vs 0.117 ms; FP64 1024 rows 0.181 vs
-// 0.218 ms, 1536 rows 0.166 vs 0.251 ms; at 512 rows the tile wins (FP32 0.084 vs
-// 0.078 ms).  At 4M unknowns FP32 1024 rows is a draw (0.028 vs 0.025 ms), FP64
-// 0.045 vs 0.054 ms.  Above 4096 rows (no interleaved tile) it replaces the solve
-// through a contiguous copy: 8192 rows 0.123 vs 0.201 ms (FP32), 0.257 vs 0.406 ms
-// (FP64); 16384 rows (64 blocks) 0.167 vs 0.213 ms (FP32), and FP64 12288 rows
-// 0.266 vs 0.363 ms.
-static int64_t coop_min_rows_il(int prec) {
+// ($TRIDIAG_COOP_MIN_ROWS overrides; a negative value turns the cooperative solve off for
+// both layouts).  Whole-piece tiles end at 512 rows; above, the one-workgroup tiles read
+// pieces of 16-64 bytes and beyond 4096 rows only the contiguous copy is left.  Measured
+// on MI355X, tile or copy / cooperative (us): FP32 600 x 16,000 65 / 55, 700 x 100 12.8 /
+// 10.2, 1100 x 500 15.5 / 11.0, 3001 x 20 29.3 / 10.4, 4096 x 4001 116 / 106, 5000 x 64
+// 30.7 / 12.8, 16,384 x 1024 213 / 167; FP64 600 x 8000 67.6 / 57.7, 700 x 2000 18.8 / 17.1,
+// 3001 x 1001 67 / 45, 3001 x 1008 64 / 35, 12,000 x 20 48.0 / 19.9.  Below: FP32 400 x 4000
+// 12.6 / 19.7, FP64 17.5 / 22.1.
+static int64_t coop_min_rows_il() {
     static const int64_t env = env_int("TRIDIAG_COOP_MIN_ROWS", 0);
-    if (env != 0) return env;
-    return 1024;
+    return env != 0 ? env : 513;
 }
+// Interleaved batches below this many rows, or with partial row blocks, or off lines where
+// a tile holds n, report the tile or the copy that they took before the cooperative solve
+// took every size (tridiag_plan_blocks says what runs).
+constexpr int64_t kCoopReportedRows = 1024;
 
-// Interleaved rows whose pitch is not a multiple of 128 bytes: the groups' row
-// pieces straddle cache lines, which costs the cooperative solve more than the
-// tiles (FP32 4096 x 4001 0.168 vs 0.117 ms, 2048 x 8191 0.157 vs 0.121 ms; FP64
-// 0.349 vs 0.230, 0.316 vs 0.227 ms), so such batches keep the tile wherever one
-// holds n.
+// Whether interleaved rows start on 128-byte lines.  Off them the row pieces of neighbouring
+// groups share lines: the loads stay cached and the neighbours run on one XCD
+// (coop_task_shared).  Streamed and in the spread order FP64 3001 x 1001 took 57.6 us
+// (44.5 this way), FP32 4096 x 4001 173 us (106).
 template <typename T> static bool il_rows_on_lines(int64_t batch) {
     return (batch * (int64_t)sizeof(T)) % 128 == 0;
 }
 // Polls of a cooperative wait before it gives up ($TRIDIAG_COOP_SPIN).
 static int32_t coop_spin_limit() {
     static const int32_t v = (int32_t)std::max<int64_t>(0, std::min<int64_t>(
-        env_int("TRIDIAG_COOP_SPIN", (int64_t)1 << 22), 0x7fffffff));
+        env_int("TRIDIAG_COOP_SPIN", (int64_t)1 << 25), 0x7fffffff));
     return v;
 }
 
@@ -484,7 +483,7 @@ static const CoopEntry<T> *choose_coop(bool il, int64_t n, int64_t batch, int &K
         if (forced >= 0 && i != forced) continue;
         const CoopEntry<T> &e = tab.entries[i];
         if (e.IL != il) continue;
-        const int64_t k = il ? (n % e.R == 0 ? n / e.R : 0) : (n + e.R - 1) / e.R;
+        const int64_t k = (n + e.R - 1) / e.R;
         if (k < 2 || k > e.kmax) continue;
         const int64_t cap = e.max_grid(il && coop_pipelined(e.pipe) != 0);
         const int64_t tasks = (batch + e.S - 1) / e.S * k;
@@ -574,13 +573,13 @@ enum PlanKind {
     kPlanThomas = 1,         // the Thomas recurrence (algorithm 1)
     kPlanTile = 2,           // on chip, one workgroup per system or per S systems
     kPlanCoop = 3,           // on chip, K workgroups per group of systems
-    kPlanChunked = 4,        // over chunks: cooperatively where a system's chunks fit on chip
-                             // at once, else three passes through global memory
+    kPlanChunked = 4,        // over chunks, in three passes through global memory
     kPlanViaContiguous = 5,  // interleaved systems solved through a contiguous copy
     kPlanBulk = 6,           // the reference's own form of ids 2-13 (bulk rows, CR levels)
     kPlanShort = 7,          // several short contiguous systems per wave
 };
 template <typename T> struct SolvePlan {
+    // how the batch is reported; with `coop` it is solved cooperatively whichever this says
     int kind = kPlanTile;
     const TileEntry<T> *tile = nullptr;
     const CoopEntry<T> *coop = nullptr;
@@ -595,12 +594,11 @@ template <typename T> struct SolvePlan {
 // 32-bit offsets, and a device that holds at least K of its workgroups at once.
 // fixed_bytes > 0: the scratch must fit a fixed buffer of that size.
 template <typename T>
-static bool coop_plan(int algo, int layout, int64_t n, int64_t batch, size_t fixed_bytes,
-                      SolvePlan<T> &pl) {
-    const int prec = sizeof(T) == 4 ? TRIDIAG_SINGLE : TRIDIAG_DOUBLE;
-    if (coop_min_rows_il(prec) < 0 || algo_spec(algo).iface != kIfaceWM) return false;
+static bool coop_plan(int algo, int layout, int64_t n, int64_t batch, const TileEntry<T> *tile,
+                      size_t fixed_bytes, SolvePlan<T> &pl) {
+    if (coop_min_rows_il() < 0 || algo_spec(algo).iface != kIfaceWM) return false;
     const bool il = layout == kInterleaved;
-    if (il && n < coop_min_rows_il(prec)) return false;
+    if (il && n < coop_min_rows_il()) return false;
     // interleaved: 32-bit offsets into whole arrays; contiguous: into one system
     const int64_t elems = il ? n * batch : n;
     if (elems * (int64_t)sizeof(T) >= (int64_t)0x7fffff00) return false;
@@ -612,12 +610,18 @@ static bool coop_plan(int algo, int layout, int64_t n, int64_t batch, size_t fix
     const int64_t ngroups = (batch + e->S - 1) / e->S;
     const int64_t ntask = ngroups * K;
     if (ntask > 0x7fffffff) return false;
+    // what a batch reports (SolvePlan::kind), and what the solve without allocations takes
+    // of the interleaved systems that no tile holds
+    const bool reported = !il || (n >= kCoopReportedRows && n % e->R == 0 &&
+                                  (!tile || il_rows_on_lines<T>(batch)));
+    if (fixed_bytes && !reported && !tile) return false;
     const size_t forms = (((size_t)ntask * e->S * 6 * sizeof(T)) + 255) & ~(size_t)255;
     const size_t words = !il ? 2 * (size_t)ntask : (size_t)ngroups * kCoopFlagStride;
     const size_t bytes = forms + words * sizeof(uint64_t);
     if (fixed_bytes && bytes > fixed_bytes) return false;
-    // (systems of more than 32 blocks report the chunked kind)
-    pl.kind = il || K <= 32 ? kPlanCoop : kPlanChunked;
+    pl.kind = !reported ? (tile ? kPlanTile : kPlanViaContiguous)
+                        : il || K <= 32 ? kPlanCoop : kPlanChunked;
+    pl.tile = reported ? nullptr : tile;
     pl.coop = e;
     pl.K = K;
     pl.grid = (int)P;
@@ -646,6 +650,7 @@ static int coop_run(const SolvePlan<T> &pl, int layout, int64_t n, int64_t batch
                     il ? coop_spin_limit() : std::min(coop_spin_limit(), kCoopTreePolls),
                     il ? coop_pipelined(e.pipe) : 0,
                     il ? coop_spread(pl.grid / pl.K) : 0,
+                    il && !il_rows_on_lines<T>(batch) ? 1 : 0,
                     reinterpret_cast<T *>(scratch),
                     reinterpret_cast<uint64_t *>(reinterpret_cast<char *>(scratch) +
                                                  pl.forms_bytes),
@@ -755,11 +760,11 @@ static SolvePlan<T> make_plan(int algo, int layout, int64_t n, int64_t batch, in
     }
     // rows beyond one workgroup: K workgroups per group of systems, on chip
     const bool on_lines = !il || il_rows_on_lines<T>(batch);
-    const bool il_tile_first = !on_lines &&
-                               choose_tile<T>(algo, layout, n, vec_ok, on_lines, bb == 0) != nullptr;
-    if ((il || n > large_min_rows<T>()) && !il_tile_first &&
-        coop_plan<T>(algo, layout, n, batch, fixed_bytes, pl))
-        return pl;
+    if (il || n > large_min_rows<T>()) {
+        const TileEntry<T> *tile =
+            il ? choose_tile<T>(algo, layout, n, vec_ok, on_lines, bb == 0) : nullptr;
+        if (coop_plan<T>(algo, layout, n, batch, tile, fixed_bytes, pl)) return pl;
+    }
     if (!il && n > large_min_rows<T>() && n > large_chunk_rows(prec, 0)) {
         pl.kind = kPlanChunked;
         return pl;
@@ -815,6 +820,7 @@ static int solve_impl(int algo, int layout, int64_t n, int64_t batch, T *a, T *b
                                          only ? only->bytes : 0);
     const int32_t bb = buffer_extent<T>(n, batch, sstride, layout);
     const bool il = layout == kInterleaved;
+    if (pl.coop) return coop_run<T>(pl, layout, n, batch, sstride, a, b, c, d, st, fx);
     switch (pl.kind) {
     case kPlanLane: {
         const hipError_t e = (sizeof(T) == 4)
@@ -857,10 +863,7 @@ static int solve_impl(int algo, int layout, int64_t n, int64_t batch, T *a, T *b
         const hipError_t e = bulk_launch<T>(algo, a, b, c, d, n, batch, sstride, bb, st);
         return e == hipSuccess ? TRIDIAG_OK : hip_fail(e, "bulk-row launch");
     }
-    case kPlanCoop:
-        return coop_run<T>(pl, layout, n, batch, sstride, a, b, c, d, st, fx);
     case kPlanChunked:
-        if (pl.coop) return coop_run<T>(pl, layout, n, batch, sstride, a, b, c, d, st, fx);
         return large_impl<T>(algo, n, batch, sstride, a, b, c, d, st, only);
     case kPlanViaContiguous:
         if (only)
@@ -1422,13 +1425,13 @@ int tridiag_plan(int precision, int algo, int layout, int64_t n_eqt, int64_t n_b
         if (const int rc = plan_impl<float>(algo, layout, n_eqt, n_batch, pl)) return rc;
         kind = pl.kind;
         if (pl.tile) { m = pl.tile->M; nw = pl.tile->NW; s = pl.tile->S; }
-        if (pl.coop) { m = pl.coop->M; nw = pl.coop->NW; s = pl.coop->S; }
+        else if (pl.coop) { m = pl.coop->M; nw = pl.coop->NW; s = pl.coop->S; }
     } else if (precision == TRIDIAG_DOUBLE) {
         SolvePlan<double> pl;
         if (const int rc = plan_impl<double>(algo, layout, n_eqt, n_batch, pl)) return rc;
         kind = pl.kind;
         if (pl.tile) { m = pl.tile->M; nw = pl.tile->NW; s = pl.tile->S; }
-        if (pl.coop) { m = pl.coop->M; nw = pl.coop->NW; s = pl.coop->S; }
+        else if (pl.coop) { m = pl.coop->M; nw = pl.coop->NW; s = pl.coop->S; }
     } else {
         return fail(TRIDIAG_EINVAL, "precision must be 0 or 1");
     }
@@ -1453,6 +1456,28 @@ int tridiag_plan_kind(int precision, int algo, int layout, int64_t n_eqt, int64_
     }
     fail(TRIDIAG_EINVAL, "precision must be 0 or 1");
     return -1;
+}
+
+int tridiag_plan_blocks(int precision, int algo, int layout, int64_t n_eqt, int64_t n_batch, int *M,
+                        int *NW, int *S) {
+    g_last_error.clear();
+    SolvePlan<float> f;
+    SolvePlan<double> d;
+    int m = 0, nw = 0, s = 0, K = 0;
+    if (precision == TRIDIAG_SINGLE) {
+        if (plan_impl<float>(algo, layout, n_eqt, n_batch, f)) return -1;
+        if (f.coop) { K = f.K; m = f.coop->M; nw = f.coop->NW; s = f.coop->S; }
+    } else if (precision == TRIDIAG_DOUBLE) {
+        if (plan_impl<double>(algo, layout, n_eqt, n_batch, d)) return -1;
+        if (d.coop) { K = d.K; m = d.coop->M; nw = d.coop->NW; s = d.coop->S; }
+    } else {
+        fail(TRIDIAG_EINVAL, "precision must be 0 or 1");
+        return -1;
+    }
+    if (M) *M = m;
+    if (NW) *NW = nw;
+    if (S) *S = s;
+    return K;
 }
 
 int64_t tridiag_scratch_bytes(int precision, int algo, int layout, int64_t n_eqt, int64_t n_batch) {

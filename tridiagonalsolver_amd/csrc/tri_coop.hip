@@ -31,18 +31,25 @@ static hipError_t launch_coop(const CoopParams<T> &p, int grid, hipStream_t st) 
     if (p.pipelined)
         hipLaunchKernelGGL((coop_pipe_kernel<T, M, NW, S, KMAX>), dim3((unsigned)grid),
                            dim3(64 * NW), 0, st, p);
+    else if (p.shared_lines)
+        hipLaunchKernelGGL((coop_kernel<T, M, NW, S, KMAX, OCC, false>), dim3((unsigned)grid),
+                           dim3(64 * NW), 0, st, p);
     else
-        hipLaunchKernelGGL((coop_kernel<T, M, NW, S, KMAX, OCC>), dim3((unsigned)grid),
+        hipLaunchKernelGGL((coop_kernel<T, M, NW, S, KMAX, OCC, true>), dim3((unsigned)grid),
                            dim3(64 * NW), 0, st, p);
     return hipGetLastError();
 }
 template <typename T, int M, int NW, int S, int KMAX, int OCC>
 static int coop_max_grid(bool pipelined) {
-    static int cache[2][64];
-    const void *fn = pipelined
-        ? reinterpret_cast<const void *>(coop_pipe_kernel<T, M, NW, S, KMAX>)
-        : reinterpret_cast<const void *>(coop_kernel<T, M, NW, S, KMAX, OCC>);
-    return resident_workgroups(fn, 64 * NW, cache[pipelined ? 1 : 0]);
+    static int cache[3][64];
+    if (pipelined)
+        return resident_workgroups(reinterpret_cast<const void *>(coop_pipe_kernel<T, M, NW, S, KMAX>),
+                                   64 * NW, cache[2]);
+    return std::min(
+        resident_workgroups(reinterpret_cast<const void *>(coop_kernel<T, M, NW, S, KMAX, OCC, false>),
+                            64 * NW, cache[0]),
+        resident_workgroups(reinterpret_cast<const void *>(coop_kernel<T, M, NW, S, KMAX, OCC, true>),
+                            64 * NW, cache[1]));
 }
 
 // Contiguous systems: the solve, and the pass over blocks whose wait gave up.

@@ -67,6 +67,7 @@ template <typename T> struct CoopParams {
     int32_t spin_limit;  // polls of a wait before it gives up
     int32_t pipelined;   // 1: coop_pipe_kernel (wait one task later), 0: coop_kernel
     int32_t spread;      // groups per round whose slots are spread over the batch (<= 1: none)
+    int32_t shared_lines;  // interleaved rows start off 128-byte lines (coop_task_shared)
     T *forms;            // [ngroups][K][S][6] block outer forms
     uint64_t *flags;     // [kCoopFlagStride * g + j]: the tag once block j of group g is published
     uint64_t tag;        // this solve's tag: different from every earlier solve's
@@ -85,9 +86,16 @@ constexpr int kCoopFlagStride = 64;
 #define TRI_COOP_POLL_SLEEP 8
 #endif
 
-// Group solved by slot s: a round's groups are spread over the batch (coop_group).
-template <typename T> __device__ __forceinline__ int coop_gi(const CoopParams<T> &p, int s) {
-    return coop_group(s, p.ngroups, p.spread);
+// Group and row block of an interleaved task.
+template <typename T>
+__device__ __forceinline__ void coop_task(const CoopParams<T> &p, int task, int &gi, int &j) {
+    if (p.shared_lines) {
+        coop_task_shared(task, (int)gridDim.x, p.K, p.ngroups, gi, j);
+    } else {
+        const int s = task / p.K;
+        j = task - s * p.K;
+        gi = coop_group(s, p.ngroups, p.spread);
+    }
 }
 
 template <typename T, int M, int NW, int S> struct CoopShape {
@@ -289,8 +297,10 @@ __device__ __forceinline__ void coop_rsrc(const CoopParams<T> &p, __amdgpu_buffe
     rr[2] = make_rsrc(p.c, p.buf_bytes); rr[3] = make_rsrc(p.d, p.buf_bytes);
 }
 
-// OCC: waves per SIMD the kernel is built for (its register budget).
-template <typename T, int M, int NW, int S, int KMAX, int OCC>
+// OCC: waves per SIMD the kernel is built for (its register budget).  LINES: rows start on
+// 128-byte lines, which are read once and streamed; otherwise neighbouring groups share
+// lines and the loads stay cached.
+template <typename T, int M, int NW, int S, int KMAX, int OCC, bool LINES>
 __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(OCC)))
     coop_kernel(CoopParams<T> p) {
     using Sh = TileShape<T, M, NW, S, true, false, false, false, false, true, true>;
@@ -319,15 +329,15 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(OC
         const int kw = lane / S;             // segment inside the wave-block
         const int ws = wave;                 // wave-block inside the block
         const int64_t wrow = (int64_t)ws * SW * M;   // first row of the wave-block, in the block
-        const int si = task / K, j = task - si * K;
-        const int gi = coop_gi(p, si);
+        int gi, j;
+        coop_task(p, task, gi, j);
         const int64_t brow = (int64_t)j * R;               // first row of the block
         const int64_t row0 = brow + wrow + (int64_t)kw * M;   // first row of the lane
         __amdgpu_buffer_rsrc_t rr[4];
         coop_rsrc(p, rr);
         T rows[4][M];
-        il_block_load<T, M, SW, S, true, false>(rr, brow + wrow, p.rstride, (int64_t)gi * S, n,
-                                                lane, sl, kw, xbuf[wave], rows);
+        il_block_load<T, M, SW, S, LINES, true>(rr, brow + wrow, p.rstride, (int64_t)gi * S, n, lane,
+                                               sl, kw, xbuf[wave], rows);
         // lane sweep; global row numbers drop a_0 and c_{n-1}
         T al_r[Sh::NI];
         SweepOut<T, Sh::NI> o;
@@ -389,8 +399,8 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(OC
 #pragma unroll
             for (int q = 0; q < M; ++q) xs[q] = __builtin_nan("");
         }
-        il_block_store<T, M, SW, S, true, false>(rr[3], brow + wrow, p.rstride, (int64_t)gi * S, n,
-                                                 p.batch, lane, sl, kw, xbuf[wave], xs);
+        il_block_store<T, M, SW, S, true, true>(rr[3], brow + wrow, p.rstride, (int64_t)gi * S, n,
+                                                p.batch, lane, sl, kw, xbuf[wave], xs);
         __syncthreads();                           // LDS of this task free before the next
     }
 }
@@ -442,7 +452,7 @@ __device__ __forceinline__ void coop_finish(const CoopParams<T> &p, int gi, int 
     }
     __amdgpu_buffer_rsrc_t rw[4];
     coop_rsrc(p, rw);
-    il_block_store<T, M, SW, S, true, false>(rw[3], brow + wrow, p.rstride, (int64_t)gi * S, p.n,
+    il_block_store<T, M, SW, S, true, true>(rw[3], brow + wrow, p.rstride, (int64_t)gi * S, p.n,
                                              p.batch, lane, sl, kw, xb, xs);
     __syncthreads();                           // LDS of this task free
 }
@@ -481,11 +491,11 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)
     int task = (int)blockIdx.x;
     u32x4 g[4][NQ];
     if (task < ntask) {
-        const int s0 = task / K, j0 = task - s0 * K;
-        const int g0 = coop_gi(p, s0);
+        int g0, j0;
+        coop_task(p, task, g0, j0);
         __amdgpu_buffer_rsrc_t rr[4];
         coop_rsrc(p, rr);
-        il_block_issue<T, M, SW, S, true, false>(rr, (int64_t)j0 * R + wrow, p.rstride,
+        il_block_issue<T, M, SW, S, true, true>(rr, (int64_t)j0 * R + wrow, p.rstride,
                                                 (int64_t)g0 * S, n, lane, g);
     }
     // the pending task: published, not yet finished
@@ -493,12 +503,13 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)
     Outer<T> poL{}, poR{};
     T pde[NI], pga[NI], pal[NI];
     for (; task < ntask; task += P) {
-        const int si = task / K, j = task - si * K;
-        const int gi = coop_gi(p, si);
+        int gi, j;
+        coop_task(p, task, gi, j);
         const int64_t brow = (int64_t)j * R;
         const int64_t row0 = brow + wrow + (int64_t)kw * M;
         T rows[4][M];
         il_block_transpose<T, M, S>(g, lane, sl, kw, xbuf[wave], rows);
+        identity_rows<T, M>(row0, n, rows);
         T al_r[NI];
         SweepOut<T, NI> o;
         RegLoader<T, Sh::CH, M> ld{rows};
@@ -532,18 +543,17 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)
                                __HIP_MEMORY_SCOPE_AGENT);
         const int next = task + P;
         if (next < ntask) {
-            const int s1 = next / K, j1 = next - s1 * K;
-            const int g1 = coop_gi(p, s1);
+            int g1, j1;
+            coop_task(p, next, g1, j1);
             __amdgpu_buffer_rsrc_t rr[4];
             coop_rsrc(p, rr);
-            il_block_issue<T, M, SW, S, true, false>(rr, (int64_t)j1 * R + wrow, p.rstride,
-                                                (int64_t)g1 * S, n, lane, g);
+            il_block_issue<T, M, SW, S, true, true>(rr, (int64_t)j1 * R + wrow, p.rstride,
+                                                    (int64_t)g1 * S, n, lane, g);
         }
         if (pend >= 0) {
-            const int ps = pend / K;
-            coop_finish<T, M, NW, S, KMAX, NI>(p, coop_gi(p, ps),
-                                                   pend - ps * K, sh_blk[par ^ 1], sh_uv,
-                                                   sh_k, &s_ok, xbuf[wave], tid, lane, sl, kw, ws,
+            int pg, pj;
+            coop_task(p, pend, pg, pj);
+            coop_finish<T, M, NW, S, KMAX, NI>(p, pg, pj, sh_blk[par ^ 1], sh_uv, sh_k, &s_ok, xbuf[wave], tid, lane, sl, kw, ws,
                                                    wrow, poL, poR, pde, pga, pal);
         }
         pend = task;
@@ -558,9 +568,9 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)
         }
     }
     if (pend >= 0) {
-        const int ps = pend / K;
-        coop_finish<T, M, NW, S, KMAX, NI>(p, coop_gi(p, ps), pend - ps * K,
-                                               sh_blk[par ^ 1], sh_uv, sh_k,
+        int pg, pj;
+        coop_task(p, pend, pg, pj);
+        coop_finish<T, M, NW, S, KMAX, NI>(p, pg, pj, sh_blk[par ^ 1], sh_uv, sh_k,
                                                &s_ok, xbuf[wave], tid, lane, sl, kw, ws, wrow, poL,
                                                poR, pde, pga, pal);
     }

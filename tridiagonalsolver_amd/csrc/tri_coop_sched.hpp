@@ -28,4 +28,23 @@ inline TRI_COOP_HD int coop_group(int s, int G, int W) {
     return c < L ? c * R + r : L * R + (c - L) * (R - 1) + r;
 }
 
+// Group gi and row block j of task `task` of a grid of P workgroups (P a multiple of K)
+// when the row pieces of neighbouring groups share lines.  A round's groups are neighbours
+// and come in clusters of C whose tasks are consecutive; a cluster's tasks are numbered row
+// block by row block, and each XCD (workgroups are dispatched to the eight in turn) takes
+// consecutive numbers, so that its L2 serves the second reader of a line.  C * K stays
+// at most 128: workgroups are dispatched in order, so wherever 128 of the grid are resident
+// a whole cluster is, and its waits end.
+inline TRI_COOP_HD void coop_task_shared(int task, int P, int K, int G, int &gi, int &j) {
+    const int C = K <= 16 ? 8 : K <= 32 ? 4 : 2;
+    const int round = task / P, b = task - round * P;
+    const int first = round * (P / K), W = G - first < P / K ? G - first : P / K;
+    const int cl = b / (C * K), c = b - cl * (C * K);
+    const int w = W - cl * C < C ? W - cl * C : C;          // groups of this cluster
+    const int active = w * K, q = active / 8, r = active % 8, x = c % 8;
+    const int pos = x * q + (x < r ? x : r) + c / 8;
+    j = pos / w;
+    gi = first + cl * C + pos - j * w;
+}
+
 }  // namespace tri
