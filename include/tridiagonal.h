@@ -144,6 +144,11 @@ int64_t tridiag_scratch_bytes(int precision, int algo, int layout, int64_t n_eqt
 int tridiag_solve_scratch(int precision, int algo, int layout, int64_t n_eqt, int64_t n_batch,
                           void *a, void *b, void *c, void *d, void *scratch, int64_t scratch_bytes,
                           void *stream);
+/* The same with x in an array of its own, apart from all inputs (or d itself); d is then
+ * only read.  c may be overwritten as by tridiag_solve.  Layouts 0 and 2. */
+int tridiag_solve_to(int precision, int algo, int layout, int64_t n_eqt, int64_t n_batch, void *a,
+                     void *b, void *c, void *d, void *x, void *scratch, int64_t scratch_bytes,
+                     void *stream);
 
 /* The reference's own form of algorithm ids 2-13 (ids 2-10 one wave per system),
  * with the reference's memory semantics (ids 3-10: c' into c and d' into d on the

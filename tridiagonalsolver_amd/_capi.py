@@ -79,6 +79,8 @@ def lib():
     L.tridiag_scratch_bytes.restype = i64
     L.tridiag_solve_scratch.argtypes = [ci, ci, ci, i64, i64, vp, vp, vp, vp, vp, i64, vp]
     L.tridiag_solve_scratch.restype = ci
+    L.tridiag_solve_to.argtypes = [ci, ci, ci, i64, i64, vp, vp, vp, vp, vp, vp, i64, vp]
+    L.tridiag_solve_to.restype = ci
     L.tridiag_solve_bulk.argtypes = [ci, ci, ci, i64, i64, vp, vp, vp, vp, vp]
     L.tridiag_solve_bulk.restype = ci
     L.tridiag_solve_noalloc.argtypes = [ci, ci, ci, i64, i64, vp, vp, vp, vp, vp]

@@ -632,7 +632,7 @@ static bool coop_plan(int algo, int layout, int64_t n, int64_t batch, const Tile
 
 template <typename T>
 static int coop_run(const SolvePlan<T> &pl, int layout, int64_t n, int64_t batch, int64_t sstride,
-                    T *a, T *b, T *c, T *d, hipStream_t st, const FixedScratch *fx) {
+                    T *a, T *b, T *c, T *d, T *x, hipStream_t st, const FixedScratch *fx) {
     const bool il = layout == kInterleaved;
     const CoopEntry<T> &e = *pl.coop;
     const int64_t ngroups = (batch + e.S - 1) / e.S;
@@ -644,7 +644,7 @@ static int coop_run(const SolvePlan<T> &pl, int layout, int64_t n, int64_t batch
         const hipError_t ea = hipMallocAsync(&scratch, pl.scratch_bytes, st);
         if (ea != hipSuccess) return hip_fail(ea, "cooperative solve scratch");
     }
-    CoopParams<T> p{a, b, c, d, n, batch, il ? 1 : sstride, il ? batch : 1,
+    CoopParams<T> p{a, b, c, d, x, n, batch, il ? 1 : sstride, il ? batch : 1,
                     (int32_t)(il ? n * batch * (int64_t)sizeof(T) : 0), (int32_t)pl.K,
                     (int32_t)ngroups,
                     il ? coop_spin_limit() : std::min(coop_spin_limit(), kCoopTreePolls),
@@ -677,14 +677,14 @@ static int convert_impl(int src_layout, int dst_layout, int64_t n, int64_t batch
                         const T *const src[4], T *const dst[4], hipStream_t st);
 template <typename T>
 static int solve_impl(int algo, int layout, int64_t n, int64_t batch, T *a, T *b, T *c, T *d,
-                      hipStream_t st, const FixedScratch *fx = nullptr);
+                      hipStream_t st, const FixedScratch *fx = nullptr, T *x = nullptr);
 
 // Interleaved systems longer than the interleaved tiles hold: converted to the
 // contiguous layout in stream-ordered scratch, solved there (the chunked solve for
 // long n), and x converted back.  Moves 8w + solve + 2w bytes per unknown.
 template <typename T>
 static int interleaved_via_contiguous(int algo, int64_t n, int64_t batch, T *a, T *b, T *c, T *d,
-                                      hipStream_t st) {
+                                      T *x, hipStream_t st) {
     const int64_t elems = n * batch;
     void *scratch = nullptr;
     hipError_t e = hipMallocAsync(&scratch, (size_t)(4 * elems) * sizeof(T), st);
@@ -697,7 +697,7 @@ static int interleaved_via_contiguous(int algo, int64_t n, int64_t batch, T *a, 
                                              dst[3], st);
     if (rc == TRIDIAG_OK) {
         const T *xs[4] = {nullptr, nullptr, nullptr, dst[3]};
-        T *xd[4] = {nullptr, nullptr, nullptr, d};
+        T *xd[4] = {nullptr, nullptr, nullptr, x};
         rc = convert_impl<T>(kContiguous, kInterleaved, n, batch, xs, xd, st);
     }
     const hipError_t ef = hipFreeAsync(scratch, st);
@@ -777,7 +777,7 @@ static SolvePlan<T> make_plan(int algo, int layout, int64_t n, int64_t batch, in
 
 template <typename T>
 static int solve_impl(int algo, int layout, int64_t n, int64_t batch, T *a, T *b, T *c, T *d,
-                      hipStream_t st, const FixedScratch *fx) {
+                      hipStream_t st, const FixedScratch *fx, T *x) {
     if (n < 1) return fail(TRIDIAG_EINVAL, "n_eqt must be >= 1");
     if (batch < 0) return fail(TRIDIAG_EINVAL, "n_batch must be >= 0");
     if (layout < 0 || layout > 2) return fail(TRIDIAG_EINVAL, "layout must be 0, 1 or 2");
@@ -803,7 +803,8 @@ static int solve_impl(int algo, int layout, int64_t n, int64_t batch, T *a, T *b
                 int rc = solve_impl<T>(algo, layout, n, cnt, a + o,
                                        layout == kPacked ? nullptr : b + o,
                                        layout == kPacked ? nullptr : c + o,
-                                       layout == kPacked ? nullptr : d + o, st, fx);
+                                       layout == kPacked ? nullptr : d + o, st, fx,
+                                       x ? x + o : nullptr);
                 if (rc != TRIDIAG_OK) return rc;
             }
             return TRIDIAG_OK;
@@ -812,30 +813,42 @@ static int solve_impl(int algo, int layout, int64_t n, int64_t batch, T *a, T *b
     if (layout == kPacked) {
         b = a + n; c = a + 2 * n; d = a + 3 * n;
     }
+    if (!x) x = d;
     const int V = 16 / (int)sizeof(T);
     const bool vec_ok = layout != kInterleaved && (sstride % V) == 0 && aligned16<T>(a) &&
-                        aligned16<T>(b) && aligned16<T>(c) && aligned16<T>(d);
+                        aligned16<T>(b) && aligned16<T>(c) && aligned16<T>(d) && aligned16<T>(x);
     const FixedScratch *only = fx && fx->only ? fx : nullptr;
     const SolvePlan<T> pl = make_plan<T>(algo, layout, n, batch, sstride, vec_ok,
                                          only ? only->bytes : 0);
     const int32_t bb = buffer_extent<T>(n, batch, sstride, layout);
     const bool il = layout == kInterleaved;
-    if (pl.coop) return coop_run<T>(pl, layout, n, batch, sstride, a, b, c, d, st, fx);
+    if (pl.coop) return coop_run<T>(pl, layout, n, batch, sstride, a, b, c, d, x, st, fx);
+    if (x != d && (pl.kind == kPlanThomas || pl.kind == kPlanBulk || pl.kind == kPlanChunked)) {
+        // these forms keep their own intermediate values in d (and c)
+        const LayoutMove<T> mv{{d}, {x}, il ? n : batch, il ? batch : n, il ? batch : n,
+                               il ? batch : n, 0};
+        hipError_t e;
+        if constexpr (sizeof(T) == 4) e = launch_layout_move_f32(mv, 1, false, st);
+        else e = launch_layout_move_f64(mv, 1, false, st);
+        if (e != hipSuccess) return hip_fail(e, "right-hand side copy");
+        d = x;
+    }
     switch (pl.kind) {
     case kPlanLane: {
         const hipError_t e = (sizeof(T) == 4)
-            ? launch_lane_thomas_f32((const float *)a, (const float *)b, (const float *)c, (float *)d,
-                                     n, batch, sstride, rstride, il, bb, st)
+            ? launch_lane_thomas_f32((const float *)a, (const float *)b, (const float *)c,
+                                     (const float *)d, (float *)x, n, batch, sstride, rstride, il, bb, st)
             : launch_lane_thomas_f64((const double *)a, (const double *)b, (const double *)c,
-                                     (double *)d, n, batch, sstride, rstride, il, bb, st);
+                                     (const double *)d, (double *)x, n, batch, sstride, rstride, il, bb, st);
         return e == hipSuccess ? TRIDIAG_OK : hip_fail(e, "lane Thomas launch");
     }
     case kPlanShort: {
         const hipError_t e = (sizeof(T) == 4)
-            ? launch_short_f32((const float *)a, (const float *)b, (const float *)c, (float *)d, n,
+            ? launch_short_f32((const float *)a, (const float *)b, (const float *)c,
+                               (const float *)d, (float *)x, n,
                                batch, st)
-            : launch_short_f64((const double *)a, (const double *)b, (const double *)c, (double *)d,
-                               n, batch, st);
+            : launch_short_f64((const double *)a, (const double *)b, (const double *)c,
+                               (const double *)d, (double *)x, n, batch, st);
         return e == hipSuccess ? TRIDIAG_OK : hip_fail(e, "short-system launch");
     }
     case kPlanThomas: {
@@ -870,12 +883,12 @@ static int solve_impl(int algo, int layout, int64_t n, int64_t batch, T *a, T *b
             return fail(TRIDIAG_EUNSUPPORTED,
                         "interleaved n_eqt=" + std::to_string(n) + " is solved through a "
                         "contiguous copy of all four arrays, which needs an allocation");
-        return interleaved_via_contiguous<T>(algo, n, batch, a, b, c, d, st);
+        return interleaved_via_contiguous<T>(algo, n, batch, a, b, c, d, x, st);
     default:
         break;
     }
     const AlgoSpec sp = algo_spec(algo);
-    TileParams<T> p{a, b, c, d, n, batch, sstride, rstride, bb, sp.iface, sp.xchg_lds};
+    TileParams<T> p{a, b, c, d, x, n, batch, sstride, rstride, bb, sp.iface, sp.xchg_lds};
     const hipError_t err = pl.tile->launch(p, st);
     if (err == hipErrorInvalidConfiguration)
         return fail(TRIDIAG_EUNSUPPORTED, "interface solver of algorithm " + std::to_string(algo) +
@@ -1073,7 +1086,7 @@ static int solve_tile_impl(int index, int iface, int layout, int64_t n, int64_t 
         return fail(TRIDIAG_EINVAL, "vector tile needs 16-byte aligned rows");
     const int32_t bb = buffer_extent<T>(n, batch, sstride, layout);
     if (bb == 0 && !e.BIG) return fail(TRIDIAG_EUNSUPPORTED, "arrays of 2 GiB or more need a BIG tile");
-    TileParams<T> p{a, b, c, d, n, batch, sstride, rstride, bb, iface, 0};
+    TileParams<T> p{a, b, c, d, d, n, batch, sstride, rstride, bb, iface, 0};
     hipError_t err = e.launch(p, st);
     return err == hipSuccess ? TRIDIAG_OK : hip_fail(err, "tile launch");
 }
@@ -1319,14 +1332,23 @@ int tridiag_algo_layout(int precision, int algo) {
 
 int tridiag_solve(int precision, int algo, int layout, int64_t n_eqt, int64_t n_batch, void *a,
                   void *b, void *c, void *d, void *stream) {
-    return tridiag_solve_scratch(precision, algo, layout, n_eqt, n_batch, a, b, c, d, nullptr, 0,
-                                 stream);
+    return tridiag_solve_to(precision, algo, layout, n_eqt, n_batch, a, b, c, d, d, nullptr, 0, stream);
 }
 
 int tridiag_solve_scratch(int precision, int algo, int layout, int64_t n_eqt, int64_t n_batch,
                           void *a, void *b, void *c, void *d, void *scratch, int64_t scratch_bytes,
                           void *stream) {
+    return tridiag_solve_to(precision, algo, layout, n_eqt, n_batch, a, b, c, d, d, scratch,
+                            scratch_bytes, stream);
+}
+
+int tridiag_solve_to(int precision, int algo, int layout, int64_t n_eqt, int64_t n_batch, void *a,
+                     void *b, void *c, void *d, void *x, void *scratch, int64_t scratch_bytes,
+                     void *stream) {
     g_last_error.clear();
+    if (x != d && (layout == kPacked || algo == kVendor))
+        return fail(TRIDIAG_EUNSUPPORTED, "packed systems and the vendor comparator are solved in place");
+    if (x != d && !x && n_batch > 0) return fail(TRIDIAG_EINVAL, "null solution pointer");
     if (precision != TRIDIAG_SINGLE && precision != TRIDIAG_DOUBLE)
         return fail(TRIDIAG_EINVAL, "precision must be 0 (single) or 1 (double)");
     if (algo != TRIDIAG_ALGO_AUTO && (algo < 0 || algo >= algo_count(precision)))
@@ -1354,9 +1376,11 @@ int tridiag_solve_scratch(int precision, int algo, int layout, int64_t n_eqt, in
     const FixedScratch given{scratch, (size_t)(scratch && scratch_bytes > 0 ? scratch_bytes : 0), false};
     if (precision == TRIDIAG_SINGLE)
         return solve_impl<float>(algo, layout, n_eqt, n_batch, (float *)a, (float *)b,
-                                 (float *)c, (float *)d, st, &given);
+                                 (float *)c, (float *)d, st, &given,
+                                 x == d ? nullptr : (float *)x);
     return solve_impl<double>(algo, layout, n_eqt, n_batch, (double *)a, (double *)b,
-                              (double *)c, (double *)d, st, &given);
+                              (double *)c, (double *)d, st, &given,
+                              x == d ? nullptr : (double *)x);
 }
 
 int tridiag_solve_bulk(int precision, int algo, int layout, int64_t n_eqt, int64_t n_batch,

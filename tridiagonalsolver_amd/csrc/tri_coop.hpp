@@ -56,8 +56,8 @@
 namespace tri {
 
 template <typename T> struct CoopParams {
-    const T *a, *b, *c;
-    T *d;
+    const T *a, *b, *c, *d;
+    T *x;                // the solution; d itself, or an array apart from all inputs
     int64_t n, batch;
     int64_t sstride;     // elements between consecutive systems (interleaved: 1)
     int64_t rstride;     // elements between consecutive rows (contiguous: 1)
@@ -399,7 +399,7 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(OC
 #pragma unroll
             for (int q = 0; q < M; ++q) xs[q] = __builtin_nan("");
         }
-        il_block_store<T, M, SW, S, true, true>(rr[3], brow + wrow, p.rstride, (int64_t)gi * S, n,
+        il_block_store<T, M, SW, S, true, true>(make_rsrc(p.x, p.buf_bytes), brow + wrow, p.rstride, (int64_t)gi * S, n,
                                                 p.batch, lane, sl, kw, xbuf[wave], xs);
         __syncthreads();                           // LDS of this task free before the next
     }
@@ -450,9 +450,7 @@ __device__ __forceinline__ void coop_finish(const CoopParams<T> &p, int gi, int 
 #pragma unroll
         for (int q = 0; q < M; ++q) xs[q] = __builtin_nan("");
     }
-    __amdgpu_buffer_rsrc_t rw[4];
-    coop_rsrc(p, rw);
-    il_block_store<T, M, SW, S, true, true>(rw[3], brow + wrow, p.rstride, (int64_t)gi * S, p.n,
+    il_block_store<T, M, SW, S, true, true>(make_rsrc(p.x, p.buf_bytes), brow + wrow, p.rstride, (int64_t)gi * S, p.n,
                                              p.batch, lane, sl, kw, xb, xs);
     __syncthreads();                           // LDS of this task free
 }

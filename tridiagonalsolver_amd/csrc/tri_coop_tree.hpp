@@ -233,7 +233,7 @@ __device__ __forceinline__ bool coop_tree_block(const CoopParams<T> &p, int task
         xn = (o.de[q] - al[64 * q] * xs[0]) - o.ga[q] * xn;
         xs[q + 1] = xn;
     }
-    contig_block_store<T, M, true>(rr[3], wrow, lane, lds.x[ws], xs);
+    contig_block_store<T, M, true>(make_rsrc(p.x + base, bytes), wrow, lane, lds.x[ws], xs);
     return true;
 }
 

@@ -98,21 +98,22 @@ template <typename T> TileTable<T> tile_table();
 template <> inline TileTable<float> tile_table<float>() { return tile_table_f32(); }
 template <> inline TileTable<double> tile_table<double>() { return tile_table_f64(); }
 
-// Systems of up to lane_thomas_max_rows() rows, one per lane, in registers.
+// Systems of up to lane_thomas_max_rows() rows, one per lane, in registers.  Here and below
+// x, where there is one, is d or an array apart from all inputs.
 int lane_thomas_max_rows(int precision);
-hipError_t launch_lane_thomas_f32(const float *a, const float *b, const float *c, float *d,
-                                  int64_t n, int64_t batch, int64_t sstride, int64_t rstride,
+hipError_t launch_lane_thomas_f32(const float *a, const float *b, const float *c, const float *d,
+                                  float *x, int64_t n, int64_t batch, int64_t sstride, int64_t rstride,
                                   bool il, int32_t bb, hipStream_t st);
-hipError_t launch_lane_thomas_f64(const double *a, const double *b, const double *c, double *d,
-                                  int64_t n, int64_t batch, int64_t sstride, int64_t rstride,
+hipError_t launch_lane_thomas_f64(const double *a, const double *b, const double *c, const double *d,
+                                  double *x, int64_t n, int64_t batch, int64_t sstride, int64_t rstride,
                                   bool il, int32_t bb, hipStream_t st);
 // Short contiguous systems (stride n, n <= kShortMaxRows), several per wave
 // (tri_short.hip); hipErrorInvalidValue beyond.
 constexpr int kShortMaxRows = 192;
-hipError_t launch_short_f32(const float *a, const float *b, const float *c, float *d, int64_t n,
-                            int64_t batch, hipStream_t st);
-hipError_t launch_short_f64(const double *a, const double *b, const double *c, double *d,
-                            int64_t n, int64_t batch, hipStream_t st);
+hipError_t launch_short_f32(const float *a, const float *b, const float *c, const float *d,
+                            float *x, int64_t n, int64_t batch, hipStream_t st);
+hipError_t launch_short_f64(const double *a, const double *b, const double *c, const double *d,
+                            double *x, int64_t n, int64_t batch, hipStream_t st);
 // Layout conversion of up to four coefficient arrays: each source is a rows x cols
 // matrix with row pitch ld_src, copied (transpose = false) or transposed into a
 // destination with row pitch ld_dst.  col_tiles is filled by the launcher.

@@ -41,12 +41,14 @@ __device__ __forceinline__ void lane_thomas_sweeps(T (&A)[N], T (&B)[N], T (&C)[
 // Interleaved layout: lane = system, one row of 64 consecutive systems per load.
 template <typename T, int N>
 __global__ void __launch_bounds__(256) lane_thomas_il_kernel(const T *a, const T *b, const T *c,
-                                                             T *d, int64_t n, int64_t batch,
-                                                             int64_t rstride, int32_t buf_bytes) {
+                                                             const T *d, T *x, int64_t n,
+                                                             int64_t batch, int64_t rstride,
+                                                             int32_t buf_bytes) {
     const int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (s >= batch) return;                       // no workgroup barriers below
     const __amdgpu_buffer_rsrc_t ra = make_rsrc(a, buf_bytes), rb = make_rsrc(b, buf_bytes),
-                                 rc = make_rsrc(c, buf_bytes), rd = make_rsrc(d, buf_bytes);
+                                 rc = make_rsrc(c, buf_bytes), rd = make_rsrc(d, buf_bytes),
+                                 rx = make_rsrc(x, buf_bytes);
     T A[N], B[N], C[N], D[N];
     const int vo = (int)(s * (int64_t)sizeof(T));
     const int rowb = (int)(rstride * (int64_t)sizeof(T));
@@ -61,7 +63,7 @@ __global__ void __launch_bounds__(256) lane_thomas_il_kernel(const T *a, const T
     lane_thomas_sweeps<T, N>(A, B, C, D, n);
 #pragma unroll
     for (int j = 0; j < N; ++j)
-        if (j < n) bstore<T, true>(D[j], rd, vo, j * rowb);
+        if (j < n) bstore<T, true>(D[j], rx, vo, j * rowb);
 }
 
 // Contiguous layout (system stride n): the 64 systems of a wave are 64*n consecutive
@@ -70,7 +72,8 @@ __global__ void __launch_bounds__(256) lane_thomas_il_kernel(const T *a, const T
 // lanes' row reads hit distinct banks.
 template <typename T, int N>
 __global__ void __launch_bounds__(256) lane_thomas_c_kernel(const T *a, const T *b, const T *c,
-                                                            T *d, int64_t n, int64_t batch) {
+                                                            const T *d, T *x, int64_t n,
+                                                            int64_t batch) {
     constexpr int VV = 16 / (int)sizeof(T);
     constexpr int NQ = (N + VV - 1) / VV;          // chunks per lane at n = N
     constexpr int PMAX = N | 1;
@@ -128,33 +131,33 @@ __global__ void __launch_bounds__(256) lane_thomas_c_kernel(const T *a, const T 
 #pragma unroll
         for (int v = 0; v < VV; ++v)
             if (e + v < lim) reinterpret_cast<T *>(&t)[v] = L[slot(e + v)];
-        tail_chunk_store<T, true>(t, rr[3], e, lim);
+        tail_chunk_store<T, true>(t, make_rsrc(x + base, nb), e, lim);
     }
 }
 
 template <typename T, int N>
-static hipError_t launch_lane(const T *a, const T *b, const T *c, T *d, int64_t n, int64_t batch,
-                              int64_t rstride, bool il, int32_t bb, hipStream_t st) {
+static hipError_t launch_lane(const T *a, const T *b, const T *c, const T *d, T *x, int64_t n,
+                              int64_t batch, int64_t rstride, bool il, int32_t bb, hipStream_t st) {
     const int64_t blocks = (batch + 255) / 256;
     if (blocks > 0x7fffffff) return hipErrorInvalidValue;
     if (il)
         hipLaunchKernelGGL((lane_thomas_il_kernel<T, N>), dim3((unsigned)blocks), dim3(256), 0, st,
-                           a, b, c, d, n, batch, rstride, bb);
+                           a, b, c, d, x, n, batch, rstride, bb);
     else
         hipLaunchKernelGGL((lane_thomas_c_kernel<T, N>), dim3((unsigned)blocks), dim3(256), 0, st,
-                           a, b, c, d, n, batch);
+                           a, b, c, d, x, n, batch);
     return hipGetLastError();
 }
 
 template <typename T>
-static hipError_t launch_lane_thomas(const T *a, const T *b, const T *c, T *d, int64_t n,
+static hipError_t launch_lane_thomas(const T *a, const T *b, const T *c, const T *d, T *x, int64_t n,
                                      int64_t batch, int64_t sstride, int64_t rstride, bool il,
                                      int32_t bb, hipStream_t st) {
     if (n < 1 || n > lane_thomas_max_rows(sizeof(T) == 4 ? 0 : 1)) return hipErrorInvalidValue;
     if (!il && sstride != n) return hipErrorInvalidValue;   // contiguous systems only
     if (batch <= 0) return hipSuccess;
 #define TRI_LANE(NN) \
-    if (n <= NN) return launch_lane<T, NN>(a, b, c, d, n, batch, rstride, il, bb, st);
+    if (n <= NN) return launch_lane<T, NN>(a, b, c, d, x, n, batch, rstride, il, bb, st);
     TRI_LANE(8)
     TRI_LANE(16)
     if constexpr (sizeof(T) == 4) { TRI_LANE(32) }
@@ -716,15 +719,15 @@ hipError_t launch_thomas_rows_f64(const double *a, const double *b, double *c, d
 
 int lane_thomas_max_rows(int precision) { return precision == 0 ? 32 : 16; }
 
-hipError_t launch_lane_thomas_f32(const float *a, const float *b, const float *c, float *d,
-                                  int64_t n, int64_t batch, int64_t sstride, int64_t rstride,
+hipError_t launch_lane_thomas_f32(const float *a, const float *b, const float *c, const float *d,
+                                  float *x, int64_t n, int64_t batch, int64_t sstride, int64_t rstride,
                                   bool il, int32_t bb, hipStream_t st) {
-    return launch_lane_thomas<float>(a, b, c, d, n, batch, sstride, rstride, il, bb, st);
+    return launch_lane_thomas<float>(a, b, c, d, x, n, batch, sstride, rstride, il, bb, st);
 }
-hipError_t launch_lane_thomas_f64(const double *a, const double *b, const double *c, double *d,
-                                  int64_t n, int64_t batch, int64_t sstride, int64_t rstride,
+hipError_t launch_lane_thomas_f64(const double *a, const double *b, const double *c, const double *d,
+                                  double *x, int64_t n, int64_t batch, int64_t sstride, int64_t rstride,
                                   bool il, int32_t bb, hipStream_t st) {
-    return launch_lane_thomas<double>(a, b, c, d, n, batch, sstride, rstride, il, bb, st);
+    return launch_lane_thomas<double>(a, b, c, d, x, n, batch, sstride, rstride, il, bb, st);
 }
 
 }  // namespace tri

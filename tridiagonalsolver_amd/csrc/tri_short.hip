@@ -28,8 +28,8 @@ template <typename T, int M> struct ShortShape {
 };
 
 template <typename T, int M, int P>
-__global__ void __launch_bounds__(256) short_kernel(const T *a, const T *b, const T *c, T *d,
-                                                    int64_t n, int64_t batch) {
+__global__ void __launch_bounds__(256) short_kernel(const T *a, const T *b, const T *c,
+                                                    const T *d, T *x, int64_t n, int64_t batch) {
     using Sh = ShortShape<T, M>;
     constexpr int G = 64 / P;                            // systems per wave
     constexpr int TOT = 64 * M * (int)sizeof(T) / 16;    // 16-byte chunks of a full block
@@ -93,24 +93,25 @@ __global__ void __launch_bounds__(256) short_kernel(const T *a, const T *b, cons
 #pragma unroll
     for (int q = 0; q < NQ; ++q)
         if ((q + 1) * 64 <= TOT || q * 64 + lane < TOT)
-            store16<true>(xb[q * 64 + lane], rr[3], lane * 16 + q * 1024);
+            store16<true>(xb[q * 64 + lane], make_rsrc(x + base, nb), lane * 16 + q * 1024);
 }
 
 template <typename T, int M, int P>
-static hipError_t launch_short_shape(const T *a, const T *b, const T *c, T *d, int64_t n,
-                                     int64_t batch, hipStream_t st) {
+static hipError_t launch_short_shape(const T *a, const T *b, const T *c, const T *d, T *x,
+                                     int64_t n, int64_t batch, hipStream_t st) {
     constexpr int G = 64 / P;
     const int64_t blocks = (batch + 4 * G - 1) / (4 * G);
     if (n > P * M || blocks > 0x7fffffff) return hipErrorInvalidValue;
     hipLaunchKernelGGL((short_kernel<T, M, P>), dim3((unsigned)blocks), dim3(256), 0, st, a, b, c,
-                       d, n, batch);
+                       d, x, n, batch);
     return hipGetLastError();
 }
 
 // Shapes by capacity P * M; the smallest that holds n runs.
 template <typename T> struct ShortEntry {
     int M, P;
-    hipError_t (*launch)(const T *, const T *, const T *, T *, int64_t, int64_t, hipStream_t);
+    hipError_t (*launch)(const T *, const T *, const T *, const T *, T *, int64_t, int64_t,
+                         hipStream_t);
 };
 #define TRI_SHORT(T, M, P) {M, P, &launch_short_shape<T, M, P>}
 #define TRI_SHORT_TABLE(T) \
@@ -125,20 +126,20 @@ static const ShortEntry<double> kShortF64[] = {TRI_SHORT_TABLE(double)};
 
 template <typename T, int N>
 static hipError_t launch_short(const ShortEntry<T> (&tab)[N], const T *a, const T *b, const T *c,
-                               T *d, int64_t n, int64_t batch, hipStream_t st) {
+                               const T *d, T *x, int64_t n, int64_t batch, hipStream_t st) {
     if (batch <= 0) return hipSuccess;
     for (const ShortEntry<T> &e : tab)
-        if (n <= e.M * e.P) return e.launch(a, b, c, d, n, batch, st);
+        if (n <= e.M * e.P) return e.launch(a, b, c, d, x, n, batch, st);
     return hipErrorInvalidValue;
 }
 
-hipError_t launch_short_f32(const float *a, const float *b, const float *c, float *d, int64_t n,
-                            int64_t batch, hipStream_t st) {
-    return launch_short(kShortF32, a, b, c, d, n, batch, st);
-}
-hipError_t launch_short_f64(const double *a, const double *b, const double *c, double *d,
+hipError_t launch_short_f32(const float *a, const float *b, const float *c, const float *d, float *x,
                             int64_t n, int64_t batch, hipStream_t st) {
-    return launch_short(kShortF64, a, b, c, d, n, batch, st);
+    return launch_short(kShortF32, a, b, c, d, x, n, batch, st);
+}
+hipError_t launch_short_f64(const double *a, const double *b, const double *c, const double *d,
+                            double *x, int64_t n, int64_t batch, hipStream_t st) {
+    return launch_short(kShortF64, a, b, c, d, x, n, batch, st);
 }
 
 }  // namespace tri

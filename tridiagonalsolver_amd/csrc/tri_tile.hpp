@@ -54,8 +54,8 @@ __device__ __forceinline__ int xcd_group(int b, int nblocks, int G) {
 }
 
 template <typename T> struct TileParams {
-    const T *a, *b, *c;
-    T *d;
+    const T *a, *b, *c, *d;
+    T *x;             // the solution; d itself, or an array apart from all inputs
     int64_t n, batch;
     int64_t sstride;  // distance between systems (IL: 1)
     int64_t rstride;  // distance between rows (IL: batch)
@@ -702,7 +702,7 @@ __global__ void __launch_bounds__(64 * NW)
 
     SweepOut<T, Sh::NI> o;
     const int32_t nb = BIG ? 0x7fffffff : prm.buf_bytes;
-    __amdgpu_buffer_rsrc_t rd_rsrc = make_rsrc(prm.d, nb);
+    const __amdgpu_buffer_rsrc_t rd_rsrc = make_rsrc(prm.d, nb), rx_rsrc = make_rsrc(prm.x, nb);
     const int vo = BIG ? 0 : (int)(((IL ? row0 * rs : row0) + base) * (int64_t)sizeof(T));
     const int rowb = (int)(rs * (int64_t)sizeof(T));
     if constexpr (BIG) {
@@ -802,7 +802,7 @@ __global__ void __launch_bounds__(64 * NW)
 #pragma unroll
         for (int j = 0; j < M; ++j)
             xs[j] = (j == 0) ? xL : ((j == M - 1) ? xR : de[(j >= 1 && j <= M - 2) ? j - 1 : 0]);
-        il_block_store<T, M, SW, S, NT, PAD>(rd_rsrc, (int64_t)ws * SW * M, rs, (int64_t)tile * S, n,
+        il_block_store<T, M, SW, S, NT, PAD>(rx_rsrc, (int64_t)ws * SW * M, rs, (int64_t)tile * S, n,
                                              prm.batch, lane, sl, kw, xbuf[wave], xs);
         return;
     }
@@ -826,14 +826,14 @@ __global__ void __launch_bounds__(64 * NW)
         wave_lds_sync();                          // all rows written before the block is read
         const int64_t sbase = PAD ? wave_uniform(base) : 0;
         const __amdgpu_buffer_rsrc_t rx =
-            PAD ? make_rsrc(prm.d + sbase, (int32_t)(n * (int64_t)sizeof(T))) : rd_rsrc;
+            PAD ? make_rsrc(prm.x + sbase, (int32_t)(n * (int64_t)sizeof(T))) : rx_rsrc;
         const int wvo = (int)(((PAD ? 0 : base) + (int64_t)ws * 64 * M) * (int64_t)sizeof(T)) + lane * 16;
 #pragma unroll
         for (int q = 0; q < NQ; ++q)
             store16<NT>(xbuf[wave][q * 64 + lane], rx, wvo + q * 1024);
         return;
     }
-    T *__restrict__ D = prm.d;
+    T *__restrict__ X = prm.x;
     if (!BIG && !fast && row0 + M <= n) {
         // padded tiles: a segment wholly inside the system (all but one per system)
         // stores without a predicate per row
@@ -849,9 +849,9 @@ __global__ void __launch_bounds__(64 * NW)
                 u32x4 xs;
 #pragma unroll
                 for (int vv = 0; vv < V; ++vv) reinterpret_cast<T *>(&xs)[vv] = xv[vv];
-                store16<NT>(xs, rd_rsrc, vo + j0 * (int)sizeof(T));   // VEC: rows are adjacent
+                store16<NT>(xs, rx_rsrc, vo + j0 * (int)sizeof(T));   // VEC: rows are adjacent
             } else {
-                bstore<T, NT>(xv[0], rd_rsrc, vo, j0 * rowb);
+                bstore<T, NT>(xv[0], rx_rsrc, vo, j0 * rowb);
             }
         }
         return;
@@ -870,12 +870,12 @@ __global__ void __launch_bounds__(64 * NW)
                 u32x4 xs;
 #pragma unroll
                 for (int vv = 0; vv < V; ++vv) reinterpret_cast<T *>(&xs)[vv] = xv[vv];
-                store16<NT>(xs, rd_rsrc, vo + j0 * (int)sizeof(T));   // VEC: rows are adjacent
+                store16<NT>(xs, rx_rsrc, vo + j0 * (int)sizeof(T));   // VEC: rows are adjacent
             } else {
 #pragma unroll
                 for (int vv = 0; vv < V; ++vv)
                     if (fast || r0 + vv < n)
-                        bstore<T, NT>(xv[vv], rd_rsrc, vo, (j0 + vv) * rowb);
+                        bstore<T, NT>(xv[vv], rx_rsrc, vo, (j0 + vv) * rowb);
             }
         } else {
             const int64_t r0 = row0 + j0;
@@ -884,12 +884,12 @@ __global__ void __launch_bounds__(64 * NW)
                 VT xs;
 #pragma unroll
                 for (int vv = 0; vv < V; ++vv) reinterpret_cast<T *>(&xs)[vv] = xv[vv];
-                *reinterpret_cast<VT *>(D + base + r0) = xs;
+                *reinterpret_cast<VT *>(X + base + r0) = xs;
             } else {
 #pragma unroll
                 for (int vv = 0; vv < V; ++vv) {
                     const int64_t r = r0 + vv;
-                    if (r < n) D[base + r * rs] = xv[vv];
+                    if (r < n) X[base + r * rs] = xv[vv];
                 }
             }
         }

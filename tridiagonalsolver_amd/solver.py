@@ -62,6 +62,18 @@ def _scratch(prec, algo, layout, n, batch, device):
     return torch.empty(size, dtype=torch.uint8, device=device) if size else None
 
 
+def _launch(prec, algo, layout, n, batch, args, x, device):
+    w = _scratch(prec, algo, layout, n, batch, device) if n > 512 and batch > 0 else None
+    if w is not None:
+        check(lib().tridiag_solve_to(prec, algo, layout, n, batch, *args, x, _ptr(w), w.numel(),
+                                     _stream_handle(device)))
+    elif x == args[3]:
+        check(lib().tridiag_solve(prec, algo, layout, n, batch, *args, _stream_handle(device)))
+    else:
+        check(lib().tridiag_solve_to(prec, algo, layout, n, batch, *args, x, None, 0,
+                                     _stream_handle(device)))
+
+
 def solve(a, b, c, d, algo=ALGO_AUTO, layout=CONTIGUOUS, n=None, batch=None):
     """Solves in place: x is written to d; c may be clobbered (naive Thomas writes c').
 
@@ -74,13 +86,7 @@ def solve(a, b, c, d, algo=ALGO_AUTO, layout=CONTIGUOUS, n=None, batch=None):
     prec = _precision(a)
     pa = _ptr(a)
     args = (pa, pa, pa, pa) if layout == PACKED else (pa, _ptr(b), _ptr(c), _ptr(d))
-    device = a.device
-    w = _scratch(prec, algo, layout, n, batch, device) if n > 512 and batch > 0 else None
-    if w is None:
-        check(lib().tridiag_solve(prec, algo, layout, n, batch, *args, _stream_handle(device)))
-    else:
-        check(lib().tridiag_solve_scratch(prec, algo, layout, n, batch, *args, _ptr(w), w.numel(),
-                                          _stream_handle(device)))
+    _launch(prec, algo, layout, n, batch, args, args[3], a.device)
     return a if layout == PACKED else d
 
 
@@ -218,7 +224,7 @@ def solve_fwd_bwd(a, b, c, d, g, layout=CONTIGUOUS, n=None, batch=None):
 class TridiagonalSolve(torch.autograd.Function):
     """x = A^{-1} d with A = tridiag(a, b, c); a_0 and c_{n-1} are not part of A.
 
-    Forward runs the on-chip solver on copies (inputs are not clobbered) and saves
+    Forward writes x to an array of its own (inputs are not clobbered) and saves
     only a, b, c and x.  Backward solves A^T lambda = dL/dx with the adjoint
     kernel, which recomputes its own elimination, and returns
     dL/da = -lambda x_{i-1}, dL/db = -lambda x, dL/dc = -lambda x_{i+1}, dL/dd = lambda.
@@ -227,9 +233,16 @@ class TridiagonalSolve(torch.autograd.Function):
     @staticmethod
     def forward(ctx, a, b, c, d, layout=CONTIGUOUS, algo=ALGO_AUTO):
         n, batch = _shape(d, layout, None, None)
-        x = d.contiguous().clone()
-        cc = c.contiguous().clone() if algo == 1 else c.contiguous()
-        solve(a.contiguous(), b.contiguous(), cc, x, algo=algo, layout=layout, n=n, batch=batch)
+        if layout == PACKED or algo == 0:           # solved in place only
+            x = d.contiguous().clone()
+            solve(a.contiguous(), b.contiguous(), c.contiguous(), x, algo=algo, layout=layout, n=n,
+                  batch=batch)
+        else:
+            cc = c.contiguous().clone() if algo == 1 else c.contiguous()
+            ts = (a.contiguous(), b.contiguous(), cc, d.contiguous())
+            _check_tensors(ts)
+            x = torch.empty_like(ts[3])
+            _launch(_precision(a), algo, layout, n, batch, [_ptr(t) for t in ts], _ptr(x), a.device)
         ctx.layout = layout
         ctx.save_for_backward(a, b, c, x)
         return x
