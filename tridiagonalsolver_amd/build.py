@@ -196,8 +196,12 @@ ADJ_C = {("float", 0): [(4, 8, 8)] + [(M, 8, S) for M in (8, 12) for S in (8, 4,
                         [(12, 4, S) for S in (4, 2, 1)] + [(12, 8, 1)],
          ("double", 1): [(4, 8, 8), (6, 8, 8)] + [(M, 4, S) for M in (8, 12) for S in (4, 2, 1)] +
                         [(8, 8, 1), (12, 8, 1)]}
-ADJ_IL = {"float": [(M, NW, 8) for M in (4, 8) for NW in (1, 2, 4, 8, 16)],
-          "double": [(M, NW, 4) for M in (4, 8) for NW in (1, 2, 4, 8, 16)]}
+# Interleaved: whole 128-byte row pieces where registers allow (a tile holds S systems'
+# rows five times), 64- and 32-byte pieces above.
+ADJ_IL = {"float": [(4, 2, 32), (4, 4, 32), (8, 4, 32), (12, 4, 32), (8, 8, 32), (12, 8, 32),
+                    (8, 16, 32), (12, 8, 16), (8, 16, 16), (8, 8, 8), (12, 8, 8), (8, 16, 8)],
+          "double": [(4, 2, 16), (6, 2, 16), (4, 4, 16), (6, 4, 16), (8, 4, 16), (6, 8, 16),
+                     (8, 8, 16), (6, 8, 8), (8, 8, 8), (6, 8, 4), (8, 8, 4)]}
 
 
 def _adjoint_source():
@@ -208,8 +212,6 @@ def _adjoint_source():
         for mode in (0, 1):
             ents += [(M, NW, S, False, mode) for (M, NW, S) in ADJ_C[T, mode]]
         for (M, NW, S) in ADJ_IL[T]:
-            if T == "double" and NW == 16:       # over the 128-VGPR budget of 1024 lanes
-                continue
             ents += [(M, NW, S, True, mode) for mode in (0, 1)]
         lines.append("AdjTable<%s> adj_table_%s() {" % (T, suffix))
         lines.append("    static const AdjEntry<%s> t[] = {" % T)

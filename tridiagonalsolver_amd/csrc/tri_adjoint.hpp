@@ -28,12 +28,8 @@ template <typename T> struct AdjParams {
     int64_t n, batch, sstride, rstride;
     int32_t buf_bytes;
     int32_t iface, xchg_lds;
+    int32_t line_tiles = 1;   // interleaved: neighbouring tiles that share lines (launch_adj)
 };
-
-template <typename T>
-__device__ __forceinline__ T rowload(__amdgpu_buffer_rsrc_t r, int vo, int64_t row, int64_t n) {
-    return (row >= 0 && row < n) ? bload<T>(r, vo, 0) : T(0);
-}
 
 // Contiguous layout: a wave's rows [wrow, wrow + 64*M) of one system are read as whole
 // 16-byte chunks (consecutive lanes, consecutive chunks; nontemporal).  The descriptor
@@ -93,12 +89,43 @@ __device__ __forceinline__ void adj_wave_store(__amdgpu_buffer_rsrc_t r, int64_t
                       (int)(wrow * (int64_t)sizeof(T)) + lane * 16 + q * 1024);
 }
 
-template <typename T, int M, int NW, int S, bool IL, int MODE>
+// Interleaved layout: the same for rows [wrow, wrow + SW*M) of S neighbouring systems, as
+// whole row pieces of S*sizeof(T) bytes; rows at or past n lie past the buffer.
+template <typename T, int M, int S, bool NT>
+__device__ __forceinline__ void adj_il_issue(__amdgpu_buffer_rsrc_t r, int64_t wrow, int64_t rs,
+                                             int64_t col0, int64_t n, int lane,
+                                             u32x4 (&g)[M * (int)sizeof(T) / 16]) {
+    constexpr int CPR = S * (int)sizeof(T) / 16;
+#pragma unroll
+    for (int q = 0; q < M * (int)sizeof(T) / 16; ++q) {
+        const int cidx = q * 64 + lane;
+        g[q] = __builtin_amdgcn_raw_buffer_load_b128(
+            r, il_chunk_offset<T, true>(wrow + cidx / CPR, rs, col0, n, cidx % CPR), 0, cpol<NT>());
+    }
+}
+
+template <typename T, int M, int S>
+__device__ __forceinline__ void adj_il_take(const u32x4 (&g)[M * (int)sizeof(T) / 16], int lane,
+                                            u32x4 *xb, T (&rows)[M], T &prev, T &next) {
+    const int sl = lane % S, kw = lane / S;
+    wave_lds_sync();                                  // the block is free
+#pragma unroll
+    for (int q = 0; q < M * (int)sizeof(T) / 16; ++q) xb[q * 64 + lane] = g[q];
+    wave_lds_sync();
+    const T *tb = reinterpret_cast<const T *>(xb);
+#pragma unroll
+    for (int j = 0; j < M; ++j) rows[j] = tb[(kw * M + j) * S + sl];
+    if (kw > 0) prev = tb[(kw * M - 1) * S + sl];
+    if (kw < 64 / S - 1) next = tb[(kw * M + M) * S + sl];
+}
+
+// NT: the loads stream (interleaved rows on 128-byte lines; contiguous rows always do).
+template <typename T, int M, int NW, int S, bool IL, int MODE, bool NT>
 __global__ void __launch_bounds__(64 * NW) tile_adj_kernel(AdjParams<T> prm) {
     using Sh = TileShape<T, M, NW, S, IL, false, false, false, true, false, false>;
     constexpr int SW = Sh::SW, NWS = Sh::NWS, LS = Sh::LS, CH = Sh::CH;
     constexpr int LANES = 64 * NW;
-    static_assert(IL || M * (int)sizeof(T) >= 16, "contiguous adjoint tiles move 16-byte chunks");
+    static_assert((IL ? S : M) * (int)sizeof(T) >= 16, "adjoint tiles move 16-byte chunks");
     extern __shared__ __attribute__((aligned(16))) char tri_dyn_lds[];
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -108,7 +135,7 @@ __global__ void __launch_bounds__(64 * NW) tile_adj_kernel(AdjParams<T> prm) {
     const int ws = IL ? wave : (wave % NWS);
     const int64_t n = prm.n;
     int tile = blockIdx.x;
-    if (IL) tile = xcd_group(blockIdx.x, gridDim.x, 128 / (S * (int)sizeof(T)));
+    if (IL) tile = xcd_group(blockIdx.x, gridDim.x, prm.line_tiles);
     const int64_t sys = (int64_t)tile * S + sl;
     const bool valid = sys < prm.batch;
     const int64_t sysc = valid ? sys : prm.batch - 1;
@@ -118,37 +145,47 @@ __global__ void __launch_bounds__(64 * NW) tile_adj_kernel(AdjParams<T> prm) {
     // raw rows j = 0..M-1 plus the neighbours needed by A^T at the segment edges
     T ra[M], rb[M], rc[M], rg[M], rx[M];
     T c_before, a_after, x_before = 0, x_after = 0;
-    __shared__ u32x4 xbuf[IL ? 1 : NW][IL ? 1 : 64 * M * (int)sizeof(T) / 16];
-    (void)xbuf;
+    __shared__ u32x4 xbuf[NW][64 * M * (int)sizeof(T) / 16];
     // contiguous: per-wave descriptors on the system's own rows (none of an idle wave)
     const int64_t sbase = IL ? 0 : wave_uniform(sysc * n);
     const int32_t sbytes = valid ? (int32_t)(n * (int64_t)sizeof(T)) : 0;
-    const int64_t wrow = (int64_t)ws * 64 * M;
+    const int64_t wrow = (int64_t)ws * SW * M;
     auto RW = [&](const T *p) { return make_rsrc(p + sbase, sbytes); };
     if constexpr (IL) {
-        const int64_t rs = prm.rstride;
-        const int nb = prm.buf_bytes;
-        const int rowb = (int)(rs * (int64_t)sizeof(T));
-        const int vo0 = (int)((sysc + row0 * rs) * (int64_t)sizeof(T));
-        auto RS = [&](const T *p) { return make_rsrc(p, nb); };
-        const __amdgpu_buffer_rsrc_t rA = RS(prm.a), rB = RS(prm.b), rC = RS(prm.c);
-#pragma unroll
-        for (int j = 0; j < M; ++j) {
-            const int64_t r = row0 + j;
-            const int vo = vo0 + j * rowb;
-            rb[j] = rowload<T>(rB, vo, r, n);
-            rc[j] = rowload<T>(rC, vo, r, n);
-            ra[j] = rowload<T>(rA, vo, r, n);
-            rg[j] = rowload<T>(RS(prm.g), vo, r, n);
-            if constexpr (MODE == kFused) rx[j] = rowload<T>(RS(prm.d), vo, r, n);
-            else rx[j] = rowload<T>(RS(prm.x), vo, r, n);
-        }
-        c_before = rowload<T>(rC, vo0 - rowb, row0 - 1, n);      // c_{row0-1}
-        a_after = rowload<T>(rA, vo0 + M * rowb, row0 + M, n);   // a_{row0+M}
+        // as below, two arrays in flight; the rows just outside the wave's block are read by
+        // the lanes at its ends.  Reading 32-byte pieces one element per lane and row took
+        // (us, before / now): FP32 fused 60 x 60,000 50.5 / 32.4, 60 x 59,999 78.2 / 35.4, 448 x
+        // 8192 67.4 / 45.9; adjoint FP32 170 x 20,000 42.7 / 25.6, FP64 250 x 8000 69.0 / 35.2
+        // (4.1 TB/s).  The fused kernels hold five arrays and two solves in registers, which
+        // leaves two or three waves per SIMD.
+        constexpr int NQ = M * (int)sizeof(T) / 16;
+        const int64_t rs = prm.rstride, col0 = (int64_t)tile * S;
+        u32x4 g[5][NQ];
+        u32x4 *xb = xbuf[wave];
+        T unused = 0;
+        auto issue = [&](const T *p, u32x4 (&q)[NQ]) {
+            adj_il_issue<T, M, S, NT>(make_rsrc(p, prm.buf_bytes), wrow, rs, col0, n, lane, q);
+        };
+        auto outside = [&](const T *p, int64_t r, bool end) {
+            const int vo = (int)((r * rs + sysc) * (int64_t)sizeof(T));
+            return bload<T>(make_rsrc(p, prm.buf_bytes), end && r >= 0 && r < n ? vo : 0x7fffff00, 0);
+        };
+        issue(prm.b, g[0]);
+        issue(prm.c, g[1]);
+        c_before = outside(prm.c, wrow - 1, kw == 0);
+        a_after = outside(prm.a, wrow + SW * M, kw == SW - 1);
         if constexpr (MODE == kAdjoint) {
-            x_before = rowload<T>(RS(prm.x), vo0 - rowb, row0 - 1, n);
-            x_after = rowload<T>(RS(prm.x), vo0 + M * rowb, row0 + M, n);
+            x_before = outside(prm.x, wrow - 1, kw == 0);
+            x_after = outside(prm.x, wrow + SW * M, kw == SW - 1);
         }
+        adj_il_take<T, M, S>(g[0], lane, xb, rb, unused, unused);
+        issue(prm.a, g[2]);
+        adj_il_take<T, M, S>(g[1], lane, xb, rc, c_before, unused);
+        issue(prm.g, g[3]);
+        adj_il_take<T, M, S>(g[2], lane, xb, ra, unused, a_after);
+        issue(MODE == kFused ? prm.d : prm.x, g[4]);
+        adj_il_take<T, M, S>(g[3], lane, xb, rg, unused, unused);
+        adj_il_take<T, M, S>(g[4], lane, xb, rx, x_before, x_after);
     } else {
         // Two arrays in flight: the next one is issued while the first goes through LDS.
         // The kernel streams, so what counts is that loads never drain: one array at a
@@ -260,7 +297,7 @@ __global__ void __launch_bounds__(64 * NW) tile_adj_kernel(AdjParams<T> prm) {
             lam[j + 1] = ln;
         }
     }
-    if (!valid) return;
+    if (!IL && !valid) return;      // interleaved stores go by position, not by system
 
     // ------------------------------------------------------------ gradients
     // ga_i = -lambda_i x_{i-1}, gb_i = -lambda_i x_i, gc_i = -lambda_i x_{i+1}, gd_i = lambda_i
@@ -278,15 +315,14 @@ __global__ void __launch_bounds__(64 * NW) tile_adj_kernel(AdjParams<T> prm) {
     T *outs[5] = {prm.ga, prm.gb, prm.gc, prm.gd, prm.xo};
     constexpr int NOUT = (MODE == kFused) ? 5 : 4;
     if constexpr (IL) {
-        const int64_t rs = prm.rstride;
-        const int rowb = (int)(rs * (int64_t)sizeof(T));
-        const int vo0 = (int)((sysc + row0 * rs) * (int64_t)sizeof(T));
 #pragma unroll
         for (int k = 0; k < NOUT; ++k) {
-            const __amdgpu_buffer_rsrc_t w = make_rsrc(outs[k], prm.buf_bytes);
+            T v[M];
 #pragma unroll
-            for (int j = 0; j < M; ++j)
-                if (row0 + j < n) bstore<T>(grad(k, j), w, vo0 + j * rowb, 0);
+            for (int j = 0; j < M; ++j) v[j] = grad(k, j);
+            il_block_store<T, M, SW, S, NT, true>(make_rsrc(outs[k], prm.buf_bytes), wrow, prm.rstride,
+                                                  (int64_t)tile * S, n, prm.batch, lane, sl, kw,
+                                                  xbuf[wave], v);
         }
     } else {
         if (wrow >= n) return;                             // wave-uniform
@@ -313,13 +349,21 @@ hipError_t launch_adj(const AdjParams<T> &p, hipStream_t st) {
     const int64_t tiles = (p.batch + S - 1) / S;
     if (tiles <= 0) return hipSuccess;
     if (tiles > 0x7fffffff) return hipErrorInvalidValue;
-    auto kern = tile_adj_kernel<T, M, NW, S, IL, MODE>;
+    // Interleaved: 128-byte pieces of rows on lines stream; narrower pieces and rows off
+    // lines share lines with their neighbours, so the loads stay cached and runs of
+    // neighbouring tiles go to one XCD.
+    constexpr int LT = IL && S * (int)sizeof(T) < 128 ? 128 / (S * (int)sizeof(T)) : 1;
+    const bool shared = IL && (LT > 1 || (p.rstride * (int64_t)sizeof(T)) % 128 != 0);
+    AdjParams<T> q = p;
+    q.line_tiles = shared && LT == 1 ? 16 : LT;
+    auto kern = tile_adj_kernel<T, M, NW, S, IL, MODE, (LT == 1)>;
+    if (shared) kern = tile_adj_kernel<T, M, NW, S, IL, MODE, !IL>;
     size_t dyn = 0;
     if (iface_family(p.iface) >= kIfacePCR) dyn = (size_t)iface_lds_bytes<T>(64 * NW);
     else if (p.xchg_lds) dyn = (size_t)6 * 64 * NW * sizeof(T);
     if (dyn) {
-        static size_t granted = 0;
-        if (dyn > granted) {
+        static size_t granted[2] = {0, 0};
+        if (dyn > granted[shared]) {
             hipFuncAttributes fa;
             hipError_t e = hipFuncGetAttributes(&fa, reinterpret_cast<const void *>(kern));
             if (e != hipSuccess) return e;
@@ -327,10 +371,10 @@ hipError_t launch_adj(const AdjParams<T> &p, hipStream_t st) {
             e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)dyn);
             if (e != hipSuccess) return e;
-            granted = dyn;
+            granted[shared] = dyn;
         }
     }
-    hipLaunchKernelGGL(kern, dim3((unsigned)tiles), dim3(64 * NW), dyn, st, p);
+    hipLaunchKernelGGL(kern, dim3((unsigned)tiles), dim3(64 * NW), dyn, st, q);
     return hipGetLastError();
 }
 
