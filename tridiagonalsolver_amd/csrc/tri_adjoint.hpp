@@ -151,6 +151,14 @@ __global__ void __launch_bounds__(64 * NW) tile_adj_kernel(AdjParams<T> prm) {
     const int32_t sbytes = valid ? (int32_t)(n * (int64_t)sizeof(T)) : 0;
     const int64_t wrow = (int64_t)ws * SW * M;
     auto RW = [&](const T *p) { return make_rsrc(p + sbase, sbytes); };
+    // The last array, which only the second half of the work reads (fused: g; adjoint: x),
+    // stays in flight during the first solve.  MI355X, taken at once / this (us): FP32 fused
+    // 600 x 8000 41.0 / 39.6, 2048 x 2000 33.9 / 32.5, FP64 2000 x 1000 37.0 / 35.3; adjoint
+    // FP32 512 x 8192 28.3 / 27.0, 100 x 40,000 35.6 / 33.5, FP64 500 x 4000 29.4 / 28.3.  The
+    // adjoint of contiguous systems of several waves does not gain (FP32 2047 x 2048 28.2 /
+    // 29.3, FP64 777 x 4000 42.8 / 43.2) and takes x at once.
+    constexpr bool kLater = MODE == kFused || IL || NWS == 1;
+    u32x4 last[M * (int)sizeof(T) / 16];
     if constexpr (IL) {
         // as below, two arrays in flight; the rows just outside the wave's block are read by
         // the lanes at its ends.  Reading 32-byte pieces one element per lane and row took
@@ -160,7 +168,7 @@ __global__ void __launch_bounds__(64 * NW) tile_adj_kernel(AdjParams<T> prm) {
         // leaves two or three waves per SIMD.
         constexpr int NQ = M * (int)sizeof(T) / 16;
         const int64_t rs = prm.rstride, col0 = (int64_t)tile * S;
-        u32x4 g[5][NQ];
+        u32x4 g[4][NQ];
         u32x4 *xb = xbuf[wave];
         T unused = 0;
         auto issue = [&](const T *p, u32x4 (&q)[NQ]) {
@@ -181,11 +189,10 @@ __global__ void __launch_bounds__(64 * NW) tile_adj_kernel(AdjParams<T> prm) {
         adj_il_take<T, M, S>(g[0], lane, xb, rb, unused, unused);
         issue(prm.a, g[2]);
         adj_il_take<T, M, S>(g[1], lane, xb, rc, c_before, unused);
-        issue(prm.g, g[3]);
+        issue(MODE == kFused ? prm.d : prm.g, g[3]);
         adj_il_take<T, M, S>(g[2], lane, xb, ra, unused, a_after);
-        issue(MODE == kFused ? prm.d : prm.x, g[4]);
-        adj_il_take<T, M, S>(g[3], lane, xb, rg, unused, unused);
-        adj_il_take<T, M, S>(g[4], lane, xb, rx, x_before, x_after);
+        issue(MODE == kFused ? prm.g : prm.x, last);
+        adj_il_take<T, M, S>(g[3], lane, xb, MODE == kFused ? rx : rg, unused, unused);
     } else {
         // Two arrays in flight: the next one is issued while the first goes through LDS.
         // The kernel streams, so what counts is that loads never drain: one array at a
@@ -197,12 +204,11 @@ __global__ void __launch_bounds__(64 * NW) tile_adj_kernel(AdjParams<T> prm) {
         // descriptor's bounds (FP64 adjoint 777 x 4000) 62.0, now 43.0; FP32 2047 x 2048
         // 35.2, now 28.4.
         constexpr int NQ = M * (int)sizeof(T) / 16;
-        u32x4 g[5][NQ];
-        const T *in[5] = {prm.b, prm.c, prm.a, prm.g, MODE == kFused ? prm.d : prm.x};
+        u32x4 g[4][NQ];
         u32x4 *xb = xbuf[wave];
         T unused = 0;
-        adj_issue<T, M>(RW(in[0]), wrow, lane, g[0]);
-        adj_issue<T, M>(RW(in[1]), wrow, lane, g[1]);
+        adj_issue<T, M>(RW(prm.b), wrow, lane, g[0]);
+        adj_issue<T, M>(RW(prm.c), wrow, lane, g[1]);
         c_before = 0;
         a_after = 0;
         if constexpr (NWS > 1) {
@@ -218,14 +224,18 @@ __global__ void __launch_bounds__(64 * NW) tile_adj_kernel(AdjParams<T> prm) {
             }
         }
         adj_take<T, M>(g[0], lane, xb, rb, unused, unused);
-        adj_issue<T, M>(RW(in[2]), wrow, lane, g[2]);
+        adj_issue<T, M>(RW(prm.a), wrow, lane, g[2]);
         adj_take<T, M>(g[1], lane, xb, rc, c_before, unused);
-        adj_issue<T, M>(RW(in[3]), wrow, lane, g[3]);
+        adj_issue<T, M>(RW(MODE == kFused ? prm.d : prm.g), wrow, lane, g[3]);
         adj_take<T, M>(g[2], lane, xb, ra, unused, a_after);
-        adj_issue<T, M>(RW(in[4]), wrow, lane, g[4]);
-        adj_take<T, M>(g[3], lane, xb, rg, unused, unused);
-        adj_take<T, M>(g[4], lane, xb, rx, x_before, x_after);
+        adj_issue<T, M>(RW(MODE == kFused ? prm.g : prm.x), wrow, lane, last);
+        adj_take<T, M>(g[3], lane, xb, MODE == kFused ? rx : rg, unused, unused);
     }
+    auto take_last = [&](T (&rows)[M], T &prev, T &next) {
+        if constexpr (IL) adj_il_take<T, M, S>(last, lane, xbuf[wave], rows, prev, next);
+        else adj_take<T, M>(last, lane, xbuf[wave], rows, prev, next);
+    };
+    if constexpr (!kLater) take_last(rx, x_before, x_after);
 #pragma unroll
     for (int j = 0; j < M; ++j)
         if (row0 + j >= n) rb[j] = 1;                    // identity rows past the end
@@ -265,6 +275,8 @@ __global__ void __launch_bounds__(64 * NW) tile_adj_kernel(AdjParams<T> prm) {
         x_before = (seg > 0) ? sh_x[sl][2 * seg - 1] : T(0);
         x_after = (seg + 1 < Sh::P) ? sh_x[sl][2 * seg + 2] : T(0);
         __syncthreads();   // interface LDS is reused by the adjoint solve
+        T unused = 0;
+        take_last(rg, unused, unused);
     }
 
     // ------------------------------------------------------------ adjoint solve
@@ -297,6 +309,7 @@ __global__ void __launch_bounds__(64 * NW) tile_adj_kernel(AdjParams<T> prm) {
             lam[j + 1] = ln;
         }
     }
+    if constexpr (MODE == kAdjoint && kLater) take_last(rx, x_before, x_after);
     if (!IL && !valid) return;      // interleaved stores go by position, not by system
 
     // ------------------------------------------------------------ gradients
