@@ -460,8 +460,7 @@ static int32_t coop_spread(int groups_per_round) {
 // The entry of the cooperative table for a batch, K = blocks per system (K >= 2) and P =
 // workgroups of its grid: the tasks, or as many whole groups as are resident at once.
 //
-// Interleaved: the first entry whose blocks divide n and whose kmax holds K (up to 64
-// blocks, 16384 rows).
+// Interleaved: up to 64 blocks (16384 rows), the last of which may be partial.
 //
 // Contiguous: small blocks up to 64 of them, or where the whole batch is one round of the
 // grid (more CUs per row); large blocks above (fewer forms to read and flags to wait

@@ -88,26 +88,25 @@ hipError_t launch_coop_clear(uint64_t *words, int64_t count, hipStream_t st) {
      &coop_tree_max_grid<T, M, NW, OCC>}
 
 // Interleaved: S systems = one 128-byte line per row, blocks of 2*NW*M (FP32) or
-// 4*NW*M (FP64) rows, up to 32 blocks, and an entry for 33-64 blocks whose larger
-// block-form staging leaves one workgroup per CU (interleaved 12288 / 16384 rows x
-// 1024: FP32 0.129 / 0.167 ms, FP64 0.266 / 0.367 ms, against 0.164 / 0.213 and
-// 0.363 / 0.477 ms through a contiguous copy).  PIPE: coop_pipe_kernel by default;
-// OCC: waves per SIMD.
-// Measured on MI355X (ms; 16.7 M unknowns):
-//   FP32 4096 x 4096: pipelined 0.109; no prefetch, 2 per CU (OCC 4) 0.108.  FP32
-//   2048 x 8192: 0.102 / 0.091 (pipelined / OCC 4); 8192 x 2048: 0.129 / 0.123.  FP64
-//   4096 x 4096: 0.223 / 0.214.  Blocks of 128 rows (M = 8 FP32, 4 FP64) with K = 32:
-//   0.148 / 0.282; 16-wave workgroups of M = 8 / 4 (one per CU): 0.133 / 0.286.
+// 4*NW*M (FP64) rows, up to 64 blocks (16384 rows), two workgroups per CU.  PIPE:
+// coop_pipe_kernel by default; OCC: waves per SIMD.  Measured on MI355X (us): pipelined
+// instead FP32 4096 x 4096 100, FP64 211; blocks of 128 rows (M = 8 FP32, 4 FP64) and
+// 16-wave workgroups were slower or even.
+// With the block forms [system][block][6] in LDS (all lanes of an access on one bank), in a
+// buffer of their own (one workgroup per CU above 32 blocks) and two serial chains, / now:
+// FP32 4096 x 4096 89.8 / 87.7, 600 x 16,000 49.6 / 48.5, 8192 x 2048 97.0 / 91.9, 16,000 x 500
+// 92.7 / 62.3; FP64 3001 x 1001 42.3 / 40.4, 3001 x 1008 34.1 / 30.0 (4.0 TB/s), 9000 x 250
+// 58.5 / 41.4.  The loads' pattern alone (pieces of one line, 256 rows per task) takes 70-86
+// us at FP32 4096 x 4096, which bounds the large sizes; the rest is the wait for the group
+// and the phases that no second workgroup covers.
 // Contiguous: one system, blocks of 64*NW*M rows, up to 64*NW blocks; small blocks
 // first (choose_coop says which).  Both run 16 waves per CU, four or two workgroups.
 static const CoopEntry<float> kCoopF32[] = {
-    TRI_COOP_ENTRY(float, 16, 8, 32, 32, false, 4),
     TRI_COOP_ENTRY(float, 16, 8, 32, 64, false, 4),
     TRI_COOP_TREE(float, 16, 4, 4),
     TRI_COOP_TREE(float, 16, 8, 4),
 };
 static const CoopEntry<double> kCoopF64[] = {
-    TRI_COOP_ENTRY(double, 8, 8, 16, 32, false, 4),
     TRI_COOP_ENTRY(double, 8, 8, 16, 64, false, 4),
     TRI_COOP_TREE(double, 8, 4, 4),
     TRI_COOP_TREE(double, 8, 8, 4),

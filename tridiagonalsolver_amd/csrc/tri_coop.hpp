@@ -8,17 +8,15 @@
 //
 //   task (g, j) = rows [j*R, (j+1)*R) of the S systems of group g
 //     1. the block's rows (whole row pieces of S*sizeof(T) bytes) go to the lanes
-//        through LDS; lane
-//        sweeps, Wang-Mou merges inside each wave and a fold over the waves give
-//        the block's first row F and last row E in outer form relative to
-//        U = x of the row before the block and V = x of the row after it
-//     2. those 6 values per system are published; the loads of the workgroup's
-//        next task are issued; then it waits until the other K-1 blocks of the
-//        group have published theirs
-//     3. a partial-elimination chain over the K block forms of each system gives
-//        U and V of the block, a second chain over the block's waves gives x at
-//        every wave boundary, and the lanes back-substitute from registers and
-//        store x
+//        through LDS; lane sweeps and Wang-Mou merges inside each wave and across the
+//        waves give the block's first row F and last row E in outer form relative to
+//        U = x of the row before the block and V = x of the row after it, and the same
+//        for every wave-block's ends
+//     2. those 6 values per system are published, and the workgroup waits until the
+//        other K-1 blocks of the group have published theirs
+//     3. partial elimination over the block forms on either side of the block gives U
+//        and V, with them the wave-blocks' ends, and the lanes back-substitute from
+//        registers and store x
 //
 // Schedule: the grid is P workgroups, all resident at once (P is at most what the
 // device holds, and a multiple of K), and workgroup w takes tasks w, w + P,
@@ -68,7 +66,7 @@ template <typename T> struct CoopParams {
     int32_t pipelined;   // 1: coop_pipe_kernel (wait one task later), 0: coop_kernel
     int32_t spread;      // groups per round whose slots are spread over the batch (<= 1: none)
     int32_t shared_lines;  // interleaved rows start off 128-byte lines (coop_task_shared)
-    T *forms;            // [ngroups][K][S][6] block outer forms
+    T *forms;            // [ngroups][K][6][S] block outer forms
     uint64_t *flags;     // [kCoopFlagStride * g + j]: the tag once block j of group g is published
     uint64_t tag;        // this solve's tag: different from every earlier solve's
     uint64_t *done;      // coop_tree_kernel: the tag once block t of the grid is solved
@@ -118,26 +116,19 @@ __device__ __forceinline__ int coop_wait(const CoopParams<T> &p, int g, int lane
     }
 }
 
-// Stages the K block forms of a group (K*S*6 values at fg, block-major) into
-// sh_k[system][block][6] with the whole workgroup.  In FP32 each thread issues 8
-// loads before it stores the first: the loads are agent-scope (they go past the
-// XCD's L2 to where all XCDs meet), and one after another their latencies add up.
-// The FP64 kernels have no registers to spare (measured: FP64 65,536 x 256 0.173
-// -> 0.182 ms with the batched form) and load one value at a time.  ok == false
-// (a wait that gave up): zeros, and no loads.
-template <typename T, int S, int NW, int KMAX>
-__device__ __forceinline__ void coop_stage_forms(const T *fg, int K, bool ok, int tid,
-                                                 T (*sh_k)[KMAX][6]) {
-    constexpr int NT = 64 * NW, B = 8;
-    const int ne = K * S * 6;
-    if constexpr (sizeof(T) != 4) {
-        for (int e = tid; e < ne; e += NT) {
-            const int k = e / (S * 6), r = e - k * (S * 6);
-            sh_k[r / 6][k][r % 6] =
-                ok ? __hip_atomic_load(fg + e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : T(0);
-        }
-        return;
-    }
+// Forms are kept value by value, [block][6][S], in global memory and in LDS: the S lanes
+// that handle one value of a block are consecutive, so global accesses coalesce and LDS
+// accesses hit distinct banks.  ([system][block][6], strides of 6 * KMAX words, put the
+// lanes of every access of the chain on one LDS bank.)
+//
+// Stages the K block forms of a group (K*6*S values at fg) into sh_k with the whole
+// workgroup.  Each thread issues several loads before it stores the first: the loads are
+// agent-scope (they go past the XCD's L2 to where all XCDs meet), and one after another
+// their latencies add up.  ok == false (a wait that gave up): zeros, and no loads.
+template <typename T, int S, int NW>
+__device__ __forceinline__ void coop_stage_forms(const T *fg, int K, bool ok, int tid, T *sh_k) {
+    constexpr int NT = 64 * NW, B = sizeof(T) == 4 ? 8 : 4;
+    const int ne = K * 6 * S;
     for (int e0 = 0; e0 < ne; e0 += NT * B) {
         T v[B];
 #pragma unroll
@@ -149,147 +140,60 @@ __device__ __forceinline__ void coop_stage_forms(const T *fg, int K, bool ok, in
 #pragma unroll
         for (int i = 0; i < B; ++i) {
             const int e = e0 + i * NT + tid;
-            if (e < ne) {
-                const int k = e / (S * 6), r = e - k * (S * 6);
-                sh_k[r / 6][k][r % 6] = v[i];
-            }
+            if (e < ne) sh_k[e] = v[i];
         }
     }
 }
 
-// Folds wave-block outer forms w = 0..nw-1 (first row at [w][0..2], last row at
-// [w][3..5]) left to right into the outer form of the whole block.
-template <typename T>
-__device__ __forceinline__ void fold_blocks(const T (*blk)[6], int nw, Outer<T> &F, Outer<T> &E) {
-    F = {blk[0][0], blk[0][1], blk[0][2]};
-    E = {blk[0][3], blk[0][4], blk[0][5]};
-    for (int w = 1; w < nw; ++w) {
-        const Outer<T> BF{blk[w][0], blk[w][1], blk[w][2]};
-        Outer<T> BE{blk[w][3], blk[w][4], blk[w][5]};
-        T RB, PB, QB, RA, PA, QA;
-        wm_pair_coeffs(E.r, E.p, E.q, BF.r, BF.p, BF.q, RB, PB, QB, RA, PA, QA);
-        wm_merge_row(F, true, RB, PB, QB, RA, PA, QA);
-        wm_merge_row(BE, false, RB, PB, QB, RA, PA, QA);
-        E = BE;
-    }
-}
-
-// Partial elimination over wave-blocks w = 0..nw-1 of one block whose outer
-// neighbours are known (x before = U, x after = V): writes u_w = x of the row
-// before wave-block w and v_w = x of the row after it.  blk is overwritten.
-template <typename T>
-__device__ __forceinline__ void chain_with_ends(T (*blk)[6], T (*uv)[2], int nw, T U, T V) {
-    T rho = U, sig = 0;                   // x_{E_{w-1}} = rho - sig x_{F_w}
-    for (int w = 0; w < nw; ++w) {
-        const T rF = blk[w][0], pF = blk[w][1], qF = blk[w][2];
-        const T rE = blk[w][3], pE = blk[w][4], qE = blk[w][5];
-        const T inv = rcp(T(1) - pF * sig);
-        const T rhoF = (rF - pF * rho) * inv;
-        const T sigF = qF * inv;
-        const T rhoE = rE - pE * (rho - sig * rhoF);
-        const T sigE = qE + pE * sig * sigF;
-        blk[w][0] = rhoF; blk[w][1] = sigF; blk[w][2] = rhoE; blk[w][3] = sigE;
-        rho = rhoE;
-        sig = sigE;
-    }
-    T xFn = V;
-    uv[0][0] = U;
-    for (int w = nw - 1; w >= 0; --w) {
-        const T xE = blk[w][2] - blk[w][3] * xFn;
-        const T xF = blk[w][0] - blk[w][1] * xFn;
-        uv[w][1] = xFn;
-        if (w + 1 < nw) uv[w + 1][0] = xE;
-        xFn = xF;
-    }
-}
-
-// block_chain (below) one block at a time: the form the FP64 kernels take.
-template <typename T>
-__device__ __forceinline__ void block_chain_serial(T (*blk)[6], int K, int j, T &U, T &V) {
-    T rho = 0, sig = 0;                   // x_{E_{k-1}} = rho - sig x_{F_k}
-    for (int k = 0; k < K; ++k) {
-        const T rF = blk[k][0], pF = blk[k][1], qF = blk[k][2];
-        const T rE = blk[k][3], pE = blk[k][4], qE = blk[k][5];
-        const T inv = rcp(T(1) - pF * sig);
-        const T rhoF = (rF - pF * rho) * inv;
-        const T sigF = qF * inv;
-        blk[k][0] = rhoF; blk[k][1] = sigF;
-        blk[k][2] = rho; blk[k][3] = sig;              // relation of x_{E_{k-1}} to x_{F_k}
-        rho = rE - pE * (rho - sig * rhoF);
-        sig = qE + pE * sig * sigF;
-    }
-    T xFn = 0;                            // x_{F_{k+1}}
-    U = 0;
-    V = 0;
-    for (int k = K - 1; k >= j; --k) {
-        if (k == j) V = xFn;
-        const T xF = blk[k][0] - blk[k][1] * xFn;
-        if (k == j) U = blk[k][2] - blk[k][3] * xF;
-        xFn = xF;
-    }
-}
-
-// Partial elimination over the K block forms of one system (blk[k][0..5]: first
-// row r, p, q then last row r, p, q; the system's ends are zero): returns
-// U = x before block j and V = x after it.  blk is overwritten.
-template <typename T>
-__device__ __forceinline__ void block_chain(T (*blk)[6], int K, int j, T &U, T &V) {
-    if constexpr (sizeof(T) != 4) {
-        block_chain_serial<T>(blk, K, j, U, V);
-        return;
-    }
-    // FP32: both sweeps take the forms of four blocks from LDS before using the
-    // first, so that the LDS latency is paid once per four steps of the dependent
-    // chain (FP32 131,072 x 128 contiguous 0.088 -> 0.083 ms).  The FP64 kernels
-    // have no registers to spare and keep the step-by-step form.
-    constexpr int U4 = 4;
-    T rho = 0, sig = 0;                   // x_{E_{k-1}} = rho - sig x_{F_k}
-    auto fwd = [&](T (&f)[6], T *out) {
-        const T inv = rcp(T(1) - f[1] * sig);
-        const T rhoF = (f[0] - f[1] * rho) * inv;
-        const T sigF = f[2] * inv;
-        out[0] = rhoF; out[1] = sigF;
-        out[2] = rho; out[3] = sig;                    // relation of x_{E_{k-1}} to x_{F_k}
-        rho = f[3] - f[4] * (rho - sig * rhoF);
-        sig = f[5] + f[4] * sig * sigF;
+// x of the rows before (ends[0][s]) and after (ends[1][s]) block j of every system, from the
+// K staged block forms.  Lane s eliminates blocks 0 .. j-1, lane S + s blocks K-1 .. j+1 (the
+// same recurrence with first and last rows, p and q exchanged): x at the near end of what
+// is eliminated is rho - sig * (x at the facing end of the next block).  Block j's own form
+// closes the two relations.
+template <typename T, int S>
+__device__ __forceinline__ void coop_block_ends(const T *k6, int K, int j, int tid, T (*ends)[S]) {
+    static_assert(2 * S <= 64, "both sides of a system in one wave");
+    if (tid >= 2 * S) return;
+    const int s = tid % S;
+    const bool right = tid >= S;
+    const int steps = right ? K - 1 - j : j;
+    const int far = right ? 3 : 0, near = 3 - far, po = right ? 2 : 1, qo = 3 - po;
+    const T *f = k6 + (right ? (K - 1) * 6 * S : 0) + s;
+    const int df = right ? -6 * S : 6 * S;
+    T rho = 0, sig = 0;
+    T a[6], b[6];
+    auto load = [&](T (&v)[6], const T *g) {
+        v[0] = g[far * S]; v[1] = g[(far + po) * S]; v[2] = g[(far + qo) * S];
+        v[3] = g[near * S]; v[4] = g[(near + po) * S]; v[5] = g[(near + qo) * S];
     };
-    int k = 0;
-    for (; k + U4 <= K; k += U4) {
-        T f[U4][6];
+    if (steps > 0) load(a, f);
+    for (int t = 0; t < steps; ++t) {
+        f += df;
+        if (t + 1 < steps) load(b, f);
+        const T inv = rcp(T(1) - a[1] * sig);
+        const T rhoF = (a[0] - a[1] * rho) * inv, sigF = a[2] * inv;
+        rho = a[3] - a[4] * (rho - sig * rhoF);
+        sig = a[5] + a[4] * sig * sigF;
 #pragma unroll
-        for (int i = 0; i < U4; ++i)
-#pragma unroll
-            for (int q = 0; q < 6; ++q) f[i][q] = blk[k + i][q];
-#pragma unroll
-        for (int i = 0; i < U4; ++i) fwd(f[i], blk[k + i]);
+        for (int q = 0; q < 6; ++q) a[q] = b[q];
     }
-    for (; k < K; ++k) {
-        T f[6];
-#pragma unroll
-        for (int q = 0; q < 6; ++q) f[q] = blk[k][q];
-        fwd(f, blk[k]);
-    }
-    T xFn = 0;                            // x_{F_{k+1}}
-    U = 0;
-    V = 0;
-    auto bwd = [&](int kk, T rhoF, T sigF, T rin, T sin) {
-        if (kk == j) V = xFn;
-        const T xF = rhoF - sigF * xFn;
-        if (kk == j) U = rin - sin * xF;
-        xFn = xF;
-    };
-    k = K - 1;
-    for (; k - (U4 - 1) >= j; k -= U4) {
-        T b[U4][4];
-#pragma unroll
-        for (int i = 0; i < U4; ++i)
-#pragma unroll
-            for (int q = 0; q < 4; ++q) b[i][q] = blk[k - i][q];
-#pragma unroll
-        for (int i = 0; i < U4; ++i) bwd(k - i, b[i][0], b[i][1], b[i][2], b[i][3]);
-    }
-    for (; k >= j; --k) bwd(k, blk[k][0], blk[k][1], blk[k][2], blk[k][3]);
+    const T rhoR = lane_read(rho, S + s), sigR = lane_read(sig, S + s);
+    if (right) return;
+    const T *o = k6 + j * 6 * S + s;
+    const T pF = o[S], qF = o[2 * S], pE = o[4 * S], qE = o[5 * S];
+    const T bF = o[0] - pF * rho - qF * rhoR, bE = o[3 * S] - pE * rho - qE * rhoR;
+    const T mFF = T(1) - pF * sig, mFE = qF * sigR, mEF = pE * sig, mEE = T(1) - qE * sigR;
+    const T inv = rcp(mFF * mEE - mFE * mEF);
+    ends[0][s] = rho - sig * ((mEE * bF + mFE * bE) * inv);
+    ends[1][s] = rhoR - sigR * ((mEF * bF + mFF * bE) * inv);
 }
+
+// Wave-blocks' forms of a task in LDS, [wave][6][S] with the waves SG apart in the banks.
+template <typename T, int NW, int S> struct CoopWaveForms {
+    static constexpr int SG = 64 / NW;             // systems whose waves one wave merges
+    static_assert(NW * SG == 64 && S % SG == 0, "a wave merges whole systems");
+    T v[NW][6 * S + SG];
+};
 
 template <typename T>
 __device__ __forceinline__ void coop_rsrc(const CoopParams<T> &p, __amdgpu_buffer_rsrc_t (&rr)[4]) {
@@ -297,144 +201,91 @@ __device__ __forceinline__ void coop_rsrc(const CoopParams<T> &p, __amdgpu_buffe
     rr[2] = make_rsrc(p.c, p.buf_bytes); rr[3] = make_rsrc(p.d, p.buf_bytes);
 }
 
-// OCC: waves per SIMD the kernel is built for (its register budget).  LINES: rows start on
-// 128-byte lines, which are read once and streamed; otherwise neighbouring groups share
-// lines and the loads stay cached.
-template <typename T, int M, int NW, int S, int KMAX, int OCC, bool LINES>
-__global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(OCC)))
-    coop_kernel(CoopParams<T> p) {
-    using Sh = TileShape<T, M, NW, S, true, false, false, false, false, true, true>;
-    constexpr int SW = 64 / S;               // segments of a system per wave
-    constexpr int R = SW * NW * M;           // rows per block
-    constexpr int NQ = M * (int)sizeof(T) / 16;
-    static_assert((S * (int)sizeof(T)) % 16 == 0, "blocks move whole 16-byte chunks");
-    static_assert(KMAX <= kCoopFlagStride, "a group's flags fit its flag words");
-    __shared__ u32x4 xbuf[NW][64 * M * (int)sizeof(T) / 16];
-    __shared__ T sh_blk[S][NW][6];
-    __shared__ T sh_uv[S][NW][2];
-    __shared__ T sh_k[S][KMAX][6];
-    __shared__ int s_ok;
-
-    const int K = p.K;
-    const int P = (int)gridDim.x;
-    const int ntask = p.ngroups * K;
-    const int64_t n = p.n;
-    for (int task = (int)blockIdx.x; task < ntask; task += P) {
-        // an opaque copy: lane-dependent addresses and masks stay inside the task loop
-        // instead of occupying registers across it
-        int tid = threadIdx.x;
-        asm volatile("" : "+v"(tid));
-        const int lane = tid & 63, wave = tid >> 6;
-        const int sl = lane % S;             // system of the lane inside the group
-        const int kw = lane / S;             // segment inside the wave-block
-        const int ws = wave;                 // wave-block inside the block
-        const int64_t wrow = (int64_t)ws * SW * M;   // first row of the wave-block, in the block
-        int gi, j;
-        coop_task(p, task, gi, j);
-        const int64_t brow = (int64_t)j * R;               // first row of the block
-        const int64_t row0 = brow + wrow + (int64_t)kw * M;   // first row of the lane
-        __amdgpu_buffer_rsrc_t rr[4];
-        coop_rsrc(p, rr);
-        T rows[4][M];
-        il_block_load<T, M, SW, S, LINES, true>(rr, brow + wrow, p.rstride, (int64_t)gi * S, n, lane,
-                                               sl, kw, xbuf[wave], rows);
-        // lane sweep; global row numbers drop a_0 and c_{n-1}
-        T al_r[Sh::NI];
-        SweepOut<T, Sh::NI> o;
-        RegLoader<T, Sh::CH, M> ld{rows};
-        lane_sweep<T, Sh>(o, ld, row0, n, [&](int q, T x) { al_r[q] = x; });
-        const T DLr = o.bL - o.cL * o.SA, ELr = o.cL * o.PI, FLr = o.dL - o.cL * o.SD;
-        const T ARr = -(o.aR * o.alp), DRr = o.bR - o.aR * o.g, FRr = o.dR - o.aR * o.del;
-        Outer<T> oL, oR;
-        segment_outer(o.aL, DLr, ELr, FLr, ARr, DRr, o.cR, FRr, oL, oR);
-        wm_wave_merges<T, SW, S>(oL, oR, lane, sl, kw, SW, false, nullptr);
-        if (kw == 0) { sh_blk[sl][ws][0] = oL.r; sh_blk[sl][ws][1] = oL.p; sh_blk[sl][ws][2] = oL.q; }
-        if (kw == SW - 1) { sh_blk[sl][ws][3] = oR.r; sh_blk[sl][ws][4] = oR.p; sh_blk[sl][ws][5] = oR.q; }
-        __syncthreads();
-
-        // publish the block's outer form for every system of the group
-        T *fg = p.forms + (int64_t)gi * K * S * 6;
-        if (tid < S) {
-            Outer<T> F, E;
-            fold_blocks<T>(sh_blk[tid], NW, F, E);
-            T *f = fg + ((int64_t)j * S + tid) * 6;
-            const T vals[6] = {F.r, F.p, F.q, E.r, E.p, E.q};
+// Publishes a task's block form.  The waves' forms (oL, oR after the merges inside each
+// wave) meet in LDS and log2(NW) merges across lanes give each wave-block's ends in terms
+// of the block's neighbours, which stay in wf for coop_finish; the first and last of them
+// are the block's form.
+template <typename T, int NW, int S>
+__device__ __forceinline__ void coop_publish(const CoopParams<T> &p, int gi, int j,
+                                             const Outer<T> &oL, const Outer<T> &oR, int tid,
+                                             CoopWaveForms<T, NW, S> &wf) {
+    constexpr int SW = 64 / S, SG = CoopWaveForms<T, NW, S>::SG;
+    const int lane = tid & 63, wave = tid >> 6, sl = lane % S, kw = lane / S;
+    T *f = wf.v[wave] + sl;
+    if (kw == 0) { f[0] = oL.r; f[S] = oL.p; f[2 * S] = oL.q; }
+    if (kw == SW - 1) { f[3 * S] = oR.r; f[4 * S] = oR.p; f[5 * S] = oR.q; }
+    __syncthreads();
+    if (tid < S * NW) {
+        const int s = wave * SG + lane % SG, w = lane / SG;
+        T *m = wf.v[w] + s;
+        Outer<T> F{m[0], m[S], m[2 * S]}, E{m[3 * S], m[4 * S], m[5 * S]};
+        wm_wave_merges<T, NW, SG>(F, E, lane, lane % SG, w, NW, false, nullptr);
+        m[0] = F.r; m[S] = F.p; m[2 * S] = F.q;
+        m[3 * S] = E.r; m[4 * S] = E.p; m[5 * S] = E.q;
+        if (w == 0 || w == NW - 1) {
+            T *out = p.forms + (((int64_t)gi * p.K + j) * 6 + (w == 0 ? 0 : 3)) * S + s;
+            const T v[3] = {w == 0 ? F.r : E.r, w == 0 ? F.p : E.p, w == 0 ? F.q : E.q};
 #pragma unroll
-            for (int q = 0; q < 6; ++q)
-                __hip_atomic_store(f + q, vals[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            // the forms are at the agent-coherent level before the barrier
-            __builtin_amdgcn_s_waitcnt(0);
+            for (int q = 0; q < 3; ++q)
+                __hip_atomic_store(out + q * S, v[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
-        __syncthreads();
-        if (tid == 0)
-            __hip_atomic_store(p.flags + kCoopFlagStride * gi + j, p.tag, __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_AGENT);
-        if (tid < 64) {
-            const int okw = coop_wait(p, gi, tid);
-            if (tid == 0) s_ok = okw;
-        }
-        __syncthreads();
-        const bool ok = s_ok != 0;
-        coop_stage_forms<T, S, NW, KMAX>(fg, K, ok, tid, sh_k);
-        __syncthreads();
-        if (tid < S) {
-            T U, V;
-            block_chain<T>(sh_k[tid], K, j, U, V);
-            chain_with_ends<T>(sh_blk[tid], sh_uv[tid], NW, U, V);
-        }
-        __syncthreads();
-        const T u = sh_uv[sl][ws][0], v = sh_uv[sl][ws][1];
-        const T xL = oL.r - oL.p * u - oL.q * v;
-        const T xR = oR.r - oR.p * u - oR.q * v;
-        T xs[M];
-        xs[0] = xL;
-        xs[M - 1] = xR;
-        T xn = xR;
-#pragma unroll
-        for (int q = M - 3; q >= 0; --q) {
-            xn = (o.de[q] - al_r[q] * xL) - o.ga[q] * xn;
-            xs[q + 1] = xn;
-        }
-        if (!ok) {
-#pragma unroll
-            for (int q = 0; q < M; ++q) xs[q] = __builtin_nan("");
-        }
-        il_block_store<T, M, SW, S, true, true>(make_rsrc(p.x, p.buf_bytes), brow + wrow, p.rstride, (int64_t)gi * S, n,
-                                                p.batch, lane, sl, kw, xbuf[wave], xs);
-        __syncthreads();                           // LDS of this task free before the next
+        // the forms are at the agent-coherent level before the barrier
+        __builtin_amdgcn_s_waitcnt(0);
     }
+    __syncthreads();
+    if (tid == 0)
+        __hip_atomic_store(p.flags + kCoopFlagStride * gi + j, p.tag, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Back-substitution of one task once its group has published: waits for the K
-// block forms of group gi, chains them to U, V of block j, chains the wave-blocks
-// (blk: this task's wave-block forms, overwritten) and stores x of the block.
+// Large LDS buffer of a task: the waves' transposition blocks while rows and x move, the
+// group's block forms in between (64 blocks' forms still leave two workgroups per CU).
+template <typename T, int M, int NW, int S, int KMAX> struct CoopBuf {
+    static constexpr int kRows = NW * 64 * M * (int)sizeof(T) / 16;
+    static constexpr int kForms = KMAX * 6 * S * (int)sizeof(T) / 16;
+    u32x4 v[kRows > kForms ? kRows : kForms];
+    __device__ __forceinline__ u32x4 *wave(int w) { return v + w * (64 * M * (int)sizeof(T) / 16); }
+    __device__ __forceinline__ T *forms() { return reinterpret_cast<T *>(v); }
+};
+template <typename T, int S> struct CoopEnds {
+    T x[2][S];      // x before and after the block
+    int ok;
+};
+
+// Back-substitution of one task once its group has published: waits for the K block forms
+// of group gi, takes x around block j from them, x around every wave-block from wf, and
+// stores x of the block.
 template <typename T, int M, int NW, int S, int KMAX, int NI>
-__device__ __forceinline__ void coop_finish(const CoopParams<T> &p, int gi, int j, T (*blk)[NW][6],
-                                            T (*sh_uv)[NW][2], T (*sh_k)[KMAX][6], int *s_ok,
-                                            u32x4 *xb, int tid, int lane, int sl, int kw, int ws,
-                                            int64_t wrow, const Outer<T> &oL, const Outer<T> &oR,
+__device__ __forceinline__ void coop_finish(const CoopParams<T> &p, int gi, int j,
+                                            const CoopWaveForms<T, NW, S> &wf,
+                                            CoopBuf<T, M, NW, S, KMAX> &buf, CoopEnds<T, S> &ends, int tid,
+                                            const Outer<T> &oL, const Outer<T> &oR,
                                             const T (&de)[NI], const T (&ga)[NI],
                                             const T (&al)[NI]) {
     constexpr int SW = 64 / S;
     constexpr int R = SW * NW * M;
-    const int K = p.K;
-    const int64_t brow = (int64_t)j * R;
-    const T *fg = p.forms + (int64_t)gi * K * S * 6;
+    const int lane = tid & 63, ws = tid >> 6, sl = lane % S, kw = lane / S;
     if (tid < 64) {
         const int ok = coop_wait(p, gi, tid);
-        if (tid == 0) *s_ok = ok;
+        if (tid == 0) ends.ok = ok;
     }
     __syncthreads();
-    const bool ok = *s_ok != 0;
-    coop_stage_forms<T, S, NW, KMAX>(fg, K, ok, tid, sh_k);
+    const bool ok = ends.ok != 0;
+    coop_stage_forms<T, S, NW>(p.forms + (int64_t)gi * p.K * 6 * S, p.K, ok, tid,
+                               buf.forms());
     __syncthreads();
-    if (tid < S) {
-        T U, V;
-        block_chain<T>(sh_k[tid], K, j, U, V);
-        chain_with_ends<T>(blk[tid], sh_uv[tid], NW, U, V);
+    coop_block_ends<T, S>(buf.forms(), p.K, j, tid, ends.x);
+    __syncthreads();
+    const T U = ends.x[0][sl], V = ends.x[1][sl];
+    T u = U, v = V;
+    if (ws > 0) {
+        const T *f = wf.v[ws - 1] + 3 * S + sl;
+        u = f[0] - f[S] * U - f[2 * S] * V;
     }
-    __syncthreads();
-    const T u = sh_uv[sl][ws][0], v = sh_uv[sl][ws][1];
+    if (ws < NW - 1) {
+        const T *f = wf.v[ws + 1] + sl;
+        v = f[0] - f[S] * U - f[2 * S] * V;
+    }
     const T xL = oL.r - oL.p * u - oL.q * v;
     const T xR = oR.r - oR.p * u - oR.q * v;
     T xs[M];
@@ -450,9 +301,66 @@ __device__ __forceinline__ void coop_finish(const CoopParams<T> &p, int gi, int 
 #pragma unroll
         for (int q = 0; q < M; ++q) xs[q] = __builtin_nan("");
     }
-    il_block_store<T, M, SW, S, true, true>(make_rsrc(p.x, p.buf_bytes), brow + wrow, p.rstride, (int64_t)gi * S, p.n,
-                                             p.batch, lane, sl, kw, xb, xs);
+    il_block_store<T, M, SW, S, true, true>(make_rsrc(p.x, p.buf_bytes),
+                                            (int64_t)j * R + (int64_t)ws * SW * M, p.rstride,
+                                            (int64_t)gi * S, p.n, p.batch, lane, sl, kw, buf.wave(ws), xs);
     __syncthreads();                           // LDS of this task free
+}
+
+// Sweep of the lane's M rows (row0 = its first) and the merges inside the wave: the lane's
+// ends in outer form relative to the wave-block's neighbours.
+template <typename T, class Sh, int M, int S>
+__device__ __forceinline__ void coop_reduce(const T (&rows)[4][M], int64_t row0, int64_t n, int lane,
+                                            SweepOut<T, Sh::NI> &o, T (&al)[Sh::NI], Outer<T> &oL,
+                                            Outer<T> &oR) {
+    RegLoader<T, Sh::CH, M> ld{rows};
+    lane_sweep<T, Sh>(o, ld, row0, n, [&](int q, T x) { al[q] = x; });   // drops a_0 and c_{n-1}
+    const T DLr = o.bL - o.cL * o.SA, ELr = o.cL * o.PI, FLr = o.dL - o.cL * o.SD;
+    const T ARr = -(o.aR * o.alp), DRr = o.bR - o.aR * o.g, FRr = o.dR - o.aR * o.del;
+    segment_outer(o.aL, DLr, ELr, FLr, ARr, DRr, o.cR, FRr, oL, oR);
+    wm_wave_merges<T, 64 / S, S>(oL, oR, lane, lane % S, lane / S, 64 / S, false, nullptr);
+}
+
+// OCC: waves per SIMD the kernel is built for (its register budget).  LINES: rows start on
+// 128-byte lines, which are read once and streamed; otherwise neighbouring groups share
+// lines and the loads stay cached.
+template <typename T, int M, int NW, int S, int KMAX, int OCC, bool LINES>
+__global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(OCC)))
+    coop_kernel(CoopParams<T> p) {
+    using Sh = TileShape<T, M, NW, S, true, false, false, false, false, true, true>;
+    constexpr int SW = 64 / S;               // segments of a system per wave
+    constexpr int R = SW * NW * M;           // rows per block
+    static_assert((S * (int)sizeof(T)) % 16 == 0, "blocks move whole 16-byte chunks");
+    static_assert(KMAX <= kCoopFlagStride, "a group's flags fit its flag words");
+    __shared__ CoopBuf<T, M, NW, S, KMAX> buf;
+    __shared__ CoopWaveForms<T, NW, S> wf;
+    __shared__ CoopEnds<T, S> ends;
+
+    const int P = (int)gridDim.x;
+    const int ntask = p.ngroups * p.K;
+    for (int task = (int)blockIdx.x; task < ntask; task += P) {
+        // an opaque copy: lane-dependent addresses and masks stay inside the task loop
+        // instead of occupying registers across it
+        int tid = threadIdx.x;
+        asm volatile("" : "+v"(tid));
+        const int lane = tid & 63, wave = tid >> 6;
+        const int sl = lane % S;             // system of the lane inside the group
+        const int kw = lane / S;             // segment inside the wave-block
+        int gi, j;
+        coop_task(p, task, gi, j);
+        const int64_t wrow = (int64_t)j * R + (int64_t)wave * SW * M;   // first row of the wave
+        __amdgpu_buffer_rsrc_t rr[4];
+        coop_rsrc(p, rr);
+        T rows[4][M], al[Sh::NI];
+        il_block_load<T, M, SW, S, LINES, true>(rr, wrow, p.rstride, (int64_t)gi * S, p.n, lane, sl, kw,
+                                                buf.wave(wave), rows);
+        SweepOut<T, Sh::NI> o;
+        Outer<T> oL, oR;
+        coop_reduce<T, Sh, M, S>(rows, wrow + (int64_t)kw * M, p.n, lane, o, al, oL, oR);
+        coop_publish<T, NW, S>(p, gi, j, oL, oR, tid, wf);
+        coop_finish<T, M, NW, S, KMAX, Sh::NI>(p, gi, j, wf, buf, ends, tid, oL, oR, o.de, o.ga,
+                                               al);
+    }
 }
 
 // The same solve with the wait taken one task later: a workgroup reduces and
@@ -474,86 +382,48 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int sl = lane % S;
     const int kw = lane / S;
-    const int ws = wave;
-    const int64_t wrow = (int64_t)ws * SW * M;
-    __shared__ u32x4 xbuf[NW][64 * M * (int)sizeof(T) / 16];
-    __shared__ T sh_blk[2][S][NW][6];
-    __shared__ T sh_uv[S][NW][2];
-    __shared__ T sh_k[S][KMAX][6];
-    __shared__ int s_ok;
+    const int64_t wrow = (int64_t)wave * SW * M;
+    __shared__ CoopBuf<T, M, NW, S, KMAX> buf;
+    __shared__ CoopWaveForms<T, NW, S> wf[2];
+    __shared__ CoopEnds<T, S> ends;
 
-    const int K = p.K;
     const int P = (int)gridDim.x;
-    const int ntask = p.ngroups * K;
+    const int ntask = p.ngroups * p.K;
     const int64_t n = p.n;
     int task = (int)blockIdx.x;
     u32x4 g[4][NQ];
-    if (task < ntask) {
-        int g0, j0;
-        coop_task(p, task, g0, j0);
+    auto issue = [&](int t) {
+        int gi, j;
+        coop_task(p, t, gi, j);
         __amdgpu_buffer_rsrc_t rr[4];
         coop_rsrc(p, rr);
-        il_block_issue<T, M, SW, S, true, true>(rr, (int64_t)j0 * R + wrow, p.rstride,
-                                                (int64_t)g0 * S, n, lane, g);
-    }
+        il_block_issue<T, M, SW, S, true, true>(rr, (int64_t)j * R + wrow, p.rstride, (int64_t)gi * S,
+                                                n, lane, g);
+    };
+    if (task < ntask) issue(task);
     // the pending task: published, not yet finished
     int pend = -1, par = 0;
     Outer<T> poL{}, poR{};
     T pde[NI], pga[NI], pal[NI];
+    auto finish = [&]() {
+        int gi, j;
+        coop_task(p, pend, gi, j);
+        coop_finish<T, M, NW, S, KMAX, NI>(p, gi, j, wf[par ^ 1], buf, ends, tid, poL, poR, pde,
+                                           pga, pal);
+    };
     for (; task < ntask; task += P) {
         int gi, j;
         coop_task(p, task, gi, j);
-        const int64_t brow = (int64_t)j * R;
-        const int64_t row0 = brow + wrow + (int64_t)kw * M;
-        T rows[4][M];
-        il_block_transpose<T, M, S>(g, lane, sl, kw, xbuf[wave], rows);
+        const int64_t row0 = (int64_t)j * R + wrow + (int64_t)kw * M;
+        T rows[4][M], al[NI];
+        il_block_transpose<T, M, S>(g, lane, sl, kw, buf.wave(wave), rows);
         identity_rows<T, M>(row0, n, rows);
-        T al_r[NI];
         SweepOut<T, NI> o;
-        RegLoader<T, Sh::CH, M> ld{rows};
-        lane_sweep<T, Sh>(o, ld, row0, n, [&](int q, T x) { al_r[q] = x; });
-        const T DLr = o.bL - o.cL * o.SA, ELr = o.cL * o.PI, FLr = o.dL - o.cL * o.SD;
-        const T ARr = -(o.aR * o.alp), DRr = o.bR - o.aR * o.g, FRr = o.dR - o.aR * o.del;
         Outer<T> oL, oR;
-        segment_outer(o.aL, DLr, ELr, FLr, ARr, DRr, o.cR, FRr, oL, oR);
-        wm_wave_merges<T, SW, S>(oL, oR, lane, sl, kw, SW, false, nullptr);
-        if (kw == 0) {
-            sh_blk[par][sl][ws][0] = oL.r; sh_blk[par][sl][ws][1] = oL.p; sh_blk[par][sl][ws][2] = oL.q;
-        }
-        if (kw == SW - 1) {
-            sh_blk[par][sl][ws][3] = oR.r; sh_blk[par][sl][ws][4] = oR.p; sh_blk[par][sl][ws][5] = oR.q;
-        }
-        __syncthreads();
-        T *fg = p.forms + (int64_t)gi * K * S * 6;
-        if (tid < S) {
-            Outer<T> F, E;
-            fold_blocks<T>(sh_blk[par][tid], NW, F, E);
-            T *f = fg + ((int64_t)j * S + tid) * 6;
-            const T vals[6] = {F.r, F.p, F.q, E.r, E.p, E.q};
-#pragma unroll
-            for (int q = 0; q < 6; ++q)
-                __hip_atomic_store(f + q, vals[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __builtin_amdgcn_s_waitcnt(0);
-        }
-        __syncthreads();
-        if (tid == 0)
-            __hip_atomic_store(p.flags + kCoopFlagStride * gi + j, p.tag, __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_AGENT);
-        const int next = task + P;
-        if (next < ntask) {
-            int g1, j1;
-            coop_task(p, next, g1, j1);
-            __amdgpu_buffer_rsrc_t rr[4];
-            coop_rsrc(p, rr);
-            il_block_issue<T, M, SW, S, true, true>(rr, (int64_t)j1 * R + wrow, p.rstride,
-                                                    (int64_t)g1 * S, n, lane, g);
-        }
-        if (pend >= 0) {
-            int pg, pj;
-            coop_task(p, pend, pg, pj);
-            coop_finish<T, M, NW, S, KMAX, NI>(p, pg, pj, sh_blk[par ^ 1], sh_uv, sh_k, &s_ok, xbuf[wave], tid, lane, sl, kw, ws,
-                                                   wrow, poL, poR, pde, pga, pal);
-        }
+        coop_reduce<T, Sh, M, S>(rows, row0, n, lane, o, al, oL, oR);
+        coop_publish<T, NW, S>(p, gi, j, oL, oR, tid, wf[par]);
+        if (task + P < ntask) issue(task + P);
+        if (pend >= 0) finish();
         pend = task;
         par ^= 1;
         poL = oL;
@@ -562,18 +432,11 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)
         for (int q = 0; q < NI; ++q) {
             pde[q] = o.de[q];
             pga[q] = o.ga[q];
-            pal[q] = al_r[q];
+            pal[q] = al[q];
         }
     }
-    if (pend >= 0) {
-        int pg, pj;
-        coop_task(p, pend, pg, pj);
-        coop_finish<T, M, NW, S, KMAX, NI>(p, pg, pj, sh_blk[par ^ 1], sh_uv, sh_k,
-                                               &s_ok, xbuf[wave], tid, lane, sl, kw, ws, wrow, poL,
-                                               poR, pde, pga, pal);
-    }
+    if (pend >= 0) finish();
 }
-
 
 template <typename T> struct CoopEntry {
     int M, NW, S;
