@@ -629,6 +629,11 @@ static bool coop_plan(int algo, int layout, int64_t n, int64_t batch, const Tile
     return true;
 }
 
+static bool capturing(hipStream_t st) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    return st && hipStreamIsCapturing(st, &cap) == hipSuccess && cap == hipStreamCaptureStatusActive;
+}
+
 template <typename T>
 static int coop_run(const SolvePlan<T> &pl, int layout, int64_t n, int64_t batch, int64_t sstride,
                     T *a, T *b, T *c, T *d, T *x, hipStream_t st, const FixedScratch *fx) {
@@ -659,8 +664,7 @@ static int coop_run(const SolvePlan<T> &pl, int layout, int64_t n, int64_t batch
     hipError_t err = hipSuccess;
     // a captured solve is replayed with the tag of its capture, which the words hold
     // from the second replay on: they are cleared in the graph
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (st && hipStreamIsCapturing(st, &cap) == hipSuccess && cap == hipStreamCaptureStatusActive)
+    if (capturing(st))
         err = launch_coop_clear(p.flags, (int64_t)((pl.scratch_bytes - pl.forms_bytes) / sizeof(uint64_t)), st);
     if (err == hipSuccess) err = e.launch(p, pl.grid, st);
     if (err != hipSuccess) rc = hip_fail(err, "cooperative solve launch");
@@ -817,10 +821,13 @@ static int solve_impl(int algo, int layout, int64_t n, int64_t batch, T *a, T *b
     const bool vec_ok = layout != kInterleaved && (sstride % V) == 0 && aligned16<T>(a) &&
                         aligned16<T>(b) && aligned16<T>(c) && aligned16<T>(d) && aligned16<T>(x);
     const FixedScratch *only = fx && fx->only ? fx : nullptr;
-    const SolvePlan<T> pl = make_plan<T>(algo, layout, n, batch, sstride, vec_ok,
+    SolvePlan<T> pl = make_plan<T>(algo, layout, n, batch, sstride, vec_ok,
                                          only ? only->bytes : 0);
     const int32_t bb = buffer_extent<T>(n, batch, sstride, layout);
     const bool il = layout == kInterleaved;
+    // A solve recorded into a graph allocates only where what it reports does.
+    if (pl.coop && il && pl.kind != kPlanCoop && !(fx && fx->bytes >= pl.scratch_bytes) && capturing(st))
+        pl.coop = nullptr;
     if (pl.coop) return coop_run<T>(pl, layout, n, batch, sstride, a, b, c, d, x, st, fx);
     if (x != d && (pl.kind == kPlanThomas || pl.kind == kPlanBulk || pl.kind == kPlanChunked)) {
         // these forms keep their own intermediate values in d (and c)

@@ -57,9 +57,12 @@ def _scratch_bytes(prec, algo, layout, n, batch, device_index, current_device):
 
 
 def _scratch(prec, algo, layout, n, batch, device):
-    """Scratch of a solve on the current stream, from torch's caching allocator, or None."""
+    """Scratch of a solve on the current stream, from torch's caching allocator, or None.
+    None while the stream is captured: a graph outlives the block."""
     size = _scratch_bytes(prec, algo, layout, n, batch, device.index, torch.cuda.current_device())
-    return torch.empty(size, dtype=torch.uint8, device=device) if size else None
+    if not size or torch.cuda.is_current_stream_capturing():
+        return None
+    return torch.empty(size, dtype=torch.uint8, device=device)
 
 
 def _launch(prec, algo, layout, n, batch, args, x, device):
