@@ -64,3 +64,19 @@ def test_refused():
     assert L.tridiag_solve_to(0, -1, 1, 64, 4, p, p, p, p, x, None, 0, None) == _capi.EUNSUPPORTED
     assert L.tridiag_solve_to(0, 0, 0, 64, 4, p, p, p, p, x, None, 0, None) == _capi.EUNSUPPORTED
     assert L.tridiag_solve_to(0, -1, 0, 64, 4, p, p, p, p, None, None, 0, None) == _capi.EINVAL
+
+
+@pytest.mark.parametrize("prec", [0, 1])
+@pytest.mark.parametrize("n", [256, 384, 512, 768, 1024, 1536, 2048, 3072, 4096, 8192])
+def test_exact_tiles(prec, n):
+    """Capacities of the contiguous tiles, whose exact kernels solve in place only."""
+    import torch
+    import tridiagonalsolver_amd as T
+    dt = torch.float64 if prec else torch.float32
+    announce("solve to, exact tiles", prec, n)
+    a, c, d = (torch.rand(33, n, device="cuda", dtype=dt) * 2 - 1 for _ in range(3))
+    b = a.abs() + c.abs() + 1
+    ref = T.solve(a, b, c, d.clone())
+    keep = d.clone()
+    x = T.tridiagonal_solve(a, b, c, d)
+    assert torch.equal(x, ref) and torch.equal(d, keep)

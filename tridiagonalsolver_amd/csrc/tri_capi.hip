@@ -829,7 +829,14 @@ static int solve_impl(int algo, int layout, int64_t n, int64_t batch, T *a, T *b
     if (pl.coop && il && pl.kind != kPlanCoop && !(fx && fx->bytes >= pl.scratch_bytes) && capturing(st))
         pl.coop = nullptr;
     if (pl.coop) return coop_run<T>(pl, layout, n, batch, sstride, a, b, c, d, x, st, fx);
-    if (x != d && (pl.kind == kPlanThomas || pl.kind == kPlanBulk || pl.kind == kPlanChunked)) {
+    // exact contiguous whole-chunk tiles solve in place only: their padded twins store to x
+    if (x != d && pl.kind == kPlanTile && pl.tile->XP && !il && !pl.tile->PAD) {
+        const TileEntry<T> &t = *pl.tile;
+        const TileEntry<T> *twin = find_tile<T>(t.M, t.NW, t.S, false, t.VEC, t.ALDS, true, false, t.NT, true);
+        if (twin && twin->XP) pl.tile = twin;
+    }
+    if (x != d && (pl.kind == kPlanThomas || pl.kind == kPlanBulk || pl.kind == kPlanChunked ||
+                   (pl.kind == kPlanTile && pl.tile->XP && !il && !pl.tile->PAD))) {
         // these forms keep their own intermediate values in d (and c)
         const LayoutMove<T> mv{{d}, {x}, il ? n : batch, il ? batch : n, il ? batch : n,
                                il ? batch : n, 0};
