@@ -41,8 +41,7 @@ __device__ __forceinline__ void adj_issue(__amdgpu_buffer_rsrc_t r, int64_t wrow
                                           u32x4 (&g)[M * (int)sizeof(T) / 16]) {
 #pragma unroll
     for (int q = 0; q < M * (int)sizeof(T) / 16; ++q)
-        g[q] = __builtin_amdgcn_raw_buffer_load_b128(r, (int)(wrow * (int64_t)sizeof(T)) + lane * 16,
-                                                     q * 1024, cpol<true>());
+        g[q] = load16<true>(r, (int)(wrow * (int64_t)sizeof(T)) + lane * 16 + q * 1024);
 }
 
 // Hands every lane its M rows of the chunks in g through the wave's LDS block `xb`, with

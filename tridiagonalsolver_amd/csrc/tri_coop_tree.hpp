@@ -38,8 +38,7 @@ __device__ __forceinline__ void contig_block_issue(const __amdgpu_buffer_rsrc_t 
     for (int q = 0; q < NQ; ++q)
 #pragma unroll
         for (int k = 0; k < 4; ++k)
-            g[k][q] = __builtin_amdgcn_raw_buffer_load_b128(
-                rr[k], (int)(wrow * (int64_t)sizeof(T)) + lane * 16, q * 1024, cpol<NT>());
+            g[k][q] = load16<NT>(rr[k], (int)(wrow * (int64_t)sizeof(T)) + lane * 16 + q * 1024);
 }
 
 template <typename T, int M>

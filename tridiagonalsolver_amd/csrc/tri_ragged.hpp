@@ -85,7 +85,7 @@ __device__ __forceinline__ void ragged_item(const RaggedParams<T> &p, const int3
         for (int k = 0; k < 4; ++k)
 #pragma unroll
             for (int q = 0; q < NQ; ++q)
-                g[k][q] = __builtin_amdgcn_raw_buffer_load_b128(rr[k], vo, q * 1024, cpol<true>());
+                g[k][q] = load16<true>(rr[k], vo + q * 1024);
         T rows[4][M];
 #pragma unroll
         for (int k = 0; k < 4; ++k) {

@@ -51,7 +51,7 @@ __global__ void __launch_bounds__(256) short_kernel(const T *a, const T *b, cons
     for (int k = 0; k < 4; ++k)
 #pragma unroll
         for (int q = 0; q < NQ; ++q)
-            g[k][q] = __builtin_amdgcn_raw_buffer_load_b128(rr[k], lane * 16, q * 1024, cpol<true>());
+            g[k][q] = load16<true>(rr[k], lane * 16 + q * 1024);
     const int row0 = (lane % P) * M;                  // the lane's first row
     const int e0 = (lane / P) * nr + row0;            // its element of the block
     T rows[4][M];

@@ -134,6 +134,18 @@ __device__ __forceinline__ void store16(u32x4 t, __amdgpu_buffer_rsrc_t r, int v
     __builtin_amdgcn_raw_buffer_store_b128(t, r, vo, 0, cpol<NT>());
 }
 
+// Loads a 16-byte chunk at byte offset vo of a buffer whose end it may straddle or pass.  The
+// whole offset goes through the address register and the instruction's immediate, which
+// the bounds check counts (dwords past the end read as zero).  The builtin's definition
+// leaves the scalar offset out of the check; gfx950 does count it (a chunk of a buffer of
+// 64 bytes read at a scalar offset of 1024 is zero), but nothing here rests on that.  Both
+// ways take the same time (FP64 1001 x 3001 22.7 / 22.8 us, 2^20 x 16 179.7 / 180.1, fused
+// FP32 512 x 8192 31.0 / 31.0).
+template <bool NT>
+__device__ __forceinline__ u32x4 load16(__amdgpu_buffer_rsrc_t r, int vo) {
+    return __builtin_amdgcn_raw_buffer_load_b128(r, vo, 0, cpol<NT>());
+}
+
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void *p, int32_t bytes) {
     // raw buffer (stride 0); word 3 = 0x00020000 selects 32-bit data format on gfx9
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), (short)0, bytes, 0x00020000);
@@ -748,7 +760,9 @@ __global__ void __launch_bounds__(64 * NW)
             for (int k = 0; k < 4; ++k)
 #pragma unroll
                 for (int q = 0; q < NQ; ++q)
-                    g[k][q] = __builtin_amdgcn_raw_buffer_load_b128(rr[k], wvo, q * 1024, cpol<NT>());
+                    g[k][q] = PAD ? load16<NT>(rr[k], wvo + q * 1024)
+                                  : __builtin_amdgcn_raw_buffer_load_b128(rr[k], wvo, q * 1024,
+                                                                          cpol<NT>());
             T rows[4][M];
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
