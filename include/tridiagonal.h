@@ -121,7 +121,12 @@ void CR_reg16_single(float *a_gbl, float *b_gbl, float *c_gbl, float *d_gbl, int
  * 6 reg PCR-half-pThomas, 7 shmem WM-pGE, 8 shmem WM-half-pGE, 9 reg WM-pGE,
  * 10 reg WM-half-pGE, 11 reg-4 CR, 12 reg-8 CR, 13 reg-16 CR; FP32 only:
  * 14 BPLG WM, 15 BPLG LF, 16 BPLG CR, 17 BPLG PCR (packed layout).
- * TRIDIAG_ALGO_AUTO picks the fastest kernel for (precision, layout, n). */
+ * TRIDIAG_ALGO_AUTO picks the fastest kernel for (precision, layout, n).
+ * No algorithm pivots.  The automatic choice solves layouts 0 and 2 of up to 32 (single)
+ * or 16 (double) rows by the Thomas recurrence, which needs its own pivots to be
+ * nonzero.  Longer systems are eliminated segment by segment, each from its second row,
+ * as by ids 2-17: that also needs nonzero pivots within the segments, whose
+ * places depend on (precision, layout, n).  Diagonally dominant systems have both. */
 #define TRIDIAG_ALGO_AUTO (-1)
 
 int tridiag_algo_count(int precision);

@@ -708,16 +708,19 @@ static int interleaved_via_contiguous(int algo, int64_t n, int64_t batch, T *a, 
     return rc;
 }
 
-// Largest n for which the automatic choice takes the one-system-per-lane Thomas
-// kernel instead of an on-chip tile ($TRIDIAG_LANE_ROWS overrides).
-template <typename T> static int64_t lane_auto_rows(int layout) {
+// Rows up to which $TRIDIAG_LANE_ROWS asks for the one-system-per-lane kernel; -1: not set.
+static int64_t lane_rows_asked() {
     static const int64_t env = [] {
         const char *e = getenv("TRIDIAG_LANE_ROWS");
-        return e ? (int64_t)atoll(e) : (int64_t)-1;
+        return e ? std::max<int64_t>(-1, atoll(e)) : (int64_t)-1;
     }();
-    if (env >= 0) return env;
-    (void)layout;
-    return lane_thomas_max_rows(sizeof(T) == 4 ? TRIDIAG_SINGLE : TRIDIAG_DOUBLE);
+    return env;
+}
+// Largest n that the automatic choice solves by the Thomas recurrence (one system per lane,
+// or the short kernel's form of it) rather than by segments ($TRIDIAG_LANE_ROWS overrides).
+template <typename T> static int64_t lane_auto_rows() {
+    const int64_t most = lane_thomas_max_rows(sizeof(T) == 4 ? TRIDIAG_SINGLE : TRIDIAG_DOUBLE);
+    return lane_rows_asked() >= 0 ? std::min(lane_rows_asked(), most) : most;
 }
 
 // The path solve_impl takes for one batch below 2 GiB per array.  algo may be
@@ -744,7 +747,7 @@ static SolvePlan<T> make_plan(int algo, int layout, int64_t n, int64_t batch, in
     // short systems: one system per lane in registers (Thomas), for the Thomas id and
     // for the automatic choice up to lane_auto_rows()
     if (bb != 0 && n <= lane_thomas_max_rows(prec) && (il || layout == kContiguous) &&
-        (algo == kThomas || (algo == TRIDIAG_ALGO_AUTO && n <= lane_auto_rows<T>(layout)))) {
+        (algo == kThomas || (algo == TRIDIAG_ALGO_AUTO && n <= lane_auto_rows<T>()))) {
         pl.kind = kPlanLane;
         return pl;
     }
@@ -856,12 +859,12 @@ static int solve_impl(int algo, int layout, int64_t n, int64_t batch, T *a, T *b
         return e == hipSuccess ? TRIDIAG_OK : hip_fail(e, "lane Thomas launch");
     }
     case kPlanShort: {
+        const bool thomas = n <= lane_auto_rows<T>();
         const hipError_t e = (sizeof(T) == 4)
             ? launch_short_f32((const float *)a, (const float *)b, (const float *)c,
-                               (const float *)d, (float *)x, n,
-                               batch, st)
+                               (const float *)d, (float *)x, n, batch, thomas, st)
             : launch_short_f64((const double *)a, (const double *)b, (const double *)c,
-                               (const double *)d, (double *)x, n, batch, st);
+                               (const double *)d, (double *)x, n, batch, thomas, st);
         return e == hipSuccess ? TRIDIAG_OK : hip_fail(e, "short-system launch");
     }
     case kPlanThomas: {

@@ -108,12 +108,13 @@ hipError_t launch_lane_thomas_f64(const double *a, const double *b, const double
                                   double *x, int64_t n, int64_t batch, int64_t sstride, int64_t rstride,
                                   bool il, int32_t bb, hipStream_t st);
 // Short contiguous systems (stride n, n <= kShortMaxRows), several per wave
-// (tri_short.hip); hipErrorInvalidValue beyond.
+// (tri_short.hip); hipErrorInvalidValue beyond.  thomas: by the Thomas recurrence
+// (n <= lane_thomas_max_rows()).
 constexpr int kShortMaxRows = 192;
 hipError_t launch_short_f32(const float *a, const float *b, const float *c, const float *d,
-                            float *x, int64_t n, int64_t batch, hipStream_t st);
+                            float *x, int64_t n, int64_t batch, bool thomas, hipStream_t st);
 hipError_t launch_short_f64(const double *a, const double *b, const double *c, const double *d,
-                            double *x, int64_t n, int64_t batch, hipStream_t st);
+                            double *x, int64_t n, int64_t batch, bool thomas, hipStream_t st);
 // Layout conversion of up to four coefficient arrays: each source is a rows x cols
 // matrix with row pitch ld_src, copied (transpose = false) or transposed into a
 // destination with row pitch ld_dst.  col_tiles is filled by the launcher.

@@ -9,6 +9,13 @@
 // rounds; the merged block is the system, so x of each segment's ends is its r.  No
 // workgroup barrier, no chain over wave blocks.
 //
+// Up to the rows that one lane holds (32 FP32, 16 FP64) the systems are solved by the Thomas
+// recurrence across their lanes instead (thomas_rows), operation by operation as the lane
+// kernel does: the segments' elimination starts at their second row, so it fails or loses
+// digits where a diagonal entry there is zero or small, which the Thomas pivots need not be.
+// Segments / Thomas at 2^22 unknowns, back to back (us): FP32 9 rows 12.7 / 12.7, 16 rows 14.3 /
+// 14.6, 28 rows 13.7 / 14.1; FP64 9 rows 26.3 / 26.4, 16 rows 27.2 / 27.8.
+//
 // What bounds it: memory, once the lanes hold rows.  The one-workgroup tiles give a
 // system at least a whole wave, so that below 64 rows per 2-row segment most lanes
 // held padding, and read their rows one element at a time.  M is odd: a lane's rows
@@ -27,7 +34,51 @@ template <typename T, int M> struct ShortShape {
     static constexpr int CH = M, NC = 1, NBUF = 1;   // rows are in registers already
 };
 
+// x of the lane's rows (the first is the system's row row0 of nr; identity rows past it) by the
+// Thomas recurrence over the P lanes of every system.  A lane's sweep starts from its
+// neighbour's last row; all lanes sweep in every round, and after round t the first t + 1
+// lanes of a system hold their final rows (P <= 4: what the others compute costs less than
+// branches around it).
 template <typename T, int M, int P>
+__device__ __forceinline__ void thomas_rows(const T (&rows)[4][M], int row0, int nr, int lane,
+                                            T (&xs)[M]) {
+    const bool first = lane % P == 0, last = lane % P == P - 1;
+    T cq[M], dq[M];
+#pragma unroll
+    for (int t = 0; t < P; ++t) {
+        T cp = 0, dp = 0;
+        if (t > 0) {
+            cp = lane_read(cq[M - 1], lane - 1);
+            dp = lane_read(dq[M - 1], lane - 1);
+            if (first) { cp = 0; dp = 0; }
+        }
+#pragma unroll
+        for (int j = 0; j < M; ++j) {
+            const T aj = (row0 + j == 0) ? T(0) : rows[0][j];        // a_0 is not part of A
+            const T cj = (row0 + j == nr - 1) ? T(0) : rows[2][j];   // nor is c_{n-1}
+            const T k = rcp(rows[1][j] - aj * cp);
+            cp = cj * k;
+            dp = (rows[3][j] - aj * dp) * k;
+            cq[j] = cp;
+            dq[j] = dp;
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < P; ++t) {
+        T xn = 0;
+        if (t > 0) {
+            xn = lane_read(xs[0], lane + 1);
+            if (last) xn = 0;
+        }
+#pragma unroll
+        for (int j = M - 1; j >= 0; --j) {
+            xn = dq[j] - cq[j] * xn;
+            xs[j] = xn;
+        }
+    }
+}
+
+template <typename T, int M, int P, bool THOMAS>
 __global__ void __launch_bounds__(256) short_kernel(const T *a, const T *b, const T *c,
                                                     const T *d, T *x, int64_t n, int64_t batch) {
     using Sh = ShortShape<T, M>;
@@ -71,24 +122,33 @@ __global__ void __launch_bounds__(256) short_kernel(const T *a, const T *b, cons
             rows[k][j] = (row0 + j < nr) ? v : T(k == 1 ? 1 : 0);
         }
     }
-    T al[Sh::NI];
-    SweepOut<T, Sh::NI> o;
-    RegLoader<T, M, M> ld{rows};
-    lane_sweep<T, Sh>(o, ld, row0, n, [&](int j, T v) { al[j] = v; });
-    const T DLr = o.bL - o.cL * o.SA, ELr = o.cL * o.PI, FLr = o.dL - o.cL * o.SD;
-    const T ARr = -(o.aR * o.alp), DRr = o.bR - o.aR * o.g, FRr = o.dR - o.aR * o.del;
-    Outer<T> oL, oR;
-    segment_outer(o.aL, DLr, ELr, FLr, ARr, DRr, o.cR, FRr, oL, oR);
-    wm_wave_merges<T, P, 1>(oL, oR, lane, 0, lane, P, false, nullptr);
-    T xn = oR.r;
-    wave_lds_sync();
-    if (row0 + M - 1 < nr) tb[e0 + M - 1] = xn;
+    if constexpr (THOMAS) {
+        T xs[M];
+        thomas_rows<T, M, P>(rows, row0, nr, lane, xs);
+        wave_lds_sync();
 #pragma unroll
-    for (int j = M - 3; j >= 0; --j) {
-        xn = (o.de[j] - al[j] * oL.r) - o.ga[j] * xn;
-        if (row0 + j + 1 < nr) tb[e0 + j + 1] = xn;
+        for (int j = 0; j < M; ++j)
+            if (row0 + j < nr) tb[e0 + j] = xs[j];
+    } else {
+        T al[Sh::NI];
+        SweepOut<T, Sh::NI> o;
+        RegLoader<T, M, M> ld{rows};
+        lane_sweep<T, Sh>(o, ld, row0, n, [&](int j, T v) { al[j] = v; });
+        const T DLr = o.bL - o.cL * o.SA, ELr = o.cL * o.PI, FLr = o.dL - o.cL * o.SD;
+        const T ARr = -(o.aR * o.alp), DRr = o.bR - o.aR * o.g, FRr = o.dR - o.aR * o.del;
+        Outer<T> oL, oR;
+        segment_outer(o.aL, DLr, ELr, FLr, ARr, DRr, o.cR, FRr, oL, oR);
+        wm_wave_merges<T, P, 1>(oL, oR, lane, 0, lane, P, false, nullptr);
+        T xn = oR.r;
+        wave_lds_sync();
+        if (row0 + M - 1 < nr) tb[e0 + M - 1] = xn;
+#pragma unroll
+        for (int j = M - 3; j >= 0; --j) {
+            xn = (o.de[j] - al[j] * oL.r) - o.ga[j] * xn;
+            if (row0 + j + 1 < nr) tb[e0 + j + 1] = xn;
+        }
+        if (row0 < nr) tb[e0] = oL.r;
     }
-    if (row0 < nr) tb[e0] = oL.r;
     wave_lds_sync();
 #pragma unroll
     for (int q = 0; q < NQ; ++q)
@@ -96,14 +156,14 @@ __global__ void __launch_bounds__(256) short_kernel(const T *a, const T *b, cons
             store16<true>(xb[q * 64 + lane], make_rsrc(x + base, nb), lane * 16 + q * 1024);
 }
 
-template <typename T, int M, int P>
+template <typename T, int M, int P, bool THOMAS>
 static hipError_t launch_short_shape(const T *a, const T *b, const T *c, const T *d, T *x,
                                      int64_t n, int64_t batch, hipStream_t st) {
     constexpr int G = 64 / P;
     const int64_t blocks = (batch + 4 * G - 1) / (4 * G);
     if (n > P * M || blocks > 0x7fffffff) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((short_kernel<T, M, P>), dim3((unsigned)blocks), dim3(256), 0, st, a, b, c,
-                       d, x, n, batch);
+    hipLaunchKernelGGL((short_kernel<T, M, P, THOMAS>), dim3((unsigned)blocks), dim3(256), 0, st, a,
+                       b, c, d, x, n, batch);
     return hipGetLastError();
 }
 
@@ -113,7 +173,7 @@ template <typename T> struct ShortEntry {
     hipError_t (*launch)(const T *, const T *, const T *, const T *, T *, int64_t, int64_t,
                          hipStream_t);
 };
-#define TRI_SHORT(T, M, P) {M, P, &launch_short_shape<T, M, P>}
+#define TRI_SHORT(T, M, P) {M, P, &launch_short_shape<T, M, P, false>}
 #define TRI_SHORT_TABLE(T) \
     TRI_SHORT(T, 5, 2), TRI_SHORT(T, 7, 2), TRI_SHORT(T, 5, 4), \
     TRI_SHORT(T, 7, 4), TRI_SHORT(T, 9, 4), TRI_SHORT(T, 5, 8), TRI_SHORT(T, 7, 8), \
@@ -123,6 +183,14 @@ static const ShortEntry<float> kShortF32[] = {TRI_SHORT_TABLE(float)};
 static const ShortEntry<double> kShortF64[] = {TRI_SHORT_TABLE(double)};
 #undef TRI_SHORT_TABLE
 #undef TRI_SHORT
+// By the Thomas recurrence: up to the rows of the lane kernel.
+#define TRI_SHORT_THOMAS(T, M, P) {M, P, &launch_short_shape<T, M, P, true>}
+static const ShortEntry<float> kThomasF32[] = {
+    TRI_SHORT_THOMAS(float, 5, 2), TRI_SHORT_THOMAS(float, 7, 2), TRI_SHORT_THOMAS(float, 5, 4),
+    TRI_SHORT_THOMAS(float, 7, 4), TRI_SHORT_THOMAS(float, 9, 4)};
+static const ShortEntry<double> kThomasF64[] = {
+    TRI_SHORT_THOMAS(double, 5, 2), TRI_SHORT_THOMAS(double, 7, 2), TRI_SHORT_THOMAS(double, 5, 4)};
+#undef TRI_SHORT_THOMAS
 
 template <typename T, int N>
 static hipError_t launch_short(const ShortEntry<T> (&tab)[N], const T *a, const T *b, const T *c,
@@ -134,12 +202,14 @@ static hipError_t launch_short(const ShortEntry<T> (&tab)[N], const T *a, const 
 }
 
 hipError_t launch_short_f32(const float *a, const float *b, const float *c, const float *d, float *x,
-                            int64_t n, int64_t batch, hipStream_t st) {
-    return launch_short(kShortF32, a, b, c, d, x, n, batch, st);
+                            int64_t n, int64_t batch, bool thomas, hipStream_t st) {
+    return thomas ? launch_short(kThomasF32, a, b, c, d, x, n, batch, st)
+                  : launch_short(kShortF32, a, b, c, d, x, n, batch, st);
 }
 hipError_t launch_short_f64(const double *a, const double *b, const double *c, const double *d,
-                            double *x, int64_t n, int64_t batch, hipStream_t st) {
-    return launch_short(kShortF64, a, b, c, d, x, n, batch, st);
+                            double *x, int64_t n, int64_t batch, bool thomas, hipStream_t st) {
+    return thomas ? launch_short(kThomasF64, a, b, c, d, x, n, batch, st)
+                  : launch_short(kShortF64, a, b, c, d, x, n, batch, st);
 }
 
 }  // namespace tri
