@@ -740,7 +740,7 @@ static SolvePlan<T> make_plan(int algo, int layout, int64_t n, int64_t batch, in
     // 28.9; 200 rows FP32 16.5 either way, FP64 29.5 / 30.2).  Up to 64 systems of 16
     // rows are one wave of the lane kernel and keep it.
     if (algo == TRIDIAG_ALGO_AUTO && layout == kContiguous && n > 8 && n <= kShortMaxRows &&
-        (n > 16 || batch > 64)) {
+        (n > 16 || batch > 64) && n > lane_rows_asked()) {
         pl.kind = kPlanShort;
         return pl;
     }
