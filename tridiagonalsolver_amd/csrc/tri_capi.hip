@@ -422,7 +422,7 @@ template <typename T> static bool il_rows_on_lines(int64_t batch) {
 // Polls of a cooperative wait before it gives up ($TRIDIAG_COOP_SPIN).
 static int32_t coop_spin_limit() {
     static const int32_t v = (int32_t)std::max<int64_t>(0, std::min<int64_t>(
-        env_int("TRIDIAG_COOP_SPIN", (int64_t)1 << 25), 0x7fffffff));
+        env_int("TRIDIAG_COOP_SPIN", kCoopPolls), 0x7fffffff));
     return v;
 }
 
@@ -651,7 +651,7 @@ static int coop_run(const SolvePlan<T> &pl, int layout, int64_t n, int64_t batch
     CoopParams<T> p{a, b, c, d, x, n, batch, il ? 1 : sstride, il ? batch : 1,
                     (int32_t)(il ? n * batch * (int64_t)sizeof(T) : 0), (int32_t)pl.K,
                     (int32_t)ngroups,
-                    il ? coop_spin_limit() : std::min(coop_spin_limit(), kCoopTreePolls),
+                    coop_spin_limit(),
                     il ? coop_pipelined(e.pipe) : 0,
                     il ? coop_spread(pl.grid / pl.K) : 0,
                     il && !il_rows_on_lines<T>(batch) ? 1 : 0,

@@ -24,10 +24,15 @@
 // round and every member publishes before it waits: with all P workgroups
 // resident, every wait ends.  The slots of a round take groups spread over the whole
 // batch (coop_group), so that a round reads whole interleaved rows rather than a strip.
-// Every wait is still bounded (spin_limit polls): a workgroup whose partners do not
-// publish in time (which needs another kernel to hold CUs that this grid
-// counted on) gives up and writes NaN for x of its block, so the kernel always
-// ends and a lost wait shows in the result rather than as a wrong finite value.
+//
+// Nothing rests on that.  Other kernels (a large solve on a second stream), or a stream
+// that may use only some of the CUs, can keep workgroups of this grid out, and with eight
+// XCDs that fill each at its own pace those that run need not hold one whole group.  So
+// every wait is bounded (spin_limit polls): a workgroup whose wait gives up publishes its
+// remaining tasks without waiting and then finishes them alone (coop_alone): it reduces the
+// blocks of a group that are not published and publishes them in their owners' place.  x of
+// a block is only ever written by its owner, so every solve ends with every row solved,
+// whichever workgroups can run.
 //
 // Publication without L2 writeback or invalidate: the block forms are written
 // with agent-scope atomic stores (which write through to the level where all
@@ -79,6 +84,9 @@ template <typename T> struct CoopParams {
 // words left by earlier solves, or never written, do not read as published and
 // the flags need no clearing between solves.
 constexpr int kCoopFlagStride = 64;
+// Polls of one wait before it gives up: about 1 ms, where a wait takes microseconds unless
+// workgroups of the grid cannot run.
+constexpr int kCoopPolls = 1024;
 // s_sleep argument between two polls of a wait (64 clocks per unit).
 #ifndef TRI_COOP_POLL_SLEEP
 #define TRI_COOP_POLL_SLEEP 8
@@ -103,7 +111,8 @@ template <typename T, int M, int NW, int S> struct CoopShape {
 
 // Wave 0 of a workgroup waits until all K blocks of group g carry the solve's tag:
 // lane k polls block k's word, and the wave goes on once every lane has seen it
-// (one vote per poll).  Returns 0 if spin_limit polls pass first.
+// (one vote per poll; its own block's word among them, so that the workgroup's flag is
+// known to be visible before it stores x).  Returns 0 if spin_limit polls pass first.
 template <typename T>
 __device__ __forceinline__ int coop_wait(const CoopParams<T> &p, int g, int lane) {
     const uint64_t *f = p.flags + kCoopFlagStride * g;
@@ -124,9 +133,9 @@ __device__ __forceinline__ int coop_wait(const CoopParams<T> &p, int g, int lane
 // Stages the K block forms of a group (K*6*S values at fg) into sh_k with the whole
 // workgroup.  Each thread issues several loads before it stores the first: the loads are
 // agent-scope (they go past the XCD's L2 to where all XCDs meet), and one after another
-// their latencies add up.  ok == false (a wait that gave up): zeros, and no loads.
+// their latencies add up.
 template <typename T, int S, int NW>
-__device__ __forceinline__ void coop_stage_forms(const T *fg, int K, bool ok, int tid, T *sh_k) {
+__device__ __forceinline__ void coop_stage_forms(const T *fg, int K, int tid, T *sh_k) {
     constexpr int NT = 64 * NW, B = sizeof(T) == 4 ? 8 : 4;
     const int ne = K * 6 * S;
     for (int e0 = 0; e0 < ne; e0 += NT * B) {
@@ -134,8 +143,8 @@ __device__ __forceinline__ void coop_stage_forms(const T *fg, int K, bool ok, in
 #pragma unroll
         for (int i = 0; i < B; ++i) {
             const int e = e0 + i * NT + tid;
-            v[i] = (ok && e < ne) ? __hip_atomic_load(fg + e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
-                                  : T(0);
+            v[i] = e < ne ? __hip_atomic_load(fg + e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                          : T(0);
         }
 #pragma unroll
         for (int i = 0; i < B; ++i) {
@@ -204,8 +213,8 @@ __device__ __forceinline__ void coop_rsrc(const CoopParams<T> &p, __amdgpu_buffe
 // Publishes a task's block form.  The waves' forms (oL, oR after the merges inside each
 // wave) meet in LDS and log2(NW) merges across lanes give each wave-block's ends in terms
 // of the block's neighbours, which stay in wf for coop_finish; the first and last of them
-// are the block's form.
-template <typename T, int NW, int S>
+// are the block's form.  ALONE: without publishing.
+template <typename T, int NW, int S, bool ALONE = false>
 __device__ __forceinline__ void coop_publish(const CoopParams<T> &p, int gi, int j,
                                              const Outer<T> &oL, const Outer<T> &oR, int tid,
                                              CoopWaveForms<T, NW, S> &wf) {
@@ -222,7 +231,7 @@ __device__ __forceinline__ void coop_publish(const CoopParams<T> &p, int gi, int
         wm_wave_merges<T, NW, SG>(F, E, lane, lane % SG, w, NW, false, nullptr);
         m[0] = F.r; m[S] = F.p; m[2 * S] = F.q;
         m[3 * S] = E.r; m[4 * S] = E.p; m[5 * S] = E.q;
-        if (w == 0 || w == NW - 1) {
+        if (!ALONE && (w == 0 || w == NW - 1)) {
             T *out = p.forms + (((int64_t)gi * p.K + j) * 6 + (w == 0 ? 0 : 3)) * S + s;
             const T v[3] = {w == 0 ? F.r : E.r, w == 0 ? F.p : E.p, w == 0 ? F.q : E.q};
 #pragma unroll
@@ -230,10 +239,10 @@ __device__ __forceinline__ void coop_publish(const CoopParams<T> &p, int gi, int
                 __hip_atomic_store(out + q * S, v[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
         // the forms are at the agent-coherent level before the barrier
-        __builtin_amdgcn_s_waitcnt(0);
+        if (!ALONE) __builtin_amdgcn_s_waitcnt(0);
     }
     __syncthreads();
-    if (tid == 0)
+    if (!ALONE && tid == 0)
         __hip_atomic_store(p.flags + kCoopFlagStride * gi + j, p.tag, __ATOMIC_RELAXED,
                            __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -254,9 +263,10 @@ template <typename T, int S> struct CoopEnds {
 
 // Back-substitution of one task once its group has published: waits for the K block forms
 // of group gi, takes x around block j from them, x around every wave-block from wf, and
-// stores x of the block.
-template <typename T, int M, int NW, int S, int KMAX, int NI>
-__device__ __forceinline__ void coop_finish(const CoopParams<T> &p, int gi, int j,
+// stores x of the block.  Returns false, with nothing stored, where the wait gave up (the same
+// for the whole workgroup).  ALONE: all forms are published, no wait.
+template <typename T, int M, int NW, int S, int KMAX, int NI, bool ALONE = false>
+__device__ __forceinline__ bool coop_finish(const CoopParams<T> &p, int gi, int j,
                                             const CoopWaveForms<T, NW, S> &wf,
                                             CoopBuf<T, M, NW, S, KMAX> &buf, CoopEnds<T, S> &ends, int tid,
                                             const Outer<T> &oL, const Outer<T> &oR,
@@ -265,14 +275,15 @@ __device__ __forceinline__ void coop_finish(const CoopParams<T> &p, int gi, int 
     constexpr int SW = 64 / S;
     constexpr int R = SW * NW * M;
     const int lane = tid & 63, ws = tid >> 6, sl = lane % S, kw = lane / S;
-    if (tid < 64) {
-        const int ok = coop_wait(p, gi, tid);
-        if (tid == 0) ends.ok = ok;
+    if constexpr (!ALONE) {
+        if (tid < 64) {
+            const int ok = coop_wait(p, gi, tid);
+            if (tid == 0) ends.ok = ok;
+        }
+        __syncthreads();
+        if (!ends.ok) return false;
     }
-    __syncthreads();
-    const bool ok = ends.ok != 0;
-    coop_stage_forms<T, S, NW>(p.forms + (int64_t)gi * p.K * 6 * S, p.K, ok, tid,
-                               buf.forms());
+    coop_stage_forms<T, S, NW>(p.forms + (int64_t)gi * p.K * 6 * S, p.K, tid, buf.forms());
     __syncthreads();
     coop_block_ends<T, S>(buf.forms(), p.K, j, tid, ends.x);
     __syncthreads();
@@ -297,14 +308,11 @@ __device__ __forceinline__ void coop_finish(const CoopParams<T> &p, int gi, int 
         xn = (de[q] - al[q] * xL) - ga[q] * xn;
         xs[q + 1] = xn;
     }
-    if (!ok) {
-#pragma unroll
-        for (int q = 0; q < M; ++q) xs[q] = __builtin_nan("");
-    }
     il_block_store<T, M, SW, S, true, true>(make_rsrc(p.x, p.buf_bytes),
                                             (int64_t)j * R + (int64_t)ws * SW * M, p.rstride,
                                             (int64_t)gi * S, p.n, p.batch, lane, sl, kw, buf.wave(ws), xs);
     __syncthreads();                           // LDS of this task free
+    return true;
 }
 
 // Sweep of the lane's M rows (row0 = its first) and the merges inside the wave: the lane's
@@ -319,6 +327,64 @@ __device__ __forceinline__ void coop_reduce(const T (&rows)[4][M], int64_t row0,
     const T ARr = -(o.aR * o.alp), DRr = o.bR - o.aR * o.g, FRr = o.dR - o.aR * o.del;
     segment_outer(o.aL, DLr, ELr, FLr, ARr, DRr, o.cR, FRr, oL, oR);
     wm_wave_merges<T, 64 / S, S>(oL, oR, lane, lane % S, lane / S, 64 / S, false, nullptr);
+}
+
+// A task after a wait gave up: the unpublished blocks of its group are reduced and
+// published here, then its own block is reduced again and finished without a wait.  In place, the
+// owner of a block stores x over the d that is read here, but only after its flag is visible:
+// the flag is looked at once the block has been read, and where it is set the owner's form
+// stands and this one is dropped.  Otherwise both write the same values.  Runs after the
+// task loop, for the task whose wait gave up and those after it, which only published: inside
+// the loop it cost registers (FP64 3001 x 1001 33.5 / 34.1 us).
+template <typename T, int M, int NW, int S, int KMAX>
+__device__ __forceinline__ void coop_alone(const CoopParams<T> &p, int task,
+                                           CoopWaveForms<T, NW, S> &wf,
+                                           CoopBuf<T, M, NW, S, KMAX> &buf, CoopEnds<T, S> &ends) {
+    using Sh = TileShape<T, M, NW, S, true, false, false, false, false, true, true>;
+    constexpr int SW = 64 / S, R = SW * NW * M;
+    int gi, j;
+    coop_task(p, task, gi, j);
+    uint64_t *flags = p.flags + kCoopFlagStride * gi;
+    auto published = [&](int k) {              // the same answer for the whole workgroup
+        __syncthreads();
+        if (threadIdx.x == 0)
+            ends.ok = __hip_atomic_load(flags + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == p.tag;
+        __syncthreads();
+        return ends.ok != 0;
+    };
+    for (int k = 0; k <= p.K; ++k) {           // block j itself is published; it comes last
+        const bool own = k == p.K;
+        if (!own && published(k)) continue;
+        int tid = threadIdx.x;
+        asm volatile("" : "+v"(tid));
+        const int lane = tid & 63, wave = tid >> 6, sl = lane % S, kw = lane / S;
+        const int64_t wrow = (int64_t)(own ? j : k) * R + (int64_t)wave * SW * M;
+        __amdgpu_buffer_rsrc_t rr[4];
+        coop_rsrc(p, rr);
+        T rows[4][M], al[Sh::NI];
+        il_block_load<T, M, SW, S, false, true>(rr, wrow, p.rstride, (int64_t)gi * S, p.n, lane, sl, kw,
+                                                buf.wave(wave), rows);
+        SweepOut<T, Sh::NI> o;
+        Outer<T> oL, oR;
+        coop_reduce<T, Sh, M, S>(rows, wrow + (int64_t)kw * M, p.n, lane, o, al, oL, oR);
+        coop_publish<T, NW, S, true>(p, gi, j, oL, oR, tid, wf);
+        if (own) {
+            coop_finish<T, M, NW, S, KMAX, Sh::NI, true>(p, gi, j, wf, buf, ends, tid, oL, oR, o.de,
+                                                         o.ga, al);
+        } else if (!published(k)) {
+            if (tid < S) {
+                T *out = p.forms + ((int64_t)gi * p.K + k) * 6 * S + tid;
+#pragma unroll
+                for (int q = 0; q < 6; ++q)
+                    __hip_atomic_store(out + q * S, wf.v[q < 3 ? 0 : NW - 1][q * S + tid], __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_AGENT);
+                __builtin_amdgcn_s_waitcnt(0);
+            }
+            __syncthreads();
+            if (tid == 0)
+                __hip_atomic_store(flags + k, p.tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+    }
 }
 
 // OCC: waves per SIMD the kernel is built for (its register budget).  LINES: rows start on
@@ -338,6 +404,7 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(OC
 
     const int P = (int)gridDim.x;
     const int ntask = p.ngroups * p.K;
+    int left = ntask;                        // first task whose wait gave up
     for (int task = (int)blockIdx.x; task < ntask; task += P) {
         // an opaque copy: lane-dependent addresses and masks stay inside the task loop
         // instead of occupying registers across it
@@ -358,9 +425,11 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(OC
         Outer<T> oL, oR;
         coop_reduce<T, Sh, M, S>(rows, wrow + (int64_t)kw * M, p.n, lane, o, al, oL, oR);
         coop_publish<T, NW, S>(p, gi, j, oL, oR, tid, wf);
-        coop_finish<T, M, NW, S, KMAX, Sh::NI>(p, gi, j, wf, buf, ends, tid, oL, oR, o.de, o.ga,
-                                               al);
+        if (left == ntask && !coop_finish<T, M, NW, S, KMAX, Sh::NI>(p, gi, j, wf, buf, ends, tid, oL,
+                                                                     oR, o.de, o.ga, al))
+            left = task;
     }
+    for (; left < ntask; left += P) coop_alone<T, M, NW, S, KMAX>(p, left, wf, buf, ends);
 }
 
 // The same solve with the wait taken one task later: a workgroup reduces and
@@ -405,11 +474,13 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)
     int pend = -1, par = 0;
     Outer<T> poL{}, poR{};
     T pde[NI], pga[NI], pal[NI];
+    int left = ntask;
     auto finish = [&]() {
         int gi, j;
         coop_task(p, pend, gi, j);
-        coop_finish<T, M, NW, S, KMAX, NI>(p, gi, j, wf[par ^ 1], buf, ends, tid, poL, poR, pde,
-                                           pga, pal);
+        if (left == ntask && !coop_finish<T, M, NW, S, KMAX, NI>(p, gi, j, wf[par ^ 1], buf, ends, tid,
+                                                                 poL, poR, pde, pga, pal))
+            left = pend;
     };
     for (; task < ntask; task += P) {
         int gi, j;
@@ -436,6 +507,7 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)
         }
     }
     if (pend >= 0) finish();
+    for (; left < ntask; left += P) coop_alone<T, M, NW, S, KMAX>(p, left, wf[0], buf, ends);
 }
 
 template <typename T> struct CoopEntry {

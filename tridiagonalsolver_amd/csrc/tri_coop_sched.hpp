@@ -33,8 +33,8 @@ inline TRI_COOP_HD int coop_group(int s, int G, int W) {
 // and come in clusters of C whose tasks are consecutive; a cluster's tasks are numbered row
 // block by row block, and each XCD (workgroups are dispatched to the eight in turn) takes
 // consecutive numbers, so that its L2 serves the second reader of a line.  C * K stays
-// at most 64, what a system of 64 blocks needs by itself: workgroups are dispatched in
-// order, so wherever 64 more of the grid are resident a whole cluster is, and its waits end.
+// at most 64, what a system of 64 blocks needs by itself, so that few workgroups wait for
+// each other where some of the grid cannot run.
 // Measured on MI355X, C * K <= 128 / <= 64 (us): FP64 3001 x 1001 40.4 / 39.9, 1024 x 4001
 // 53.9 / 55.5, 9000 x 250 41.7 / 43.2, FP32 4096 x 4001 103.5 / 103.5, 600 x 15,999 66.0 / 64.0.
 inline TRI_COOP_HD void coop_task_shared(int task, int P, int K, int G, int &gi, int &j) {

@@ -13,9 +13,8 @@
 //     that block's form into registers, and 6 rounds across the wave's lanes plus
 //     log2(NW) rounds over the waves' merged forms give x at every block boundary.
 //
-// A wait needs the K workgroups of a system resident at once.  Other kernels (another
-// long solve on a second stream among them) can hold the CUs this grid counted on, so
-// a workgroup waits a bounded number of polls, then leaves its block unsolved (x is not
+// Waits are bounded here too: with hundreds of blocks per system a workgroup whose partners
+// do not publish waits a bounded number of polls, then leaves its block unsolved (x is not
 // written, d is intact) and goes on: every block's form is published in the end, no
 // wait depends on a workgroup that cannot run, and coop_mend_kernel, launched after it,
 // solves the blocks that were left.  It reads one word per block when there are none.
@@ -23,9 +22,6 @@
 #include "tri_coop.hpp"
 
 namespace tri {
-
-// Polls of one wait before the block is left to coop_mend_kernel.
-constexpr int kCoopTreePolls = 1024;
 
 // Contiguous blocks: whole 16-byte chunks of the wave's 64*M rows, issued
 // unconditionally (the buffer ends at the system's last row, so chunks past it
