@@ -142,9 +142,9 @@ int tridiag_solve(int precision, int algo, int layout, int64_t n_eqt, int64_t n_
 /* tridiag_solve with device scratch from the caller, such as a framework's caching
  * allocator, in place of the stream-ordered allocation that the cooperative solve
  * makes on each call (10-15 us of host time).  tridiag_scratch_bytes says how much
- * (0: the solve needs none, or allocates its own), for the current GPU.  Smaller or
- * null scratch is not used and the solve allocates.  The scratch needs no clearing;
- * it belongs to the solve until the stream has passed it. */
+ * (0: the solve needs none, or allocates its own), for the current GPU.  Scratch that
+ * is smaller, null or not aligned to 8 bytes is not used and the solve allocates.  The
+ * scratch needs no clearing; it belongs to the solve until the stream has passed it. */
 int64_t tridiag_scratch_bytes(int precision, int algo, int layout, int64_t n_eqt, int64_t n_batch);
 int tridiag_solve_scratch(int precision, int algo, int layout, int64_t n_eqt, int64_t n_batch,
                           void *a, void *b, void *c, void *d, void *scratch, int64_t scratch_bytes,

@@ -1395,7 +1395,10 @@ int tridiag_solve_to(int precision, int algo, int layout, int64_t n_eqt, int64_t
                                           (int)n_eqt, (int)n_batch);
     }
     hipStream_t st = (hipStream_t)stream;
-    const FixedScratch given{scratch, (size_t)(scratch && scratch_bytes > 0 ? scratch_bytes : 0), false};
+    // the kernels keep 64-bit words in it
+    const bool usable = scratch && scratch_bytes > 0 &&
+                        reinterpret_cast<uintptr_t>(scratch) % sizeof(uint64_t) == 0;
+    const FixedScratch given{scratch, (size_t)(usable ? scratch_bytes : 0), false};
     if (precision == TRIDIAG_SINGLE)
         return solve_impl<float>(algo, layout, n_eqt, n_batch, (float *)a, (float *)b,
                                  (float *)c, (float *)d, st, &given,
