@@ -861,8 +861,9 @@ def run_large(torch, T, steps, warmup):
         out[name] = {"n": n, "batch": batch, "ms_per_step": wall, "kernel_ms": kern,
                      "unknowns_per_s": U / (wall * 1e-3), "achieved_gbs": achieved,
                      "hbm_frac": achieved / HBM_PEAK_GBS, "parity": par, "plan": pl,
-                     "path": {"chunked": "chunked: reduce / chunk-interface merge / solve",
-                              "cooperative": "cooperative row blocks (5 words per unknown)"}
+                     # a plan with K row blocks is solved cooperatively, whatever its kind
+                     "path": "cooperative row blocks (5 words per unknown)" if "K" in pl
+                     else {"chunked": "chunked: reduce / chunk-interface merge / solve"}
                      .get(pl["kind"], pl["kind"])}
         log(name, json.dumps(out[name]))
     return out
