@@ -398,24 +398,26 @@ static int64_t env_int(const char *name, int64_t dflt) {
 // ($TRIDIAG_COOP_MIN_ROWS overrides; a negative value turns the cooperative solve off for
 // both layouts).  Whole-piece tiles end at 512 rows; above, the one-workgroup tiles read
 // pieces of 16-64 bytes and beyond 4096 rows only the contiguous copy is left.  Measured
-// on MI355X, tile or copy / cooperative (us): FP32 600 x 16,000 65 / 55, 700 x 100 12.8 /
-// 10.2, 1100 x 500 15.5 / 11.0, 3001 x 20 29.3 / 10.4, 4096 x 4001 116 / 106, 5000 x 64
-// 30.7 / 12.8, 16,384 x 1024 213 / 167; FP64 600 x 8000 67.6 / 57.7, 700 x 2000 18.8 / 17.1,
-// 3001 x 1001 67 / 45, 3001 x 1008 64 / 35, 12,000 x 20 48.0 / 19.9.  Below: FP32 400 x 4000
-// 12.6 / 19.7, FP64 17.5 / 22.1.
+// on MI355X, tile or copy / cooperative (us, back to back on the same arrays): FP32 600 x 33
+// 10.8 / 8.9, 600 x 16,000 51.7 / 45.7, 700 x 100 12.3 / 9.2, 1100 x 500 14.4 / 10.1, 3001 x 20
+// 27.9 / 10.3, 4096 x 4001 109 / 78.9, 16,000 x 500 113 / 66.8; FP64 700 x 2000 13.7 / 13.7,
+// 3001 x 1001 58.0 / 34.4, 3001 x 1008 51.1 / 27.1, 5000 x 9 28 / 11.2, 9000 x 250 83.7 / 42.0.
+// Below, each call alone: FP32 400 x 4000 12.6 / 19.7, FP64 17.5 / 22.1.
 static int64_t coop_min_rows_il() {
     static const int64_t env = env_int("TRIDIAG_COOP_MIN_ROWS", 0);
     return env != 0 ? env : 513;
 }
 // Interleaved batches below this many rows, or with partial row blocks, or off lines where
-// a tile holds n, report the tile or the copy that they took before the cooperative solve
-// took every size (tridiag_plan_blocks says what runs).
+// a tile holds n, report the tile or the copy that they take without the cooperative solve,
+// which is also what a solve recorded into a graph without scratch runs
+// (tridiag_plan_blocks says what runs otherwise).
 constexpr int64_t kCoopReportedRows = 1024;
 
 // Whether interleaved rows start on 128-byte lines.  Off them the row pieces of neighbouring
 // groups share lines: the loads stay cached and the neighbours run on one XCD
-// (coop_task_shared).  Streamed and in the spread order FP64 3001 x 1001 took 57.6 us
-// (44.5 this way), FP32 4096 x 4001 173 us (106).
+// (coop_task_shared).  Streamed and in the spread order FP64 3001 x 1001 took 57.6 us and this
+// way 44.5, FP32 4096 x 4001 173 and 106 (each call alone, before the block forms were
+// merged across lanes).
 template <typename T> static bool il_rows_on_lines(int64_t batch) {
     return (batch * (int64_t)sizeof(T)) % 128 == 0;
 }
@@ -734,11 +736,12 @@ static SolvePlan<T> make_plan(int algo, int layout, int64_t n, int64_t batch, in
     const int prec = sizeof(T) == 4 ? TRIDIAG_SINGLE : TRIDIAG_DOUBLE;
     const int32_t bb = buffer_extent<T>(n, batch, sstride, layout);
     // short contiguous systems: several per wave, for the automatic choice above the 8
-    // rows that fill the lane kernel (2^22 unknowns, lane / this: 9 rows FP32 21.1 / 14.7
-    // us, 16 rows 15.8 / 15.8, FP64 32.4 / 28.7) and up to where a tile's wave per system
-    // holds few padding rows (192 rows, tile / this: FP32 14.8 / 15.4 us, FP64 31.2 /
-    // 28.9; 200 rows FP32 16.5 either way, FP64 29.5 / 30.2).  Up to 64 systems of 16
-    // rows are one wave of the lane kernel and keep it.
+    // rows that fill the lane kernel (2^22 unknowns back to back, lane / this: 9 rows FP32
+    // 20.5 / 12.7 us, 16 rows 15.6 / 14.6, FP64 32.0 / 27.8) and up to where a tile's wave
+    // per system holds few padding rows (192 rows, each call alone, tile / this: FP32 14.8 /
+    // 15.4 us, FP64 31.2 / 28.9; 200 rows FP32 16.5 either way, FP64 29.5 / 30.2).  Up to 64
+    // systems of 16 rows are one wave of the lane kernel and keep it, as all do that
+    // $TRIDIAG_LANE_ROWS asks for.
     if (algo == TRIDIAG_ALGO_AUTO && layout == kContiguous && n > 8 && n <= kShortMaxRows &&
         (n > 16 || batch > 64) && n > lane_rows_asked()) {
         pl.kind = kPlanShort;

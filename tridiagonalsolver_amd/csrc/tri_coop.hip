@@ -93,10 +93,11 @@ hipError_t launch_coop_clear(uint64_t *words, int64_t count, hipStream_t st) {
 // instead FP32 4096 x 4096 100, FP64 211; blocks of 128 rows (M = 8 FP32, 4 FP64) and
 // 16-wave workgroups were slower or even.
 // With the block forms [system][block][6] in LDS (all lanes of an access on one bank), in a
-// buffer of their own (one workgroup per CU above 32 blocks) and two serial chains, / now:
-// FP32 4096 x 4096 89.8 / 87.7, 600 x 16,000 49.6 / 48.5, 8192 x 2048 97.0 / 91.9, 16,000 x 500
-// 92.7 / 62.3; FP64 3001 x 1001 42.3 / 40.4, 3001 x 1008 34.1 / 30.0 (4.0 TB/s), 9000 x 250
-// 58.5 / 41.4.  The loads' pattern alone (pieces of one line, 256 rows per task) takes 70-86
+// buffer of their own (one workgroup per CU above 32 blocks) and two serial chains, / now
+// (back to back on the same arrays, scratch from the caller): FP32 4096 x 4096 81.1 / 80.2, 600 x
+// 16,000 46.5 / 45.7, 8192 x 2048 108 / 106 (other placements of the arrays 85-97), 16,000 x 500
+// 87.0 / 66.8; FP64 3001 x 1001 37.8 / 34.4, 3001 x 1008 32.1 / 27.1 (4.5 TB/s), 9000 x 250
+// 54.1 / 42.0.  The loads' pattern alone (pieces of one line, 256 rows per task) takes 70-86
 // us at FP32 4096 x 4096, which bounds the large sizes; the rest is the wait for the group
 // and the phases that no second workgroup covers.
 // Contiguous: one system, blocks of 64*NW*M rows, up to 64*NW blocks; small blocks

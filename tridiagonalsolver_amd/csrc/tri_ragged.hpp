@@ -75,8 +75,8 @@ __device__ __forceinline__ void ragged_item(const RaggedParams<T> &p, const int3
         // checks each dword, so chunks that straddle or pass the end need no predicate (loads
         // past it give zero, stores are dropped) and rows may start at any element.
         // Measured on MI355X, with an address and a tail branch per chunk / this (us): 65,536
-        // systems of 32 ... 8192 rows FP32 387 / 374 (5.15 TB/s), 30,000 FP64 431 / 380
-        // (208 / 194 VGPRs), 10,000 of 500 ... 1000 rows FP64 76.6 / 65.9.  Cached instead
+        // systems of 32 ... 8192 rows FP32 381 / 373 (5.17 TB/s), 30,000 FP64 430 / 378
+        // (208 / 194 VGPRs), 10,000 of 500 ... 1000 rows FP64 76.4 / 66.1.  Cached instead
         // of nontemporal: 414 / 384 / 71.0.
         const __amdgpu_buffer_rsrc_t rr[4] = {ra, rb, rc, rd};
         const int vo = (int)(wrow * (int64_t)sizeof(T)) + lane * 16;

@@ -714,8 +714,8 @@ __global__ void __launch_bounds__(64 * NW)
 
     SweepOut<T, Sh::NI> o;
     const int32_t nb = BIG ? 0x7fffffff : prm.buf_bytes;
-    // Exact contiguous tiles store over d: a second base address costs them 0.5 % (FP32 4096 x
-    // 4096 55.38 / 55.65 us).  Their padded twins serve an x of its own (solve_impl picks them).
+    // Exact contiguous tiles store over d: a second base address costs them 0.4 % (FP32 4096 x
+    // 4096 55.72 / 55.96 us in three pairs of runs, one side's runs within 0.1).  Their padded twins serve an x of its own (solve_impl picks them).
     constexpr bool kInPlace = XP && !IL && !PAD;
     const __amdgpu_buffer_rsrc_t rd_rsrc = make_rsrc(prm.d, nb);
     const __amdgpu_buffer_rsrc_t rx_rsrc = kInPlace ? rd_rsrc : make_rsrc(prm.x, nb);
